@@ -102,6 +102,9 @@ struct ExtendArgs {
   const uint32_t* tri_src;    // non-null (batched queries): hits name source triangles
   const uint32_t* order;      // non-null: queue position k traverses path order[k]
   uint32_t parts;             // lane refill: 1 (one cursor) or kParts queue partitions
+  uint32_t n;                 // batched queries: the number of rays
+  bool deal;                  // batched queries: the rays are dealt out to the launch's waves
+                              // beforehand, without cursors
 };
 
 // The ray sort before a bounce's traversal: a counting sort of the paths

@@ -791,6 +791,51 @@ __device__ __forceinline__ void trav_step_wide(const float4* __restrict__ wn,
   }
 }
 
+// A short queue dealt out beforehand: the rays one wave takes, with no cursor.
+// Local index l of the wave is queue position (l / 64 * waves + mine) * 64 +
+// l % 64 below `whole` (stripes of 64 rays a wave; WHOLE == false: none) and
+// the wave's share of the remainder above, `end` being the wave's last; the
+// waves of one XCD (workgroup b runs on XCD b % 8) are neighbours, as are
+// their rays.
+struct Deal {
+  uint32_t mine, whole, rest, end;
+  __device__ __forceinline__ uint32_t position(uint32_t l, uint32_t waves) const {
+    return l < whole ? ((l >> 6) * waves + mine) * 64u + (l & 63u)
+                     : whole * waves + mine * rest + (l - whole);
+  }
+};
+// Fewer rays than lanes go to as few waves as the 1024 SIMDs can each hold
+// one of, at least kDealLanes rays a wave (below that a wave's steps get no
+// shorter), then to waves of 64 rays: half-filled waves on a SIMD only slow
+// each other down (262,144 rays in a 200,000-triangle room: 0.74 ms in 8192
+// waves of 32, 0.56 ms in 4096 of 64).
+constexpr uint32_t kDealLanes = 4, kDealSimds = 1024;
+template <bool WHOLE>
+__device__ __forceinline__ Deal deal_rays(uint32_t n, uint32_t waves) {
+  Deal d;
+  const uint32_t bw = blockDim.x >> 6, wave = threadIdx.x >> 6;
+  d.whole = WHOLE ? n / (64u * waves) * 64u : 0u;
+  const uint32_t left = n - d.whole * waves;
+  d.rest = (left + waves - 1) / waves;
+  uint32_t blocks = gridDim.x;
+  if (d.whole == 0) {
+    d.rest = max(d.rest, min(max((n + kDealSimds - 1) / kDealSimds, kDealLanes), 64u));
+    blocks = (n + d.rest * bw - 1) / (d.rest * bw);
+  }
+  uint32_t b = blockIdx.x;
+  if ((gridDim.x & 7u) == 0) {
+    // ceil(blocks / 8) consecutive shares per XCD, of which the grid has
+    // enough workgroups since it has a multiple of 8
+    const uint32_t per_xcd = (blocks + 7) / 8;
+    b = (b >> 3) < per_xcd ? (b & 7u) * per_xcd + (b >> 3) : blocks;
+  }
+  d.mine = __builtin_amdgcn_readfirstlane(min(b, blocks) * bw + wave);
+  const uint32_t at = b < blocks ? d.mine * d.rest : left;
+  d.end = __builtin_amdgcn_readfirstlane((b < blocks ? d.whole : 0u) +
+                                         (at < left ? min(d.rest, left - at) : 0u));
+  return d;
+}
+
 // Traversal with lane refill: a lane whose ray is finished takes a new ray
 // from the queue while the other lanes continue, so a wave stays full until
 // the queue is empty.  A wave refills when at least `refill` lanes are idle
@@ -798,15 +843,17 @@ __device__ __forceinline__ void trav_step_wide(const float4* __restrict__ wn,
 // traverse(), one trav_step per loop iteration.
 // Workgroups of 1, 2 or 4 independent waves (the launch's choice); each
 // wave owns S * 64 entries of the dynamic LDS.
-template <bool COUNT, int S, bool PACKED, bool MULTI, bool QUERY = false, int W = 2>
-__global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
-  extern __shared__ uint2 lds_waves[];
+// DEALT: the queue is dealt out beforehand, known at compile time (queries:
+// the dealt positions in the cursors' kernel cost 10^7 rays on the bunny 5 %).
+template <bool COUNT, int S, bool PACKED, bool MULTI, bool QUERY, int W, bool DEALT>
+__device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_waves) {
   const uint32_t lane = lane_id();
   uint2* lds = lds_waves + (threadIdx.x >> 6) * (S * 64);
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t stride = gridDim.x * blockDim.x;
-  const uint32_t n = a.ctrl->count[a.bounce];
-  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&a.ctrl->total_rays, (unsigned long long)n);
+  const uint32_t n = QUERY ? a.n : a.ctrl->count[a.bounce];
+  if (!QUERY && blockIdx.x == 0 && threadIdx.x == 0)
+    atomicAdd(&a.ctrl->total_rays, (unsigned long long)n);
   const uint64_t lt = (1ull << lane) - 1ull;
   // Queue partitions (parts == kParts): the queue is cut into chunks of
   // 2^glog rays, chunk c belonging to partition c % parts.  A wave takes
@@ -816,7 +863,18 @@ __global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
   // the others in turn.  Local position l of partition x is queue position
   // ((l >> glog) * parts + x) << glog | (l & (2^glog - 1)).  parts == 1: one
   // cursor, local position = queue position.
-  const uint32_t parts = a.parts == kParts ? kParts : 1u;
+  // A render's queue of at most one ray per lane and DEALT queries are dealt
+  // out beforehand instead: every wave of the launch taking its atomics from the
+  // cursors, most to find them used up, keeps a launch of few rays busy for
+  // 100-200 us (256 rays on 968 triangles: 207 us, dealt 60; 600,000 in a
+  // 200,000-triangle room: 1.00 ms, dealt 0.69).  A render's bounce of more
+  // rays stays with the cursors: neighbouring paths cost alike, so fixed
+  // shares end further apart (1280 x 736 frames: no faster).
+  const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+  const bool dealt = DEALT || (!QUERY && n <= waves * 64u);
+  Deal deal{};
+  if (dealt) deal = deal_rays<DEALT>(n, waves);
+  const uint32_t parts = !dealt && a.parts == kParts ? kParts : 1u;
   uint32_t glog = 31u - (uint32_t)__builtin_clz(max(n / parts, 1u));
   glog = min(max(glog, 12u), 18u);
   const uint32_t gmask = (1u << glog) - 1u;
@@ -848,7 +906,11 @@ __global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
   // a cursor.  `drained`: the cursors have passed the last ray of every
   // partition.  (Wave-uniform values.)
   uint32_t pool = 0, pool_end = 0, pool_part = 0;
-  bool drained = false;
+  if (dealt) {
+    pool = DEALT ? 0u : deal.mine * deal.rest;
+    pool_end = pool + deal.end;
+  }
+  bool drained = dealt;
   const uint32_t chunk = 64u * (a.batches ? a.batches : 1u);
   uint64_t na = 0, nt = 0;
   for (;;) {
@@ -888,7 +950,9 @@ __global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
         const uint32_t l = old ? base0 + rank : base1 + (rank - from_pool);
         if (old || l < end1) {
           const uint32_t x = old ? part0 : pool_part;
-          const uint32_t k = parts == 1 ? l : (((l >> glog) * parts + x) << glog) | (l & gmask);
+          const uint32_t k = DEALT        ? deal.position(l, waves)
+                             : parts == 1 ? l
+                                          : (((l >> glog) * parts + x) << glog) | (l & gmask);
           // hits-only queries are never sorted
           const uint32_t i = !QUERY && a.order ? a.order[k] : k;
           if (MULTI) {
@@ -974,6 +1038,20 @@ __global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
       atomicAdd(&a.ctrl->sum_tri, (unsigned long long)nt);
     }
   }
+}
+
+template <bool COUNT, int S, bool PACKED, bool MULTI, bool QUERY = false, int W = 2>
+__global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
+  extern __shared__ uint2 lds_waves[];
+  extend_refill<COUNT, S, PACKED, MULTI, QUERY, W, false>(a, lds_waves);
+}
+
+// Hits-only queries of few rays per lane of the launch, dealt out to its
+// waves.
+template <int S, bool PACKED, int W>
+__global__ __launch_bounds__(256) void k_query_dealt(ExtendArgs a) {
+  extern __shared__ uint2 lds_waves[];
+  extend_refill<false, S, PACKED, false, true, W, true>(a, lds_waves);
 }
 
 // ---------------------------------------------------------------------------
@@ -1654,6 +1732,8 @@ static hipError_t launch_extend_wide(const ExtendArgs& a, bool multi, uint32_t b
   if (!b.refill) b.refill = 64;
   if (multi)
     hipLaunchKernelGGL((k_extend_refill<COUNT, S, true, true, false, W>), grid, block, shmem, s, b);
+  else if (b.rays6 && !COUNT && b.deal)
+    hipLaunchKernelGGL((k_query_dealt<S, true, W>), grid, block, shmem, s, b);
   else if (b.rays6 && !COUNT)
     hipLaunchKernelGGL((k_extend_refill<false, S, true, false, true, W>), grid, block, shmem, s,
                        b);
@@ -1679,7 +1759,11 @@ static hipError_t launch_extend_s(const ExtendArgs& a, bool packed, bool multi, 
   } else if (a.refill && a.rays6 && !COUNT) {
     // batched queries: the caller's rays and source ids, compiled apart so
     // that the render instantiations carry neither
-    if (packed)
+    if (a.deal && packed)
+      hipLaunchKernelGGL((k_query_dealt<S, true, 2>), grid, block, shmem, s, a);
+    else if (a.deal)
+      hipLaunchKernelGGL((k_query_dealt<S, false, 2>), grid, block, shmem, s, a);
+    else if (packed)
       hipLaunchKernelGGL((k_extend_refill<false, S, true, false, true>), grid, block, shmem, s, a);
     else
       hipLaunchKernelGGL((k_extend_refill<false, S, false, false, true>), grid, block, shmem, s,

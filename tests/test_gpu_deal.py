@@ -1,0 +1,48 @@
+"""Short queues dealt out to the traversal's waves beforehand (no cursor):
+every ray is traversed once and gives the oracle's hit at the sizes where the
+dealing changes shape -- fewer rays than the smallest share, one more than a
+share or a stripe of 64 rays per wave, the last dealt size and the first that
+goes through the cursors -- for grids that are and are not a multiple of the
+8 XCDs."""
+import numpy as np
+import pytest
+
+from convector_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+LANES = 256 * 64  # one wave per CU
+
+
+@pytest.mark.parametrize("block_waves", [1, 2, 4])
+@pytest.mark.parametrize("waves_per_cu", [1, 3])
+def test_dealt_queries_equal_oracle(cv, oracle, block_waves, waves_per_cu):
+    sd = scenes.config0(subdivisions=2)
+    g = cv.Scene.from_scene_data(sd)
+    o = oracle.Scene.from_scene_data(sd)
+    g.set_tuning(extend_waves_per_cu=waves_per_cu, block_waves=block_waves)
+    lanes = LANES * waves_per_cu
+    rays = scenes.rays_inward(4 * lanes + 1, 7, radius=0.9, target_scale=0.6)
+    ref = o.intersect(rays)
+    for n in (1, 3, 4, 5, 63, 65, 4096, 4097, lanes - 1, lanes, lanes + 1, lanes + 4097,
+              4 * lanes - 63, 4 * lanes, 4 * lanes + 1):
+        print("%d rays, %d waves per CU, %d per block" % (n, waves_per_cu, block_waves), flush=True)
+        hits = g.intersect_nearest(rays[:n])
+        assert (hits["tri_id"] == ref["tri"][:n]).all(), n
+        assert (hits["t"].view(np.uint32) == ref["tuv"][:n, 0].copy().view(np.uint32)).all(), n
+
+
+@pytest.mark.parametrize("w,h", [(16, 4), (128, 124), (128, 128), (128, 132)])
+def test_dealt_frames_equal_oracle(cv, oracle, w, h):
+    """Bounces below, at and above one ray per lane of a one-wave-per-CU
+    launch (16,384 paths)."""
+    print("%dx%d" % (w, h), flush=True)
+    sd = scenes.config0(subdivisions=2)
+    g = cv.Scene.from_scene_data(sd)
+    o = oracle.Scene.from_scene_data(sd)
+    g.set_tuning(extend_waves_per_cu=1)
+    r = cv.Renderer(g, w, h)
+    hdr = r.new_buffer_f32()
+    r.accumulate_frames_f32(hdr, 1, 1)
+    ohdr, _ = o.accumulate_frames(w, h, 1, 1, oracle.RNG_PIXEL, 4)
+    assert hdr.tobytes() == ohdr.tobytes()
