@@ -64,32 +64,137 @@ const char* last_error() { return g_last_error.c_str(); }
 namespace {
 // One pinned bounce buffer for the whole process, allocated on first use and
 // kept until the process ends (freeing pinned memory at exit can run after
-// the HIP runtime is torn down).
-constexpr size_t kBounceBytes = 16u << 20;
+// the HIP runtime is torn down).  Copies go through it in pieces, each with
+// an event of its own, so that the host's copy of one piece overlaps the
+// device's of the next (a 1280 x 736 bitmap and gbuffer, 7.5 MB: 10.2 ms by
+// hipMemcpy2DAsync into pageable memory, row by row; 1.0 ms this way).
+constexpr size_t kPieceBytes = 2u << 20;
+constexpr uint32_t kPieces = 8;
 std::mutex g_bounce_mu;
 char* g_bounce = nullptr;
+hipEvent_t g_piece_done[kPieces] = {};
+
+cv_status bounce_init() {
+  if (!g_bounce)
+    HIPTRY(hipHostMalloc((void**)&g_bounce, kPieceBytes * kPieces, hipHostMallocDefault),
+           "pinned alloc");
+  for (uint32_t k = 0; k < kPieces; k++)
+    if (!g_piece_done[k])
+      HIPTRY(hipEventCreateWithFlags(&g_piece_done[k], hipEventDisableTiming), "event");
+  return CV_OK;
+}
+
+// Rows of `words` 16-byte words between a pitched and a packed buffer.
+__global__ void k_copy_rows(const uint4* src, size_t spitch, uint4* dst, size_t dpitch,
+                            uint32_t words, uint32_t rows) {
+  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < words * rows;
+       k += gridDim.x * blockDim.x)
+    dst[(size_t)(k / words) * dpitch + k % words] = src[(size_t)(k / words) * spitch + k % words];
+}
+
+// The part of a rect that one piece of the bounce buffer takes: rows
+// [row, row + rows) of `bytes` bytes from byte `col` on.
+struct Piece {
+  const CallerRect* rc;
+  size_t col, bytes, row, rows;
+};
 }  // namespace
+
+cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st) {
+  std::vector<Piece> ps;
+  for (size_t i = 0; i < n; i++) {
+    const CallerRect& r = rects[i];
+    if (!r.bytes || !r.rows) continue;
+    const bool packed = r.rows == 1 || (r.host_pitch == r.bytes && r.dev_pitch == r.bytes);
+    if (packed || r.bytes > kPieceBytes) {
+      // contiguous, or rows longer than a piece: bytes of one row (or of all)
+      const size_t row_bytes = packed ? r.bytes * r.rows : r.bytes;
+      for (size_t y = 0; y < (packed ? 1 : r.rows); y++)
+        for (size_t c = 0; c < row_bytes; c += kPieceBytes)
+          ps.push_back(Piece{&r, c, std::min(kPieceBytes, row_bytes - c), y, 1});
+    } else {
+      const size_t per = kPieceBytes / r.bytes;
+      for (size_t y = 0; y < r.rows; y += per)
+        ps.push_back(Piece{&r, 0, r.bytes, y, std::min(per, r.rows - y)});
+    }
+  }
+  if (ps.empty()) return CV_OK;
+  std::lock_guard<std::mutex> lk(g_bounce_mu);
+  cv_status cs = bounce_init();
+  if (cs != CV_OK) return cs;
+  auto host_of = [](const Piece& p) { return (char*)p.rc->host + p.row * p.rc->host_pitch + p.col; };
+  auto dev_of = [](const Piece& p) { return (char*)p.rc->dev + p.row * p.rc->dev_pitch + p.col; };
+  auto host_copy = [&](size_t k) {
+    const Piece& p = ps[k];
+    char* b = g_bounce + (k % kPieces) * kPieceBytes;
+    for (size_t y = 0; y < p.rows; y++) {
+      char* h = host_of(p) + y * p.rc->host_pitch;
+      if (to_device)
+        memcpy(b + y * p.bytes, h, p.bytes);
+      else
+        memcpy(h, b + y * p.bytes, p.bytes);
+    }
+  };
+  auto dev_copy = [&](size_t k) -> cv_status {
+    const Piece& p = ps[k];
+    char* b = g_bounce + (k % kPieces) * kPieceBytes;
+    const bool words = !((p.bytes | p.rc->dev_pitch | (size_t)dev_of(p)) & 15);
+    if (p.rows == 1 && (to_device || !words)) {
+      HIPTRY(hipMemcpyAsync(to_device ? dev_of(p) : b, to_device ? b : dev_of(p), p.bytes,
+                            to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, st),
+             "copy");
+    } else if (!words) {
+      HIPTRY(hipMemcpy2DAsync(to_device ? dev_of(p) : b, to_device ? p.rc->dev_pitch : p.bytes,
+                              to_device ? b : dev_of(p), to_device ? p.bytes : p.rc->dev_pitch,
+                              p.bytes, p.rows,
+                              to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, st),
+             "copy");
+    } else {
+      const uint4* src = (const uint4*)(to_device ? b : dev_of(p));
+      uint4* dst = (uint4*)(to_device ? dev_of(p) : b);
+      const size_t pk = p.bytes / 16, pitch = p.rc->dev_pitch / 16;
+      hipLaunchKernelGGL(k_copy_rows, dim3(grid_for(pk * p.rows, 256, 256)), dim3(256), 0, st, src,
+                         to_device ? pk : pitch, dst, to_device ? pitch : pk, (uint32_t)pk,
+                         (uint32_t)p.rows);
+      HIPTRY(hipGetLastError(), "copy");
+    }
+    HIPTRY(hipEventRecord(g_piece_done[k % kPieces], st), "event");
+    return CV_OK;
+  };
+  hipError_t we = hipSuccess;
+  if (to_device) {
+    for (size_t k = 0; k < ps.size() && cs == CV_OK; k++) {
+      if (k >= kPieces) we = hipEventSynchronize(g_piece_done[k % kPieces]);
+      if (we != hipSuccess) break;
+      host_copy(k);
+      cs = dev_copy(k);
+    }
+  } else {
+    size_t sent = 0;
+    for (size_t k = 0; k < ps.size() && cs == CV_OK; k++) {
+      while (sent < ps.size() && sent < k + kPieces && cs == CV_OK) cs = dev_copy(sent++);
+      if (cs != CV_OK) break;
+      we = hipEventSynchronize(g_piece_done[k % kPieces]);
+      if (we != hipSuccess) break;
+      host_copy(k);
+    }
+  }
+  // the bounce buffer is the next caller's from here on
+  const hipError_t se = hipStreamSynchronize(st);
+  if (cs != CV_OK) return cs;
+  HIPTRY(we, "copy");
+  HIPTRY(se, "copy");
+  return CV_OK;
+}
 
 cv_status copy_caller_memory(void* dst, const void* src, size_t bytes, bool to_device,
                              hipStream_t st) {
-  if (bytes == 0) return CV_OK;
-  std::lock_guard<std::mutex> lk(g_bounce_mu);
-  if (!g_bounce) HIPTRY(hipHostMalloc((void**)&g_bounce, kBounceBytes, hipHostMallocDefault),
-                        "pinned alloc");
-  for (size_t off = 0; off < bytes; off += kBounceBytes) {
-    const size_t c = bytes - off < kBounceBytes ? bytes - off : kBounceBytes;
-    if (to_device) {
-      memcpy(g_bounce, (const char*)src + off, c);
-      HIPTRY(hipMemcpyAsync((char*)dst + off, g_bounce, c, hipMemcpyHostToDevice, st), "upload");
-      HIPTRY(hipStreamSynchronize(st), "upload");
-    } else {
-      HIPTRY(hipMemcpyAsync(g_bounce, (const char*)src + off, c, hipMemcpyDeviceToHost, st),
-             "download");
-      HIPTRY(hipStreamSynchronize(st), "download");
-      memcpy((char*)dst + off, g_bounce, c);
-    }
-  }
-  return CV_OK;
+  CallerRect r;
+  r.host = to_device ? const_cast<void*>(src) : dst;
+  r.dev = to_device ? dst : const_cast<void*>(src);
+  r.bytes = r.host_pitch = r.dev_pitch = bytes;
+  r.rows = 1;
+  return copy_caller_rects(&r, 1, to_device, st);
 }
 
 cv_status validate_tuning(const cv_tuning& t) {
@@ -503,8 +608,7 @@ static cv_status scene_apply_tuning(cv_scene* s, const cv_tuning& t) {
   return CV_OK;
 }
 
-static cv_status scene_finish(cv_scene* s, const std::vector<float>& v9,
-                              const std::vector<float>& uv6, const std::vector<uint32_t>& mat,
+static cv_status scene_finish(cv_scene* s, const cv_mesh* const* meshes, size_t nmeshes,
                               const cv_bvh_node* nodes_in, size_t nnodes_in,
                               const uint32_t* order_in) {
   const uint32_t N = s->ntris;
@@ -512,8 +616,24 @@ static cv_status scene_finish(cv_scene* s, const std::vector<float>& v9,
   DevBuf<float> d_v9;
   DevBuf<float> d_uv;
   DevBuf<uint32_t> d_mat;
-  HIPTRY(d_v9.alloc(v9.size()), "alloc");
-  HIPTRY(hipMemcpyAsync(d_v9.p, v9.data(), v9.size() * 4, hipMemcpyHostToDevice, st), "upload");
+  // the meshes one after the other, straight from their own arrays
+  HIPTRY(d_v9.alloc(9ull * N), "alloc");
+  HIPTRY(d_uv.alloc(6ull * N), "alloc");
+  HIPTRY(d_mat.alloc(N), "alloc");
+  {
+    std::vector<cvh::CallerRect> up;
+    size_t at = 0;
+    for (size_t i = 0; i < nmeshes; i++) {
+      const cv_mesh& m = *meshes[i];
+      const size_t k = m.ntris();
+      up.push_back(cvh::CallerRect::flat(m.v9.data(), d_v9.p + 9 * at, k * 36));
+      up.push_back(cvh::CallerRect::flat(m.uv6.data(), d_uv.p + 6 * at, k * 24));
+      up.push_back(cvh::CallerRect::flat(m.mat.data(), d_mat.p + at, k * 4));
+      at += k;
+    }
+    cv_status us = cvh::copy_caller_rects(up.data(), up.size(), true, st);
+    if (us != CV_OK) return us;
+  }
   HIPTRY(s->tri_src.alloc(N), "alloc");
   if (nodes_in) {
     HIPTRY(s->nodes.alloc(nnodes_in), "alloc");
@@ -571,10 +691,6 @@ static cv_status scene_finish(cv_scene* s, const std::vector<float>& v9,
   s->info.num_triangles = N;
   HIPTRY(s->tris.alloc(N), "alloc");
   HIPTRY(cvk::launch_prepare_tris(d_v9.p, s->tri_src.p, N, s->tris.p, st), "prepare");
-  HIPTRY(d_mat.alloc(N), "alloc");
-  HIPTRY(hipMemcpyAsync(d_mat.p, mat.data(), N * 4ull, hipMemcpyHostToDevice, st), "upload");
-  HIPTRY(d_uv.alloc(6ull * N), "alloc");
-  HIPTRY(hipMemcpyAsync(d_uv.p, uv6.data(), N * 24ull, hipMemcpyHostToDevice, st), "upload");
   HIPTRY(s->tri_mat.alloc(N), "alloc");
   HIPTRY(s->tri_uv.alloc(6ull * N), "alloc");
   hipLaunchKernelGGL(k_gather_u32, dim3(grid_for(N, 256, 65535)), dim3(256), 0, st, d_mat.p,
@@ -621,18 +737,15 @@ static cv_status scene_create_impl(const cv_mesh* const* meshes, size_t n,
   if (opts && opts->builder != CV_BUILDER_REFERENCE && opts->builder != CV_BUILDER_BINS_32 &&
       opts->builder != CV_BUILDER_BINS_16)
     return fail(CV_ERR_INVALID_ARGUMENT, "unknown builder");
-  std::vector<float> v9, uv6;
-  std::vector<uint32_t> mat;
+  size_t total = 0;
   for (size_t i = 0; i < n; i++) {
     if (!meshes[i]) return fail(CV_ERR_INVALID_ARGUMENT, "null mesh");
-    v9.insert(v9.end(), meshes[i]->v9.begin(), meshes[i]->v9.end());
-    uv6.insert(uv6.end(), meshes[i]->uv6.begin(), meshes[i]->uv6.end());
-    mat.insert(mat.end(), meshes[i]->mat.begin(), meshes[i]->mat.end());
+    total += meshes[i]->ntris();
   }
-  if (mat.empty()) return fail(CV_ERR_BVH_NO_SPLIT, "scene has no triangles");
-  if (mat.size() >= (1ull << 31)) return fail(CV_ERR_INVALID_ARGUMENT, "too many triangles");
+  if (total == 0) return fail(CV_ERR_BVH_NO_SPLIT, "scene has no triangles");
+  if (total >= (1ull << 31)) return fail(CV_ERR_INVALID_ARGUMENT, "too many triangles");
   cv_scene* s = new cv_scene();
-  s->ntris = (uint32_t)mat.size();
+  s->ntris = (uint32_t)total;
   s->info.bins = nodes ? 0u : (opts && opts->builder ? opts->builder : 64u);
   // Camera::new (scene.rs:33-42)
   s->cam.q[0] = 1.0f;
@@ -646,7 +759,7 @@ static cv_status scene_create_impl(const cv_mesh* const* meshes, size_t n,
     delete s;
     return hip_fail(e, "hipStreamCreate");
   }
-  cv_status st = scene_finish(s, v9, uv6, mat, nodes, nnodes, order);
+  cv_status st = scene_finish(s, meshes, n, nodes, nnodes, order);
   if (st != CV_OK) {
     cv_scene_destroy(s);
     return st;
@@ -699,12 +812,10 @@ cv_status cv_scene_get_bvh_info(const cv_scene* s, cv_bvh_info* info) {
 
 cv_status cv_scene_copy_bvh(const cv_scene* s, cv_bvh_node* nodes, uint32_t* order) {
   if (!s) return fail(CV_ERR_INVALID_ARGUMENT, "null scene");
-  if (nodes)
-    HIPTRY(hipMemcpy(nodes, s->nodes.p, (size_t)s->info.num_nodes * 32, hipMemcpyDeviceToHost),
-           "download");
-  if (order)
-    HIPTRY(hipMemcpy(order, s->tri_src.p, (size_t)s->ntris * 4, hipMemcpyDeviceToHost), "download");
-  return CV_OK;
+  const cvh::CallerRect down[2] = {
+      cvh::CallerRect::flat(nodes, s->nodes.p, nodes ? (size_t)s->info.num_nodes * 32 : 0),
+      cvh::CallerRect::flat(order, s->tri_src.p, order ? (size_t)s->ntris * 4 : 0)};
+  return cvh::copy_caller_rects(down, 2, false, s->stream);
 }
 
 void cv_scene_destroy(cv_scene* s) {

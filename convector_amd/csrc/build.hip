@@ -36,6 +36,10 @@
 // reference.
 #include <math.h>
 
+#include <algorithm>
+#include <exception>
+#include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "internal.hpp"
@@ -1204,15 +1208,18 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   using namespace bvh;
   res->error = 0;
   if (nbins != 16 && nbins != 32 && nbins != 64) return hipErrorInvalidValue;
-  std::vector<void*> allocs;
+  // One allocation for all scratch: every hipMalloc / hipFree of the build's
+  // 26 buffers waits for the device.  The first pass over the requests (base
+  // null) adds up the sizes.
+  char* arena = nullptr;
+  size_t arena_bytes = 0;
   auto cleanup = [&]() {
-    for (void* p : allocs) (void)hipFree(p);
-    allocs.clear();
+    if (arena) (void)hipFree(arena);
+    arena = nullptr;
   };
-  auto alloc = [&](void** p, size_t bytes) -> hipError_t {
-    hipError_t e = hipMalloc(p, bytes ? bytes : 16);
-    if (e == hipSuccess) allocs.push_back(*p);
-    return e;
+  auto take = [&](auto** p, size_t count) {
+    *p = reinterpret_cast<std::remove_reference_t<decltype(*p)>>(arena + arena_bytes);
+    arena_bytes += (count * sizeof(**p) + 255) / 256 * 256;
   };
   const size_t N = ntris;
   Args a{};
@@ -1221,17 +1228,6 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   a.small_max = nbins / 2;
   float4 *A, *B;
   float* C;
-  BVH_CHECK(alloc((void**)&A, N * sizeof(float4)));
-  BVH_CHECK(alloc((void**)&B, N * sizeof(float4)));
-  BVH_CHECK(alloc((void**)&C, N * sizeof(float)));
-  a.A = A;
-  a.B = B;
-  a.C = C;
-  for (int k = 0; k < 2; k++) BVH_CHECK(alloc((void**)&a.buf[k], N * 4));
-  for (int k = 0; k < 3; k++) {
-    BVH_CHECK(alloc((void**)&a.sorted[k], N * 4));
-    BVH_CHECK(alloc((void**)&a.tmp[k], N * 4));
-  }
   // Node ids: the levels take 1 + 2 S for S splits of nodes of more than 32
   // triangles, and each small subtree of n triangles reserves 2 (n - 1).
   // Those S splits form a full binary tree whose leaves are the small
@@ -1239,34 +1235,68 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   // their number - 1 and all ids together are 2 (singles + unsplit large
   // nodes + triangles of small subtrees) - 1 <= 2 N - 1.
   const size_t ninodes_cap = 2 * N + 2;
-  BVH_CHECK(alloc((void**)&a.nodes, ninodes_cap * sizeof(INode)));
   Ctx* ctx;
-  BVH_CHECK(alloc((void**)&ctx, sizeof(Ctx)));
-  a.ctx = ctx;
   const size_t list_cap = N / (a.small_max + 1) + 2;
-  uint32_t *listA, *listB, *small;
-  BVH_CHECK(alloc((void**)&listA, list_cap * 4));
-  BVH_CHECK(alloc((void**)&listB, list_cap * 4));
-  BVH_CHECK(alloc((void**)&small, (N / 2 + 2) * 4));
-  a.small_list = small;
+  uint32_t *listA, *listB, *small, *dcount, *dlist;
   // chunks of the wide nodes of one level: their triangles are disjoint, so
   // at most N / kChunk + (number of wide nodes) chunks
   const size_t max_chunks = N / kChunk + N / kWide + 2;
-  BVH_CHECK(alloc((void**)&a.chunk_node, max_chunks * 4));
-  BVH_CHECK(alloc((void**)&a.part, max_chunks * kBinWords * 4));
-  BVH_CHECK(alloc((void**)&a.offs, max_chunks * 64 * 4));
-  BVH_CHECK(alloc((void**)&a.side, max_chunks * 24 * 4));
-  // TreeSAH power tables with the C library (same values as the CPU build)
-  std::vector<float> tpm(N + 1), tpm1(N + 1);
-  for (size_t n = 1; n <= N; n++) {
-    float m = log2f((float)n);
-    tpm[n] = powf(0.8f, m);
-    tpm1[n] = powf(0.8f, m - 1.0f);
-  }
-  tpm[0] = tpm1[0] = 0.0f;
+  // depths: at most one level per triangle
+  const size_t dcount_cap = N + 64;
   float *d_tpm, *d_tpm1;
-  BVH_CHECK(alloc((void**)&d_tpm, (N + 1) * 4));
-  BVH_CHECK(alloc((void**)&d_tpm1, (N + 1) * 4));
+  for (int pass = 0; pass < 2; pass++) {
+    arena_bytes = 0;
+    take(&A, N);
+    take(&B, N);
+    take(&C, N);
+    for (int k = 0; k < 2; k++) take(&a.buf[k], N);
+    for (int k = 0; k < 3; k++) {
+      take(&a.sorted[k], N);
+      take(&a.tmp[k], N);
+    }
+    take(&a.nodes, ninodes_cap);
+    take(&ctx, 1);
+    take(&listA, list_cap);
+    take(&listB, list_cap);
+    take(&small, N / 2 + 2);
+    take(&a.chunk_node, max_chunks);
+    take(&a.part, max_chunks * kBinWords);
+    take(&a.offs, max_chunks * 64);
+    take(&a.side, max_chunks * 24);
+    take(&d_tpm, N + 1);
+    take(&d_tpm1, N + 1);
+    take(&dcount, dcount_cap);
+    take(&dlist, ninodes_cap);
+    if (pass == 0) BVH_CHECK(hipMalloc((void**)&arena, arena_bytes));
+  }
+  a.A = A;
+  a.B = B;
+  a.C = C;
+  a.ctx = ctx;
+  a.small_list = small;
+  // TreeSAH power tables with the C library (same values as the CPU build)
+  // (two powf and a log2f per triangle count: 33 ms for 1.33 M counts on one
+  // thread, so large tables are filled by up to 8)
+  std::vector<float> tpm(N + 1), tpm1(N + 1);
+  auto fill = [&](size_t lo, size_t hi) {
+    for (size_t n = lo; n < hi; n++) {
+      float m = log2f((float)n);
+      tpm[n] = powf(0.8f, m);
+      tpm1[n] = powf(0.8f, m - 1.0f);
+    }
+  };
+  tpm[0] = tpm1[0] = 0.0f;
+  const size_t parts = std::min<size_t>(8, N / 16384 + 1), per = N / parts + 1;
+  std::vector<std::thread> workers;
+  size_t first = 1;
+  try {
+    for (size_t k = 1; k < parts; k++, first += per)
+      workers.emplace_back(fill, first, std::min(first + per, N + 1));
+  } catch (const std::exception&) {
+    // no thread to be had: the rest of the table is filled here
+  }
+  fill(first, N + 1);
+  for (std::thread& w : workers) w.join();
   BVH_CHECK(hipMemcpyAsync(d_tpm, tpm.data(), (N + 1) * 4, hipMemcpyHostToDevice, s));
   BVH_CHECK(hipMemcpyAsync(d_tpm1, tpm1.data(), (N + 1) * 4, hipMemcpyHostToDevice, s));
   a.tpm = d_tpm;
@@ -1384,9 +1414,6 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   // depths: the level phase's nodes lie at most `levels` deep and a small
   // subtree of at most 32 triangles adds at most 31 levels
   const uint32_t dcap = levels + 34;
-  uint32_t *dcount, *dlist;
-  BVH_CHECK(alloc((void**)&dcount, (size_t)dcap * 4));
-  BVH_CHECK(alloc((void**)&dlist, (size_t)ninodes * 4));
   BVH_CHECK(hipMemsetAsync(dcount, 0, (size_t)dcap * 4, s));
   hipLaunchKernelGGL(k_depth, dim3(blocks), dim3(256), 0, s, a, ninodes, dcount, dcap);
   BVH_CHECK(hipGetLastError());

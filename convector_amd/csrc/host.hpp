@@ -22,10 +22,21 @@ cv_status hip_fail(hipError_t e, const char* what);
 cv_status ensure_device();
 uint32_t num_cus();
 const char* last_error();
+// `rows` rows of `bytes` bytes of caller host memory and their place on the
+// device.
+struct CallerRect {
+  void* host;
+  void* dev;
+  size_t bytes, rows, host_pitch, dev_pitch;
+  static CallerRect flat(const void* host, void* dev, size_t bytes) {
+    return CallerRect{const_cast<void*>(host), dev, bytes, 1, bytes, bytes};
+  }
+};
 // Copies between caller host memory and the device through a pinned bounce
-// buffer, a chunk at a time, waiting for each chunk (and so for the work
-// queued before it on st): the runtime never copies from or to the caller's
+// buffer, a piece at a time, waiting for the copies (and so for the work
+// queued before them on st): the runtime never copies from or to the caller's
 // pageable memory, and nothing touches that memory after the call returns.
+cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st);
 cv_status copy_caller_memory(void* dst, const void* src, size_t bytes, bool to_device,
                              hipStream_t st);
 

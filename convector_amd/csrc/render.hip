@@ -95,6 +95,14 @@ struct StepHeader {
   uint32_t jobs;
 };
 
+// The counters at the end of Ctrl's first part, read back after the steps.
+struct StepTotals {
+  unsigned long long sum_aabb, sum_tri, total_rays;
+};
+static_assert(offsetof(cvk::Ctrl, total_rays) - offsetof(cvk::Ctrl, sum_aabb) ==
+                  offsetof(StepTotals, total_rays),
+              "the counters follow each other");
+
 }  // namespace
 
 // Queues, control block, job table and the staging of one pipeline.  Owned
@@ -108,6 +116,7 @@ struct Pipeline {
   DevBuf<cvk::Ctrl> ctrl;
   DevBuf<cvk::JobDesc> jobs[kRingSlots];
   size_t max_jobs = 0;
+  HostBuf<StepTotals> totals;
   HostBuf<StepHeader> head[kRingSlots];
   HostBuf<cvk::JobDesc> stage[kRingSlots];
   hipEvent_t slot_done[kRingSlots] = {};
@@ -142,6 +151,7 @@ struct Pipeline {
     }
     hits.reset();
     ctrl.reset();
+    totals.reset();
     spill.reset();
     sort_keys.reset();
     sort_order.reset();
@@ -163,6 +173,7 @@ struct Pipeline {
   cv_status init() {
     HIPTRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
     HIPTRY(ctrl.alloc(1), "alloc ctrl");
+    HIPTRY(totals.reserve(1), "pinned alloc");
     for (uint32_t k = 0; k < kRingSlots; k++) {
       HIPTRY(hipEventCreateWithFlags(&slot_done[k], hipEventDisableTiming), "event");
       HIPTRY(head[k].reserve(1), "pinned alloc");
@@ -502,6 +513,9 @@ cv_status pipeline_run(Pipeline& p, const std::vector<StepPlan>& steps, const Ru
     }
   }
   (void)hipEventRecord(t1, st);
+  // the counters come back with the wait for the steps
+  hipError_t te = hipMemcpyAsync(p.totals.p, &p.ctrl.p->sum_aabb, sizeof(StepTotals),
+                                 hipMemcpyDeviceToHost, st);
   hipError_t se = hipStreamSynchronize(st);
   if (status == CV_OK && se != hipSuccess) status = hip_fail(se, "render");
   cv_render_stats stt{};
@@ -530,13 +544,10 @@ cv_status pipeline_run(Pipeline& p, const std::vector<StepPlan>& steps, const Ru
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
   if (!timing) stt.extend_launches = (uint64_t)nsteps * o.max_bounces;
-  if (status == CV_OK) {
-    cvk::Ctrl hc;
-    if (hipMemcpy(&hc, p.ctrl.p, sizeof hc, hipMemcpyDeviceToHost) == hipSuccess) {
-      stt.sum_numi_aabb = hc.sum_aabb;
-      stt.sum_numi_tri = hc.sum_tri;
-      stt.extend_rays = hc.total_rays;
-    }
+  if (status == CV_OK && te == hipSuccess) {
+    stt.sum_numi_aabb = p.totals.p->sum_aabb;
+    stt.sum_numi_tri = p.totals.p->sum_tri;
+    stt.extend_rays = p.totals.p->total_rays;
   }
   if (out) *out = stt;
   return status;
@@ -687,11 +698,12 @@ cv_status run_frames(cv_renderer* r, const Rect& rc, uint32_t first, uint32_t nf
   float* hdr_dev = nullptr;
   if (hdr_mode) {
     hdr_dev = dev ? hdr : r->hdr.p;
-    if (!dev)
-      HIPTRY(hipMemcpy2DAsync((char*)r->hdr.p + rect_blk_off, blk_row_bytes,
-                              (const char*)hdr + rect_blk_off, blk_row_bytes, rect_blk_w, rc.h / 4,
-                              hipMemcpyHostToDevice, st),
-             "upload hdr");
+    if (!dev) {
+      const cvh::CallerRect up{(char*)hdr + rect_blk_off, (char*)r->hdr.p + rect_blk_off, rect_blk_w,
+                               rc.h / 4,                  blk_row_bytes,                  blk_row_bytes};
+      cv_status us = cvh::copy_caller_rects(&up, 1, true, st);
+      if (us != CV_OK) return us;
+    }
   }
   uint32_t* bm_dev = nullptr;
   if (bitmap) bm_dev = dev ? bitmap : r->bitmap.p;
@@ -704,8 +716,8 @@ cv_status run_frames(cv_renderer* r, const Rect& rc, uint32_t first, uint32_t nf
       ft_dev = features;
     } else {
       if (r->features.n < npix_all * 8) HIPTRY(r->features.alloc(npix_all * 8), "alloc features");
-      HIPTRY(hipMemcpyAsync(r->features.p, features, npix_all * 32, hipMemcpyHostToDevice, st),
-             "upload features");
+      cv_status us = cvh::copy_caller_memory(r->features.p, features, npix_all * 32, true, st);
+      if (us != CV_OK) return us;
       ft_dev = r->features.p;
     }
   }
@@ -796,29 +808,15 @@ cv_status run_frames(cv_renderer* r, const Rect& rc, uint32_t first, uint32_t nf
   if (status == CV_OK && !dev) {
     const size_t row = (size_t)W * 4;
     const size_t off = ((size_t)rc.y * W + rc.x) * 4;
-    if (hdr_mode)
-      status = hipMemcpy2DAsync((char*)hdr + rect_blk_off, blk_row_bytes,
-                                (const char*)r->hdr.p + rect_blk_off, blk_row_bytes, rect_blk_w,
-                                rc.h / 4, hipMemcpyDeviceToHost, st) == hipSuccess
-                   ? CV_OK
-                   : fail(CV_ERR_DEVICE, "download hdr");
-    if (status == CV_OK && bitmap)
-      status = hipMemcpy2DAsync((char*)bitmap + off, row, (const char*)r->bitmap.p + off, row,
-                                (size_t)rc.w * 4, rc.h, hipMemcpyDeviceToHost, st) == hipSuccess
-                   ? CV_OK
-                   : fail(CV_ERR_DEVICE, "download bitmap");
-    if (status == CV_OK && gbuffer)
-      status = hipMemcpy2DAsync((char*)gbuffer + off, row, (const char*)r->gbuffer.p + off, row,
-                                (size_t)rc.w * 4, rc.h, hipMemcpyDeviceToHost, st) == hipSuccess
-                   ? CV_OK
-                   : fail(CV_ERR_DEVICE, "download gbuffer");
-    if (status == CV_OK && features)
-      status = hipMemcpyAsync(features, r->features.p, npix_all * 32, hipMemcpyDeviceToHost, st) ==
-                       hipSuccess
-                   ? CV_OK
-                   : fail(CV_ERR_DEVICE, "download features");
-    hipError_t se = hipStreamSynchronize(st);
-    if (status == CV_OK && se != hipSuccess) status = hip_fail(se, "download");
+    std::vector<cvh::CallerRect> down;
+    auto rect = [&](void* h, void* d, size_t o, size_t bytes, size_t rows, size_t pitch) {
+      down.push_back(cvh::CallerRect{(char*)h + o, (char*)d + o, bytes, rows, pitch, pitch});
+    };
+    if (hdr_mode) rect(hdr, r->hdr.p, rect_blk_off, rect_blk_w, rc.h / 4, blk_row_bytes);
+    if (bitmap) rect(bitmap, r->bitmap.p, off, (size_t)rc.w * 4, rc.h, row);
+    if (gbuffer) rect(gbuffer, r->gbuffer.p, off, (size_t)rc.w * 4, rc.h, row);
+    if (features) rect(features, r->features.p, 0, npix_all * 32, 1, npix_all * 32);
+    status = cvh::copy_caller_rects(down.data(), down.size(), false, st);
   }
   return status;
 }
@@ -944,12 +942,13 @@ cv_status cv_renderer_buffer_f32_into_bitmap(cv_renderer* r, const float* hdr, u
   const float* hp = hdr;
   uint32_t* bp = bitmap;
   if (!dev) {
-    HIPTRY(hipMemcpyAsync(r->hdr.p, hdr, npix * 12, hipMemcpyHostToDevice, st), "upload");
+    cv_status us = cvh::copy_caller_memory(r->hdr.p, hdr, npix * 12, true, st);
+    if (us != CV_OK) return us;
     hp = r->hdr.p;
     bp = r->bitmap.p;
   }
   HIPTRY(cvk::launch_hdr_to_bitmap(hp, bp, r->width, r->height, num_samples, st), "convert");
-  if (!dev) HIPTRY(hipMemcpyAsync(bitmap, bp, npix * 4, hipMemcpyDeviceToHost, st), "download");
+  if (!dev) return cvh::copy_caller_memory(bitmap, bp, npix * 4, false, st);
   HIPTRY(hipStreamSynchronize(st), "sync");
   return CV_OK;
 }
@@ -1430,8 +1429,8 @@ cv_status finish_request(cv_server* sv, cv_denoiser* dn, ServeReq& r) {
   const bool dev = q.flags & CV_PTR_DEVICE;
   if (q.denoise && dn)
     return cvh::denoise_image(dn, r.hdr.p, r.feat.p, q.width, q.height, q.spp, q.hdr, dev);
-  HIPTRY(hipMemcpyAsync(q.hdr, r.hdr.p, npix * 12, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
-                        sv->fin_stream),
+  if (!dev) return cvh::copy_caller_memory(q.hdr, r.hdr.p, npix * 12, false, sv->fin_stream);
+  HIPTRY(hipMemcpyAsync(q.hdr, r.hdr.p, npix * 12, hipMemcpyDeviceToDevice, sv->fin_stream),
          "deliver result");
   HIPTRY(hipStreamSynchronize(sv->fin_stream), "deliver result");
   return CV_OK;
