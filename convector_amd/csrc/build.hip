@@ -356,10 +356,11 @@ __global__ __launch_bounds__(BS) void k_decide(Args a) {
   const uint32_t umask = a.mode == 1 ? nd->uniform_mask : 0u;
   __shared__ uint32_t cnt[3][64];
   __shared__ uint32_t bx[3][64][6];
-  __shared__ float cost[3][64];
-  __shared__ uint32_t valid_axes;
+  __shared__ float axis_cost[3];     // the cheapest position of each axis (64: none),
+  __shared__ uint32_t axis_pos[3];   // its cost and the triangles left of it
+  __shared__ uint32_t axis_left[3];
+  __shared__ bool deferred;
   __shared__ int s_axis;
-  __shared__ uint32_t s_bin;
   const uint32_t tid = threadIdx.x;
   const uint32_t nch = nd->nchunks, cbase = nd->chunk_base;
   clear_bins<BS>(cnt, bx);
@@ -445,73 +446,81 @@ __global__ __launch_bounds__(BS) void k_decide(Args a) {
         nd->flags = flags | kPending;
       }
     }
-    if (lane == 0) valid_axes = fb ? 0xffffffffu : 0u;  // reuse as "deferred" marker
+    if (lane == 0) deferred = fb != 0;
   }
   __syncthreads();
-  if (a.mode == 0 && valid_axes == 0xffffffffu) return;
-  // split costs (find_cheapest_split, bvh.rs:218-261), one lane per position
+  if (a.mode == 0 && deferred) return;
+  // split costs (find_cheapest_split, bvh.rs:218-261): a wave per axis (or
+  // one wave axis by axis), one lane per position.  Lane i holds bin i, and
+  // the boxes and counts left of position i (bins below i) and right of it
+  // are scans over the lanes (ordered min / max and sums: any order gives the
+  // same values).  Every lane walking all 64 bins by itself and one thread
+  // comparing the costs took 52 us a launch on the levels of a 20,506-triangle
+  // build, the scans 13 us.
   const float parent_area = area6(nd->box);
-  if (tid < 64) {
-    const uint32_t i = tid;
-    uint32_t va = 0;
-    for (uint32_t axis = 0; axis < 3; axis++) {
-      uint64_t ne = __ballot(cnt[axis][i] != 0);
-      uint32_t first = __ffsll((unsigned long long)ne);  // first non-empty + 1
-      uint32_t last = 64 - __clzll((long long)ne);        // last non-empty + 1
-      bool valid = __popcll(ne) > 1;
-      if (valid) va |= 1u << axis;
-      float cst = 0.0f;
-      if (valid && i >= first && i < last) {
-        float lb[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        float rb[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        uint32_t lc = 0, rc = 0;
-        for (uint32_t j = 0; j < 64; j++) {
-          uint32_t cj = cnt[axis][j];
-          if (!cj) continue;
-          float* tb = j < i ? lb : rb;
-          for (int k = 0; k < 3; k++) {
-            tb[k] = tmin_f(tb[k], okey_dec(bx[axis][j][k]));
-            tb[3 + k] = tmax_f(tb[3 + k], okey_dec(bx[axis][j][3 + k]));
-          }
-          if (j < i)
-            lc += cj;
-          else
-            rc += cj;
-        }
-        cst = tree_sah(a, parent_area, lb, lc) + tree_sah(a, parent_area, rb, rc);
+  for (uint32_t axis = tid >> 6; axis < 3; axis += BS / 64) {
+    const uint32_t i = tid & 63u;
+    const uint32_t ci = cnt[axis][i];
+    const uint64_t ne = __ballot(ci != 0);
+    const uint32_t first = __ffsll((unsigned long long)ne);  // first non-empty + 1
+    const uint32_t last = 64 - __clzll((long long)ne);        // last non-empty + 1
+    float pre[6], suf[6];
+    uint32_t below = ci;
+    for (int k = 0; k < 6; k++)
+      pre[k] = suf[k] = ci ? okey_dec(bx[axis][i][k]) : k < 3 ? INFINITY : -INFINITY;
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+      const uint32_t cu = __shfl_up(below, d);
+      if (i >= d) below += cu;
+      for (int k = 0; k < 6; k++) {
+        const float up = __shfl_up(pre[k], d), dn = __shfl_down(suf[k], d);
+        if (i >= d) pre[k] = k < 3 ? tmin_f(pre[k], up) : tmax_f(pre[k], up);
+        if (i + d < 64) suf[k] = k < 3 ? tmin_f(suf[k], dn) : tmax_f(suf[k], dn);
       }
-      cost[axis][i] = cst;
     }
-    if (i == 0) valid_axes = va;
+    float lb[6];
+    for (int k = 0; k < 6; k++) lb[k] = __shfl_up(pre[k], 1);
+    below -= ci;
+    float cst = 0.0f;
+    bool in = __popcll(ne) > 1 && i >= first && i < last;
+    if (in) cst = tree_sah(a, parent_area, lb, below) + tree_sah(a, parent_area, suf, n - below);
+    // the reference scans the positions upward and replaces its choice only
+    // by a strictly smaller cost, so that a NaN is chosen at the first
+    // position only, and then for good
+    uint32_t pos = 64;
+    if (in && (cst == cst || i == first)) pos = i;
+    const bool nan_first = __any(in && i == first && cst != cst);
+    for (uint32_t d = 32; d > 0; d >>= 1) {
+      const float cd = __shfl_xor(cst, d);
+      const uint32_t pd = __shfl_xor(pos, d);
+      if (pd < 64 && (pos == 64 || cd < cst || (cd == cst && pd < pos))) {
+        cst = cd;
+        pos = pd;
+      }
+    }
+    if (nan_first) {
+      pos = first;
+      cst = NAN;
+    }
+    if (i == 0) {
+      axis_pos[axis] = pos;
+      axis_cost[axis] = cst;
+    }
+    if (i == pos) axis_left[axis] = below;
   }
   __syncthreads();
   if (tid == 0) {
-    // the reference's scan order: axes X, Y, Z; positions ascending;
-    // replace only on a strictly smaller cost
+    // the reference's scan order: axes X, Y, Z; replace only on a strictly
+    // smaller cost
     int best_axis = -1;
-    uint32_t best_i = 0;
+    uint32_t best_i = 0, best_left = 0;
     float best = 0.0f;
     for (uint32_t axis = 0; axis < 3; axis++) {
-      if (!((valid_axes >> axis) & 1u)) continue;
-      int abest = -1;
-      float acost = 0.0f;
-      uint32_t first = 64, last = 0;
-      for (uint32_t j = 0; j < 64; j++)
-        if (cnt[axis][j]) {
-          if (first == 64) first = j + 1;
-          last = j + 1;
-        }
-      for (uint32_t j = first; j < last; j++) {
-        float c = cost[axis][j];
-        if (abest < 0 || c < acost) {
-          acost = c;
-          abest = (int)j;
-        }
-      }
-      if (best_axis < 0 || acost < best) {
-        best = acost;
+      if (axis_pos[axis] >= 64) continue;
+      if (best_axis < 0 || axis_cost[axis] < best) {
+        best = axis_cost[axis];
         best_axis = (int)axis;
-        best_i = (uint32_t)abest;
+        best_i = axis_pos[axis];
+        best_left = axis_left[axis];
       }
     }
     uint32_t f = flags & ~kPending;
@@ -522,15 +531,12 @@ __global__ __launch_bounds__(BS) void k_decide(Args a) {
     } else if ((float)n * 120.0f < best) {
       f |= kLeaf;  // bvh.rs:311-314
     } else {
-      uint32_t lc = 0;
-      for (uint32_t j = 0; j < best_i; j++) lc += cnt[best_axis][j];
       nd->axis = (uint32_t)best_axis;
       nd->split_bin = best_i;
-      nd->left_count = lc;
+      nd->left_count = best_left;
       if (a.mode == 0) nd->uniform_mask = 0;
       f |= kSplit;
       s_axis = best_axis;
-      s_bin = best_i;
     }
     nd->flags = f;
   }
@@ -834,27 +840,18 @@ __global__ __launch_bounds__(BS) void k_partition(Args a) {
 }
 
 // ---------------------------------------------------------------------------
-// k_small: one wave finishes the subtree of a node of 2..32 triangles.  With
-// at most 32 triangles every split uses sorted single-triangle bins
-// (bvh.rs:145-147), so a node is three sorts of the lanes and two scans.
-// A sort ranks each lane of the node's segment [off, off + cnt) by its key
-// (ties by lane: the stable order) with cnt readlanes, and one ds_permute
-// sends every lane to its rank; lanes outside the segment keep their place.
+// k_small: finishes the subtrees of nodes of 2..32 triangles, two per wave (32
+// lanes each), breadth first: the lanes hold the triangles of all nodes of one
+// depth, each node a segment [off, off + cnt) of consecutive lanes, and every
+// sort and scan runs over all segments at once.  With at most 32 triangles
+// every split uses sorted single-triangle bins (bvh.rs:145-147), so a depth is
+// three sorts of the lanes and two scans.  A sort ranks each lane within its
+// segment by its key (ties by lane: the stable order), and one ds_permute
+// sends every lane to its rank; lanes of finished nodes keep their place.
+// Bound by the latency of the lane exchanges: node after node in depth-first
+// order, one subtree a wave, took 7.06 ms for 1.33 M triangles and 490 us for
+// 20,506, now 0.65 ms and 128 us.
 // ---------------------------------------------------------------------------
-
-__device__ __forceinline__ uint32_t stable_rank_src(uint32_t key, bool inside, uint32_t off,
-                                                    uint32_t cnt, uint32_t lane) {
-  uint32_t rank = lane;
-  if (inside) {
-    rank = off;
-    for (uint32_t j = off; j < off + cnt; j++) {
-      const uint32_t kj = __builtin_amdgcn_readlane(key, j);
-      rank += (kj < key || (kj == key && j < lane)) ? 1u : 0u;
-    }
-  }
-  // lane `rank` receives this lane's index: the source of each sorted position
-  return (uint32_t)__builtin_amdgcn_ds_permute((int)(rank * 4), (int)lane);
-}
 
 // tree_sah with the power terms of counts up to 32 from LDS
 __device__ __forceinline__ float tree_sah_small(const float (*tp)[33], float parent_area,
@@ -868,183 +865,169 @@ __device__ __forceinline__ float tree_sah_small(const float (*tp)[33], float par
 }
 
 __global__ __launch_bounds__(256) void k_small(Args a) {
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t lane = threadIdx.x & 63, half = lane >> 5;
   __shared__ float tp[2][33];
   if (threadIdx.x < 66) {
     const uint32_t k = threadIdx.x % 33;
     tp[threadIdx.x / 33][k] = k <= a.ntris ? (threadIdx.x < 33 ? a.tpm[k] : a.tpm1[k]) : 0.0f;
   }
   __syncthreads();
-  const uint32_t si = blockIdx.x * 4 + wave;
-  if (si >= a.ctx->small_count) return;
-  const uint32_t root = a.small_list[si];
-  const INode R = a.nodes[root];
-  const uint32_t n = R.count;
-  const uint32_t sbegin = R.begin;
-  const uint32_t par = (R.flags & kParity) ? 1u : 0u;
-  uint32_t* seg = a.buf[par] + sbegin;
+  const uint32_t si = blockIdx.x * 8 + (threadIdx.x >> 5);
+  const bool here = si < a.ctx->small_count;
+  uint32_t root = 0, n = 0, sbegin = 0, rflags = 0;
+  int32_t parent = -1;
+  float box[6] = {0, 0, 0, 0, 0, 0};
+  if (here) {
+    root = a.small_list[si];
+    const INode& R = a.nodes[root];
+    n = R.count;
+    sbegin = R.begin;
+    rflags = R.flags;
+    parent = R.parent;
+    for (int k = 0; k < 6; k++) box[k] = R.box[k];
+  }
+  const uint32_t par = rflags & kParity;
+  uint32_t* seg = a.buf[par ? 1 : 0] + sbegin;
+  const uint32_t pos = lane & 31u;
   uint32_t ref = 0;
   float bmn[3] = {0, 0, 0}, bmx[3] = {0, 0, 0}, c[3] = {0, 0, 0};
-  if (lane < n) {
-    ref = seg[lane];
+  bool open = here && pos < n;
+  if (open) {
+    ref = seg[pos];
     float4 A = a.A[ref], B = a.B[ref];
     bmn[0] = A.x; bmn[1] = A.y; bmn[2] = A.z;
     bmx[0] = B.x; bmx[1] = B.y; bmx[2] = B.z;
     c[0] = A.w; c[1] = B.w; c[2] = a.C[ref];
   }
   // The subtree has at most n - 1 inner nodes, so its nodes take ids from
-  // 2 (n - 1) reserved with one atomic (one counter for every wave would
+  // 2 (n - 1) reserved with one atomic (one counter for every node would
   // serialise them); ids left over are written as holes at the end.
   uint32_t ids = 0;
-  if (lane == 0) ids = atomicAdd(&a.ctx->node_count, 2u * (n - 1u));
-  ids = __shfl(ids, 0);
-  const uint32_t ids_end = ids + 2u * (n - 1u);
-  // Pending nodes: off, cnt, id, parent, base flags, outer box.  Every node
-  // record of the subtree is written once, when its node is popped.
-  __shared__ uint32_t stk[4][40][11];
-  if (lane == 0) {
-    uint32_t* e = stk[wave][0];
-    e[0] = 0; e[1] = n; e[2] = root; e[3] = (uint32_t)R.parent; e[4] = R.flags;
-    for (int k = 0; k < 6; k++) e[5 + k] = f2u(R.box[k]);
-  }
-  __builtin_amdgcn_wave_barrier();
-  int sp = 1;
-  while (sp > 0) {
-    sp--;
-    // the entry is the same for the whole wave: scalar values, so that the
-    // loops over the segment below are scalar loops with readlanes
-    const uint32_t* e = stk[wave][sp];
-    const uint32_t off = __builtin_amdgcn_readfirstlane(e[0]);
-    const uint32_t cnt = __builtin_amdgcn_readfirstlane(e[1]);
-    const uint32_t id = __builtin_amdgcn_readfirstlane(e[2]);
-    const int32_t parent = (int32_t)__builtin_amdgcn_readfirstlane(e[3]);
-    const uint32_t bflags = __builtin_amdgcn_readfirstlane(e[4]);
-    float nbox[6];
-    for (int k = 0; k < 6; k++) nbox[k] = u2f(e[5 + k]);
-    __builtin_amdgcn_wave_barrier();
-    auto write_node = [&](uint32_t flags, int32_t c0, int32_t c1) {
-      if (lane != 0) return;
-      INode w;
-      for (int k = 0; k < 6; k++) {
-        w.box[k] = nbox[k];
-        w.cbox[k] = id == root ? R.cbox[k] : 0.0f;
-      }
-      w.begin = sbegin + off;
-      w.count = cnt;
-      w.parent = parent;
-      w.child[0] = c0;
-      w.child[1] = c1;
-      w.flags = flags;
-      w.leaves = 0;
-      w.sar = 0.0f;
-      w.depth = 0;
-      w.axis = w.split_bin = w.left_count = w.uniform_mask = 0;
-      w.chunk_base = w.nchunks = 0;
-      a.nodes[id] = w;
-    };
-    if (cnt <= 1) {
-      write_node(bflags | kLeaf, -1, -1);
-      continue;
+  if (here && pos == 0) ids = atomicAdd(&a.ctx->node_count, 2u * (n - 1u));
+  ids = __shfl(ids, (int)(half << 5));
+  const uint32_t ids_end = here ? ids + 2u * (n - 1u) : ids;
+  // the lane's node
+  uint32_t off = open ? half << 5 : lane, cnt = open ? n : 0u, id = root, flags = rflags;
+  auto write_node = [&](uint32_t f, int32_t c0, int32_t c1) {
+    INode& w = a.nodes[id];
+    for (int k = 0; k < 6; k++) w.box[k] = box[k];
+    w.begin = sbegin + (off & 31u);
+    w.count = cnt;
+    w.parent = parent;
+    w.child[0] = c0;
+    w.child[1] = c1;
+    w.flags = f;
+  };
+  while (__any(open)) {
+    if (open && cnt == 1) {
+      write_node(flags | kLeaf, -1, -1);
+      open = false;
     }
-    const float parent_area = area6(nbox);
-    const bool inside = lane >= off && lane < off + cnt;
-    uint32_t perm[3];
+    uint32_t most = open ? cnt : 0u;
+    for (int o = 32; o > 0; o >>= 1) most = max(most, (uint32_t)__shfl_xor(most, o));
+    most = __builtin_amdgcn_readfirstlane(most);
+    if (most == 0) break;
+    const uint32_t at = lane - off;  // position in the segment
+    const float parent_area = area6(box);
     int best_axis = -1;
-    uint32_t best_i = 0;
+    uint32_t best_i = 0, best_src = lane;
     float best = 0.0f;
+    float lb[6], rb[6];  // the best axis' prefix and suffix boxes at this lane
+    for (int k = 0; k < 6; k++) lb[k] = rb[k] = 0.0f;
     for (uint32_t axis = 0; axis < 3; axis++) {
-      const uint32_t src = stable_rank_src(sort_key(c[axis]), inside, off, cnt, lane);
-      perm[axis] = src;
-      float s[6];
-      for (int k = 0; k < 3; k++) {
-        s[k] = __shfl(bmn[k], (int)src);
-        s[3 + k] = __shfl(bmx[k], (int)src);
+      const uint32_t key = sort_key(axis == 0 ? c[0] : axis == 1 ? c[1] : c[2]);
+      uint32_t rank = 0;
+      for (uint32_t j = 0; j < most; j++) {
+        const uint32_t kj = __shfl(key, (int)(off + j));  // wraps beyond the wave: not used
+        rank += j < cnt && (kj < key || (kj == key && j < at)) ? 1u : 0u;
       }
+      // lane off + rank receives this lane's index: the source of each
+      // sorted position
+      const uint32_t src = (uint32_t)__builtin_amdgcn_ds_permute(
+          (int)((open ? off + rank : lane) * 4), (int)lane);
       float pre[6], suf[6];
-      for (int k = 0; k < 6; k++) {
-        float idv = k < 3 ? INFINITY : -INFINITY;
-        pre[k] = inside ? s[k] : idv;
-        suf[k] = pre[k];
+      for (int k = 0; k < 3; k++) {
+        pre[k] = suf[k] = __shfl(bmn[k], (int)src);
+        pre[3 + k] = suf[3 + k] = __shfl(bmx[k], (int)src);
       }
-      // the segment lies in lanes 0..31: scans over 32 lanes
-      for (uint32_t d = 1; d < 32; d <<= 1)
+      for (uint32_t d = 1; d < most; d <<= 1)
         for (int k = 0; k < 6; k++) {
-          float up = __shfl_up(pre[k], d);
-          float dn = __shfl_down(suf[k], d);
-          if (lane >= d) pre[k] = k < 3 ? tmin_f(pre[k], up) : tmax_f(pre[k], up);
-          if (lane + d < 32) suf[k] = k < 3 ? tmin_f(suf[k], dn) : tmax_f(suf[k], dn);
+          const float up = __shfl_up(pre[k], d), dn = __shfl_down(suf[k], d);
+          if (at >= d) pre[k] = k < 3 ? tmin_f(pre[k], up) : tmax_f(pre[k], up);
+          if (at + d < cnt) suf[k] = k < 3 ? tmin_f(suf[k], dn) : tmax_f(suf[k], dn);
         }
       float rsuf[6];
       for (int k = 0; k < 6; k++) rsuf[k] = __shfl_down(suf[k], 1);
+      // the cost of splitting after this lane, and its position (0: none);
+      // the reference scans the positions upward and replaces its choice only
+      // by a strictly smaller cost, so that a NaN is chosen at the first
+      // position only
       float cst = 0.0f;
-      if (lane >= off && lane + 1 < off + cnt) {
-        uint32_t lc = lane - off + 1;
-        cst = tree_sah_small(tp, parent_area, pre, lc) +
-              tree_sah_small(tp, parent_area, rsuf, cnt - lc);
+      uint32_t pick = 0;
+      if (open && at + 1 < cnt) {
+        cst = tree_sah_small(tp, parent_area, pre, at + 1) +
+              tree_sah_small(tp, parent_area, rsuf, cnt - at - 1);
+        pick = at == 0 || cst == cst ? at + 1 : 0u;
       }
-      // first strictly smallest position; then strictly smaller than earlier axes
-      int abest = -1;
-      float acost = 0.0f;
-      for (uint32_t k = off; k + 1 < off + cnt; k++) {
-        const float ck = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cst), k));
-        if (abest < 0 || ck < acost) {
-          acost = ck;
-          abest = (int)(k - off + 1);
+      for (uint32_t d = 1; d < most; d <<= 1) {
+        const float cd = __shfl_down(cst, d);
+        const uint32_t pd = __shfl_down(pick, d);
+        if (at + d < cnt && pd && (!pick || cd < cst)) {
+          cst = cd;
+          pick = pd;
         }
       }
-      if (best_axis < 0 || acost < best) {
+      const float acost = __shfl(cst, (int)off);
+      const uint32_t apick = __shfl(pick, (int)off);
+      if (open && (best_axis < 0 || acost < best)) {
         best = acost;
         best_axis = (int)axis;
-        best_i = (uint32_t)abest;
-      }
-    }
-    if ((float)cnt * 120.0f < best) {
-      write_node(bflags | kLeaf, -1, -1);
-      continue;
-    }
-    uint32_t p = best_axis == 0 ? perm[0] : best_axis == 1 ? perm[1] : perm[2];
-    ref = __shfl(ref, (int)p);
-    for (int k = 0; k < 3; k++) {
-      bmn[k] = __shfl(bmn[k], (int)p);
-      bmx[k] = __shfl(bmx[k], (int)p);
-      c[k] = __shfl(c[k], (int)p);
-    }
-    float cbx[2][6];
-    for (int side = 0; side < 2; side++) {
-      uint32_t lo = side == 0 ? off : off + best_i;
-      uint32_t hi = side == 0 ? off + best_i : off + cnt;
-      bool in = lane >= lo && lane < hi;
-      for (int k = 0; k < 6; k++) {
-        float v = k < 3 ? (in ? bmn[k] : INFINITY) : (in ? bmx[k - 3] : -INFINITY);
-        for (int o = 32; o > 0; o >>= 1) {
-          float w = __shfl_xor(v, o);
-          v = k < 3 ? tmin_f(v, w) : tmax_f(v, w);
+        best_i = apick;
+        best_src = src;
+        for (int k = 0; k < 6; k++) {
+          lb[k] = pre[k];
+          rb[k] = suf[k];
         }
-        cbx[side][k] = v;
       }
     }
-    const uint32_t cid = ids;
-    ids += 2;
-    // smaller area first (bvh.rs:337-345)
-    const bool swap = area6(cbx[0]) > area6(cbx[1]);
-    write_node((bflags & ~kLeaf) | kSplit, (int32_t)(swap ? cid + 1 : cid),
-               (int32_t)(swap ? cid : cid + 1));
-    if (lane == 0) {
-      for (int s = 0; s < 2; s++) {
-        uint32_t* q = stk[wave][sp + (s == 0 ? 1 : 0)];
-        q[0] = s == 0 ? off : off + best_i;
-        q[1] = s == 0 ? best_i : cnt - best_i;
-        q[2] = cid + s;
-        q[3] = id;
-        q[4] = (par ? kParity : 0u) | (((s == 1) != swap) ? kIsC1 : 0u);
-        for (int k = 0; k < 6; k++) q[5 + k] = f2u(cbx[s][k]);
-      }
+    if (open && (float)cnt * 120.0f < best) {
+      if (at == 0) write_node(flags | kLeaf, -1, -1);
+      open = false;
+      best_src = lane;
     }
-    __builtin_amdgcn_wave_barrier();
-    sp += 2;
+    // the triangles in the order of the chosen axis, the two children's
+    // boxes, ids and segments
+    ref = __shfl(ref, (int)best_src);
+    for (int k = 0; k < 3; k++) {
+      bmn[k] = __shfl(bmn[k], (int)best_src);
+      bmx[k] = __shfl(bmx[k], (int)best_src);
+      c[k] = __shfl(c[k], (int)best_src);
+    }
+    float cl[6], cr[6];
+    for (int k = 0; k < 6; k++) {
+      cl[k] = __shfl(lb[k], (int)(off + best_i - 1u));
+      cr[k] = __shfl(rb[k], (int)(off + best_i));
+    }
+    const uint32_t heads = (uint32_t)(__ballot(open && at == 0) >> (half << 5));
+    const uint32_t cid = ids + 2u * __popc(heads & ((1u << (off & 31u)) - 1u));
+    ids += 2u * __popc(heads);
+    if (open) {
+      // smaller area first (bvh.rs:337-345)
+      const bool swap = area6(cl) > area6(cr);
+      if (at == 0)
+        write_node((flags & ~kLeaf) | kSplit, (int32_t)(swap ? cid + 1 : cid),
+                   (int32_t)(swap ? cid : cid + 1));
+      const uint32_t side = at >= best_i ? 1u : 0u;
+      parent = (int32_t)id;
+      id = cid + side;
+      flags = par | (((side == 1) != swap) ? kIsC1 : 0u);
+      off += side ? best_i : 0u;
+      cnt = side ? cnt - best_i : best_i;
+      for (int k = 0; k < 6; k++) box[k] = side ? cr[k] : cl[k];
+    }
   }
-  if (lane < n) seg[lane] = ref;
-  for (uint32_t h = ids + lane; h < ids_end; h += 64) {
+  if (here && pos < n) seg[pos] = ref;
+  for (uint32_t h = ids + pos; h < ids_end; h += 32) {
     INode w{};
     w.flags = kHole;
     w.parent = -1;
@@ -1386,7 +1369,7 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   BVH_CHECK(hipMemcpyAsync(&hc, ctx, sizeof(Ctx), hipMemcpyDeviceToHost, s));
   BVH_CHECK(hipStreamSynchronize(s));
   if (hc.error == 0 && hc.small_count > 0) {
-    hipLaunchKernelGGL(k_small, dim3((hc.small_count + 3) / 4), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_small, dim3((hc.small_count + 7) / 8), dim3(256), 0, s, a);
     BVH_CHECK(hipGetLastError());
   }
   BVH_CHECK(hipMemcpyAsync(&hc, ctx, sizeof(Ctx), hipMemcpyDeviceToHost, s));
