@@ -53,7 +53,7 @@ constexpr uint32_t kHole = 32;
 constexpr uint32_t kBlock = 512;
 constexpr uint32_t kChunk = 2048;   // references per chunk of a wide node
 constexpr uint32_t kWide = 4096;    // nodes above this many triangles are chunked
-constexpr uint32_t kNarrow = 2048;  // levels with no larger node use 64-thread blocks
+constexpr uint32_t kSub = 1024;     // nodes of at most this many triangles go to k_subtree
 constexpr uint32_t kBinWords = 3 * 64 * 7;  // counts, then outer bounds, of 3 x 64 bins
 
 struct INode {
@@ -77,7 +77,8 @@ struct Ctx {
   uint32_t error;
   uint32_t next_wide;     // wide nodes in the next level's list
   uint32_t total_chunks;  // chunks of the current level
-  uint32_t next_max;      // largest triangle count in the next level's list
+  uint32_t sub_count;     // nodes for k_subtree
+  uint32_t sub_levels;    // most levels that a subtree of k_subtree took
   uint32_t max_depth;
   uint32_t max_leaf;
   uint32_t root_box[6];   // okeys
@@ -96,6 +97,7 @@ struct Args {
   const uint32_t* list;
   uint32_t nlist;
   uint32_t* next_list;
+  uint32_t* sub_list;
   uint32_t* small_list;
   const float* tpm;   // powf(0.8f, log2f(n))
   const float* tpm1;  // powf(0.8f, log2f(n) - 1.0f)
@@ -234,13 +236,44 @@ __global__ void k_root(INode* nodes, Ctx* ctx, uint32_t n) {
   ctx->node_count = 1;
 }
 
+// The helpers below run on a group of BS threads: a workgroup, or (BS == 64)
+// one wave of a workgroup of any size.
+template <uint32_t BS>
+__device__ __forceinline__ uint32_t group_tid() {
+  return BS == 64 ? threadIdx.x & 63u : threadIdx.x;
+}
+// Orders the group's memory accesses; a wave's lanes run in step, so it needs
+// the waits only.
+template <uint32_t BS>
+__device__ __forceinline__ void group_sync() {
+  if (BS == 64) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// Grows a bin's bounds (LDS).  Few triangles of a bin move its bounds, and
+// the atomics of many lanes on one bin follow each other, so a bound is read
+// first (the reads of one bin are a broadcast) and left alone when the
+// triangle lies within: a stale value is only further in, never past the
+// bound, so nothing is missed.
+__device__ __forceinline__ void grow_bin(uint32_t* b, const uint32_t* kmn, const uint32_t* kmx) {
+  volatile uint32_t* v = b;
+  for (int j = 0; j < 3; j++) {
+    if (kmn[j] < v[j]) atomicMin(&b[j], kmn[j]);
+    if (kmx[j] > v[3 + j]) atomicMax(&b[3 + j], kmx[j]);
+  }
+}
+
 // Centroid bins of refs[0, n) on the axes not in umask (bin_triangles,
 // bvh.rs:149-156): counts and outer bounds as ordered integers in LDS.
 template <uint32_t BS>
 __device__ __forceinline__ void bin_centroids(const Args& a, const uint32_t* refs, uint32_t n,
                                               const float* cmn, const float* csz, uint32_t umask,
                                               uint32_t (*cnt)[64], uint32_t (*bx)[64][6]) {
-  for (uint32_t e = threadIdx.x; e < n; e += BS) {
+  for (uint32_t e = group_tid<BS>(); e < n; e += BS) {
     uint32_t r = refs[e];
     float4 A = a.A[r], B = a.B[r];
     float cz = a.C[r];
@@ -251,19 +284,126 @@ __device__ __forceinline__ void bin_centroids(const Args& a, const uint32_t* ref
       if ((umask >> axis) & 1u) continue;
       uint32_t b = centroid_bin(c[axis], cmn[axis], csz[axis], a.nbins);
       atomicAdd(&cnt[axis][b], 1u);
-      for (int j = 0; j < 3; j++) {
-        atomicMin(&bx[axis][b][j], kmn[j]);
-        atomicMax(&bx[axis][b][3 + j], kmx[j]);
-      }
+      grow_bin(bx[axis][b], kmn, kmx);
     }
   }
 }
 
 template <uint32_t BS>
 __device__ __forceinline__ void clear_bins(uint32_t (*cnt)[64], uint32_t (*bx)[64][6]) {
-  for (uint32_t k = threadIdx.x; k < 3 * 64; k += BS) {
+  for (uint32_t k = group_tid<BS>(); k < 3 * 64; k += BS) {
     (&cnt[0][0])[k] = 0;
     for (int j = 0; j < 6; j++) (&bx[0][0][0])[k * 6 + j] = j < 3 ? 0xffffffffu : 0u;
+  }
+}
+
+// The cheapest split position of each axis (find_cheapest_split,
+// bvh.rs:218-261): a wave per axis, or one wave axis by axis; one lane per
+// position.  Lane i holds bin i, and the boxes and counts left of position i
+// (bins below i) and right of it are scans over the lanes (ordered min / max
+// and sums: any order gives the same values).  Every lane walking all 64 bins
+// by itself and one thread comparing the costs took 52 us a launch on the
+// levels of a 20,506-triangle build, the scans 13 us.
+struct AxisSplits {
+  float cost[3];
+  uint32_t pos[3];   // 64: none
+  uint32_t left[3];  // triangles left of pos
+};
+template <uint32_t BS>
+__device__ __forceinline__ void axis_splits(const Args& a, float parent_area, uint32_t n,
+                                            const uint32_t (*cnt)[64],
+                                            const uint32_t (*bx)[64][6], AxisSplits* out) {
+  for (uint32_t axis = group_tid<BS>() >> 6; axis < 3; axis += BS / 64) {
+    const uint32_t i = threadIdx.x & 63u;
+    const uint32_t ci = cnt[axis][i];
+    const uint64_t ne = __ballot(ci != 0);
+    const uint32_t first = __ffsll((unsigned long long)ne);  // first non-empty + 1
+    const uint32_t last = 64 - __clzll((long long)ne);        // last non-empty + 1
+    float pre[6], suf[6];
+    uint32_t below = ci;
+    for (int k = 0; k < 6; k++)
+      pre[k] = suf[k] = ci ? okey_dec(bx[axis][i][k]) : k < 3 ? INFINITY : -INFINITY;
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+      const uint32_t cu = __shfl_up(below, d);
+      if (i >= d) below += cu;
+      for (int k = 0; k < 6; k++) {
+        const float up = __shfl_up(pre[k], d), dn = __shfl_down(suf[k], d);
+        if (i >= d) pre[k] = k < 3 ? tmin_f(pre[k], up) : tmax_f(pre[k], up);
+        if (i + d < 64) suf[k] = k < 3 ? tmin_f(suf[k], dn) : tmax_f(suf[k], dn);
+      }
+    }
+    float lb[6];
+    for (int k = 0; k < 6; k++) lb[k] = __shfl_up(pre[k], 1);
+    below -= ci;
+    float cst = 0.0f;
+    bool in = __popcll(ne) > 1 && i >= first && i < last;
+    if (in) cst = tree_sah(a, parent_area, lb, below) + tree_sah(a, parent_area, suf, n - below);
+    // the reference scans the positions upward and replaces its choice only
+    // by a strictly smaller cost, so that a NaN is chosen at the first
+    // position only, and then for good
+    uint32_t pos = 64;
+    if (in && (cst == cst || i == first)) pos = i;
+    const bool nan_first = __any(in && i == first && cst != cst);
+    for (uint32_t d = 32; d > 0; d >>= 1) {
+      const float cd = __shfl_xor(cst, d);
+      const uint32_t pd = __shfl_xor(pos, d);
+      if (pd < 64 && (pos == 64 || cd < cst || (cd == cst && pd < pos))) {
+        cst = cd;
+        pos = pd;
+      }
+    }
+    if (nan_first) {
+      pos = first;
+      cst = NAN;
+    }
+    if (i == 0) {
+      out->pos[axis] = pos;
+      out->cost[axis] = cst;
+    }
+    if (i == pos) out->left[axis] = below;
+  }
+}
+
+// The choice between the axes: the reference's scan order X, Y, Z, replaced
+// only by a strictly smaller cost (bvh.rs:265-322).  -1: no axis splits.
+__device__ __forceinline__ int choose_axis(const AxisSplits& s, float* best) {
+  int axis = -1;
+  for (int k = 0; k < 3; k++) {
+    if (s.pos[k] >= 64) continue;
+    if (axis < 0 || s.cost[k] < *best) {
+      *best = s.cost[k];
+      axis = k;
+    }
+  }
+  return axis;
+}
+
+// Axes whose centroid bins fall back to sorted bins (bvh.rs:159-169): some
+// bin above n / 8 with n > bins.  One wave.
+__device__ __forceinline__ uint32_t fallback_axes(const Args& a, uint32_t n,
+                                                  const uint32_t (*cnt)[64]) {
+  uint32_t fb = 0;
+  for (uint32_t axis = 0; axis < 3; axis++) {
+    const uint64_t over = __ballot(cnt[axis][threadIdx.x & 63u] > n / 8);
+    if (over && n > a.nbins) fb |= 1u << axis;
+  }
+  return fb;
+}
+
+// bin_triangles_uniform (bvh.rs:176-201): chunks of ceil(n/bins) of the
+// stably sorted references of one axis.
+template <uint32_t BS>
+__device__ __forceinline__ void bin_sorted(const Args& a, const uint32_t* srt, uint32_t n,
+                                           uint32_t* cnt, uint32_t (*bx)[6]) {
+  const uint32_t tpb = (n + a.nbins - 1) / a.nbins;
+  for (uint32_t s = group_tid<BS>(); s < n; s += BS) {
+    const uint32_t r = srt[s];
+    const float4 A = a.A[r], B = a.B[r];
+    const uint32_t b = s / tpb;
+    const uint32_t kmn[3] = {okey(A.x), okey(A.y), okey(A.z)};
+    const uint32_t kmx[3] = {okey(B.x), okey(B.y), okey(B.z)};
+    atomicAdd(&cnt[b], 1u);
+    grow_bin(bx[b], kmn, kmx);
   }
 }
 
@@ -342,11 +482,8 @@ __global__ __launch_bounds__(kBlock) void k_bin_chunks(Args a) {
 // mode 1: pending nodes only; sorted (uniform) bins from k_sort's output.
 // ---------------------------------------------------------------------------
 
-// BS threads per node: 512, or 64 on levels whose nodes all have at most
-// kNarrow triangles (8 times as many nodes in flight per CU; the decision's
-// serial scans dominate there).
-template <uint32_t BS>
-__global__ __launch_bounds__(BS) void k_decide(Args a) {
+__global__ __launch_bounds__(kBlock) void k_decide(Args a) {
+  constexpr uint32_t BS = kBlock;
   const uint32_t id = a.list[blockIdx.x];
   INode* nd = &a.nodes[id];
   const uint32_t flags = nd->flags;
@@ -356,9 +493,7 @@ __global__ __launch_bounds__(BS) void k_decide(Args a) {
   const uint32_t umask = a.mode == 1 ? nd->uniform_mask : 0u;
   __shared__ uint32_t cnt[3][64];
   __shared__ uint32_t bx[3][64][6];
-  __shared__ float axis_cost[3];     // the cheapest position of each axis (64: none),
-  __shared__ uint32_t axis_pos[3];   // its cost and the triangles left of it
-  __shared__ uint32_t axis_left[3];
+  __shared__ AxisSplits splits;
   __shared__ bool deferred;
   __shared__ int s_axis;
   const uint32_t tid = threadIdx.x;
@@ -410,119 +545,26 @@ __global__ __launch_bounds__(BS) void k_decide(Args a) {
     bin_centroids<BS>(a, refs, n, cmn, csz, umask, cnt, bx);
   }
   if (umask) {
-    // bin_triangles_uniform (bvh.rs:176-201): chunks of ceil(n/bins) of the
-    // stably sorted references.
-    const uint32_t tpb = (n + a.nbins - 1) / a.nbins;
-    for (uint32_t axis = 0; axis < 3; axis++) {
-      if (!((umask >> axis) & 1u)) continue;
-      const uint32_t* srt = a.sorted[axis] + begin;
-      for (uint32_t s = tid; s < n; s += BS) {
-        uint32_t r = srt[s];
-        float4 A = a.A[r], B = a.B[r];
-        uint32_t b = s / tpb;
-        atomicAdd(&cnt[axis][b], 1u);
-        atomicMin(&bx[axis][b][0], okey(A.x));
-        atomicMin(&bx[axis][b][1], okey(A.y));
-        atomicMin(&bx[axis][b][2], okey(A.z));
-        atomicMax(&bx[axis][b][3], okey(B.x));
-        atomicMax(&bx[axis][b][4], okey(B.y));
-        atomicMax(&bx[axis][b][5], okey(B.z));
-      }
-    }
+    for (uint32_t axis = 0; axis < 3; axis++)
+      if ((umask >> axis) & 1u)
+        bin_sorted<BS>(a, a.sorted[axis] + begin, n, cnt[axis], bx[axis]);
   }
   __syncthreads();
   if (a.mode == 0 && tid < 64) {
-    // fallback test (bvh.rs:159-169): some bin above n/8 with n > bins
-    uint32_t lane = tid;
-    uint32_t fb = 0;
-    for (uint32_t axis = 0; axis < 3; axis++) {
-      uint32_t c = cnt[axis][lane];
-      uint64_t over = __ballot(c > n / 8);
-      if (over && n > a.nbins) fb |= 1u << axis;
+    const uint32_t fb = fallback_axes(a, n, cnt);
+    if (fb && tid == 0) {
+      nd->uniform_mask = fb;
+      nd->flags = flags | kPending;
     }
-    if (fb) {
-      if (lane == 0) {
-        nd->uniform_mask = fb;
-        nd->flags = flags | kPending;
-      }
-    }
-    if (lane == 0) deferred = fb != 0;
+    if (tid == 0) deferred = fb != 0;
   }
   __syncthreads();
   if (a.mode == 0 && deferred) return;
-  // split costs (find_cheapest_split, bvh.rs:218-261): a wave per axis (or
-  // one wave axis by axis), one lane per position.  Lane i holds bin i, and
-  // the boxes and counts left of position i (bins below i) and right of it
-  // are scans over the lanes (ordered min / max and sums: any order gives the
-  // same values).  Every lane walking all 64 bins by itself and one thread
-  // comparing the costs took 52 us a launch on the levels of a 20,506-triangle
-  // build, the scans 13 us.
-  const float parent_area = area6(nd->box);
-  for (uint32_t axis = tid >> 6; axis < 3; axis += BS / 64) {
-    const uint32_t i = tid & 63u;
-    const uint32_t ci = cnt[axis][i];
-    const uint64_t ne = __ballot(ci != 0);
-    const uint32_t first = __ffsll((unsigned long long)ne);  // first non-empty + 1
-    const uint32_t last = 64 - __clzll((long long)ne);        // last non-empty + 1
-    float pre[6], suf[6];
-    uint32_t below = ci;
-    for (int k = 0; k < 6; k++)
-      pre[k] = suf[k] = ci ? okey_dec(bx[axis][i][k]) : k < 3 ? INFINITY : -INFINITY;
-    for (uint32_t d = 1; d < 64; d <<= 1) {
-      const uint32_t cu = __shfl_up(below, d);
-      if (i >= d) below += cu;
-      for (int k = 0; k < 6; k++) {
-        const float up = __shfl_up(pre[k], d), dn = __shfl_down(suf[k], d);
-        if (i >= d) pre[k] = k < 3 ? tmin_f(pre[k], up) : tmax_f(pre[k], up);
-        if (i + d < 64) suf[k] = k < 3 ? tmin_f(suf[k], dn) : tmax_f(suf[k], dn);
-      }
-    }
-    float lb[6];
-    for (int k = 0; k < 6; k++) lb[k] = __shfl_up(pre[k], 1);
-    below -= ci;
-    float cst = 0.0f;
-    bool in = __popcll(ne) > 1 && i >= first && i < last;
-    if (in) cst = tree_sah(a, parent_area, lb, below) + tree_sah(a, parent_area, suf, n - below);
-    // the reference scans the positions upward and replaces its choice only
-    // by a strictly smaller cost, so that a NaN is chosen at the first
-    // position only, and then for good
-    uint32_t pos = 64;
-    if (in && (cst == cst || i == first)) pos = i;
-    const bool nan_first = __any(in && i == first && cst != cst);
-    for (uint32_t d = 32; d > 0; d >>= 1) {
-      const float cd = __shfl_xor(cst, d);
-      const uint32_t pd = __shfl_xor(pos, d);
-      if (pd < 64 && (pos == 64 || cd < cst || (cd == cst && pd < pos))) {
-        cst = cd;
-        pos = pd;
-      }
-    }
-    if (nan_first) {
-      pos = first;
-      cst = NAN;
-    }
-    if (i == 0) {
-      axis_pos[axis] = pos;
-      axis_cost[axis] = cst;
-    }
-    if (i == pos) axis_left[axis] = below;
-  }
+  axis_splits<BS>(a, area6(nd->box), n, cnt, bx, &splits);
   __syncthreads();
   if (tid == 0) {
-    // the reference's scan order: axes X, Y, Z; replace only on a strictly
-    // smaller cost
-    int best_axis = -1;
-    uint32_t best_i = 0, best_left = 0;
     float best = 0.0f;
-    for (uint32_t axis = 0; axis < 3; axis++) {
-      if (axis_pos[axis] >= 64) continue;
-      if (best_axis < 0 || axis_cost[axis] < best) {
-        best = axis_cost[axis];
-        best_axis = (int)axis;
-        best_i = axis_pos[axis];
-        best_left = axis_left[axis];
-      }
-    }
+    const int best_axis = choose_axis(splits, &best);
     uint32_t f = flags & ~kPending;
     s_axis = -1;
     if (best_axis < 0) {
@@ -532,8 +574,8 @@ __global__ __launch_bounds__(BS) void k_decide(Args a) {
       f |= kLeaf;  // bvh.rs:311-314
     } else {
       nd->axis = (uint32_t)best_axis;
-      nd->split_bin = best_i;
-      nd->left_count = best_left;
+      nd->split_bin = splits.pos[best_axis];
+      nd->left_count = splits.left[best_axis];
       if (a.mode == 0) nd->uniform_mask = 0;
       f |= kSplit;
       s_axis = best_axis;
@@ -579,25 +621,31 @@ __device__ __forceinline__ void wg_stable_pass(uint32_t n, LoadFn load, DigitFn 
                                                const uint32_t* start = nullptr) {
   constexpr uint32_t R = 1u << BITS;
   constexpr uint32_t W = BS / 64;
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t tid = group_tid<BS>(), lane = tid & 63, wave = tid >> 6;
   if (start) {
     for (uint32_t k = tid; k < R; k += BS) hist[k] = start[k];
   } else {
     for (uint32_t k = tid; k < R; k += BS) hist[k] = 0;
-    __syncthreads();
+    group_sync<BS>();
     for (uint32_t e = tid; e < n; e += BS) atomicAdd(&hist[digit_of(load(e))], 1u);
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t s = 0;
-      for (uint32_t k = 0; k < R; k++) {
-        uint32_t c = hist[k];
-        hist[k] = s;
-        s += c;
+    group_sync<BS>();
+    if (tid < 64) {  // exclusive prefix sums, R / 64 digits a lane
+      constexpr uint32_t E = R / 64;
+      uint32_t c[E], own = 0;
+      for (uint32_t k = 0; k < E; k++) {
+        c[k] = own;
+        own += hist[tid * E + k];
       }
+      uint32_t inc = own;
+      for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(inc, d);
+        if (lane >= d) inc += y;
+      }
+      for (uint32_t k = 0; k < E; k++) hist[tid * E + k] = c[k] + inc - own;
     }
   }
   for (uint32_t k = tid; k < W * R; k += BS) wcount[k] = 0;
-  __syncthreads();
+  group_sync<BS>();
   const uint64_t lt = (1ull << lane) - 1ull;
   for (uint32_t t0 = 0; t0 < n; t0 += BS) {
     uint32_t e = t0 + tid;
@@ -611,13 +659,13 @@ __device__ __forceinline__ void wg_stable_pass(uint32_t n, LoadFn load, DigitFn 
     }
     uint32_t rank = __popcll(match & lt);
     if (valid && rank == 0) wcount[wave * R + d] = __popcll(match);
-    __syncthreads();
+    group_sync<BS>();
     if (valid) {
       uint32_t prior = 0;
       for (uint32_t w = 0; w < wave; w++) prior += wcount[w * R + d];
       dst[hist[d] + prior + rank] = v;
     }
-    __syncthreads();
+    group_sync<BS>();
     for (uint32_t k = tid; k < R; k += BS) {
       uint32_t s = 0;
       for (uint32_t w = 0; w < W; w++) {
@@ -626,7 +674,7 @@ __device__ __forceinline__ void wg_stable_pass(uint32_t n, LoadFn load, DigitFn 
       }
       hist[k] += s;
     }
-    __syncthreads();
+    group_sync<BS>();
   }
 }
 
@@ -665,7 +713,7 @@ __device__ __forceinline__ void side_bounds(const Args& a, const uint32_t* order
   uint32_t lk[2][12];
   for (int s = 0; s < 2; s++)
     for (int k = 0; k < 12; k++) lk[s][k] = (k % 6) < 3 ? 0xffffffffu : 0u;
-  for (uint32_t e = lo + threadIdx.x; e < hi; e += BS) {
+  for (uint32_t e = lo + group_tid<BS>(); e < hi; e += BS) {
     uint32_t r = order[e];
     int side = uniform ? (e < L ? 0 : 1) : (bin_of(r) < split ? 0 : 1);
     float4 A = a.A[r], B = a.B[r];
@@ -692,14 +740,14 @@ __device__ __forceinline__ void side_bounds(const Args& a, const uint32_t* order
         uint32_t o = __shfl_xor(v, off);
         v = (k % 6) < 3 ? min(v, o) : max(v, o);
       }
-      if ((threadIdx.x & 63) == 0) {
+      if ((threadIdx.x & 63u) == 0) {
         if ((k % 6) < 3)
           atomicMin(&cb[s][k], v);
         else
           atomicMax(&cb[s][k], v);
       }
     }
-  __syncthreads();
+  group_sync<BS>();
 }
 
 // One chunk of a wide node that splits: its references go to the positions
@@ -739,10 +787,47 @@ __global__ __launch_bounds__(kBlock) void k_part_chunks(Args a) {
   if (tid < 24) a.side[(size_t)c * 24 + tid] = (&cb[0][0])[tid];
 }
 
+// The two children of a node split at left_count, with their bounds from cb
+// (per side: outer min.xyz max.xyz, barycenter min.xyz max.xyz as okeys).
+// Returns the first child's id.  One thread.
+__device__ __forceinline__ uint32_t make_children(const Args& a, INode* nd, uint32_t id,
+                                                  const uint32_t (*cb)[12]) {
+  const uint32_t c = atomicAdd(&a.ctx->node_count, 2u);
+  const uint32_t L = nd->left_count, n = nd->count;
+  const uint32_t par = (nd->flags & kParity) ? 1u : 0u;
+  INode ch[2];
+  for (int s = 0; s < 2; s++) {
+    for (int k = 0; k < 6; k++) {
+      ch[s].box[k] = okey_dec(cb[s][k]);
+      ch[s].cbox[k] = okey_dec(cb[s][6 + k]);
+    }
+    ch[s].begin = nd->begin + (s == 0 ? 0 : L);
+    ch[s].count = s == 0 ? L : n - L;
+    ch[s].parent = (int32_t)id;
+    ch[s].child[0] = ch[s].child[1] = -1;
+    ch[s].flags = (par ^ 1u) ? kParity : 0u;
+    ch[s].leaves = 0;
+    ch[s].sar = 0.0f;
+    ch[s].depth = 0;
+    ch[s].axis = ch[s].split_bin = ch[s].left_count = ch[s].uniform_mask = 0;
+    ch[s].chunk_base = ch[s].nchunks = 0;
+  }
+  // smaller area first (bvh.rs:337-345)
+  const bool swap = area6(ch[0].box) > area6(ch[1].box);
+  ch[swap ? 0 : 1].flags |= kIsC1;
+  for (int s = 0; s < 2; s++) {
+    if (ch[s].count == 1) ch[s].flags |= kLeaf;
+    a.nodes[c + s] = ch[s];
+  }
+  nd->child[0] = (int32_t)(swap ? c + 1 : c);
+  nd->child[1] = (int32_t)(swap ? c : c + 1);
+  return c;
+}
+
 // Reorders the segment as split() collects the children (bins in order,
 // references in push order) and creates the children.
-template <uint32_t BS>
-__global__ __launch_bounds__(BS) void k_partition(Args a) {
+__global__ __launch_bounds__(kBlock) void k_partition(Args a) {
+  constexpr uint32_t BS = kBlock;
   const uint32_t id = a.list[blockIdx.x];
   INode* nd = &a.nodes[id];
   const uint32_t flags = nd->flags;
@@ -798,45 +883,164 @@ __global__ __launch_bounds__(BS) void k_partition(Args a) {
     side_bounds<BS>(a, uniform ? a.sorted[axis] + begin : src, 0, n, uniform, L, split, bin_of, cb);
   }
   if (tid == 0) {
-    uint32_t c = atomicAdd(&a.ctx->node_count, 2u);
-    INode ch[2];
-    for (int s = 0; s < 2; s++) {
-      for (int k = 0; k < 6; k++) {
-        ch[s].box[k] = okey_dec(cb[s][k]);
-        ch[s].cbox[k] = okey_dec(cb[s][6 + k]);
-      }
-      ch[s].begin = begin + (s == 0 ? 0 : L);
-      ch[s].count = s == 0 ? L : n - L;
-      ch[s].parent = (int32_t)id;
-      ch[s].child[0] = ch[s].child[1] = -1;
-      ch[s].flags = (par ^ 1u) ? kParity : 0u;
-      ch[s].leaves = 0;
-      ch[s].sar = 0.0f;
-      ch[s].depth = 0;
-      ch[s].axis = ch[s].split_bin = ch[s].left_count = ch[s].uniform_mask = 0;
-      ch[s].chunk_base = ch[s].nchunks = 0;
-    }
-    // smaller area first (bvh.rs:337-345)
-    bool swap = area6(ch[0].box) > area6(ch[1].box);
-    uint32_t first = swap ? c + 1 : c, second = swap ? c : c + 1;
-    ch[swap ? 0 : 1].flags |= kIsC1;
-    for (int s = 0; s < 2; s++) {
-      uint32_t cid = c + s;
-      if (ch[s].count == 1) ch[s].flags |= kLeaf;
-      a.nodes[cid] = ch[s];
-      if (ch[s].count > a.small_max) {
-        uint32_t slot = atomicAdd(&a.ctx->next_large, 1u);
-        a.next_list[slot] = cid;
-        if (ch[s].count > kWide) atomicAdd(&a.ctx->next_wide, 1u);
-        atomicMax(&a.ctx->next_max, ch[s].count);
-      } else if (ch[s].count >= 2) {
-        uint32_t slot = atomicAdd(&a.ctx->small_count, 1u);
-        a.small_list[slot] = cid;
+    const uint32_t c = make_children(a, nd, id, cb);
+    for (uint32_t s = 0; s < 2; s++) {
+      const uint32_t count = s == 0 ? L : n - L;
+      if (count > kSub) {
+        a.next_list[atomicAdd(&a.ctx->next_large, 1u)] = c + s;
+        if (count > kWide) atomicAdd(&a.ctx->next_wide, 1u);
+      } else if (count > a.small_max) {
+        a.sub_list[atomicAdd(&a.ctx->sub_count, 1u)] = c + s;
+      } else if (count >= 2) {
+        a.small_list[atomicAdd(&a.ctx->small_count, 1u)] = c + s;
       }
     }
-    nd->child[0] = (int32_t)first;
-    nd->child[1] = (int32_t)second;
   }
+}
+
+// ---------------------------------------------------------------------------
+// k_subtree: one workgroup of kSubWaves waves splits a node of at most kSub
+// triangles down to nodes of at most 32, level by level within the workgroup:
+// the whole workgroup per node of more than kSubWide triangles, then a wave
+// per node for the rest; a node's bins, the sorts of axes that fall back to
+// sorted bins, its split and its partition follow each other.  Bound by the
+// latency of the passes over a node's references; a launch per pass and level
+// for the whole tree, with 512-thread workgroups for nodes of a few hundred
+// triangles, took 4.5 ms for 1.33 M triangles, this 1.6 ms.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kSubWaves = 8;
+constexpr uint32_t kSubWide = 256;
+constexpr uint32_t kSubList = kSub / 9 + 1;  // nodes of more than 8 triangles (16 bins)
+
+struct SubWork {
+  uint32_t cnt[3][64];
+  uint32_t bx[3][64][6];
+  uint32_t hist[256];
+  uint32_t cb[2][12];
+  AxisSplits splits;
+};
+
+// Splits node id with BS threads; children of more than small_max triangles
+// join `next`.
+template <uint32_t BS>
+__device__ __forceinline__ void split_node(const Args& a, uint32_t id, SubWork& w,
+                                           uint32_t* wcount, uint32_t* next, uint32_t* nnext) {
+  const uint32_t tid = group_tid<BS>();
+  INode* nd = &a.nodes[id];
+  const uint32_t n = __builtin_amdgcn_readfirstlane(nd->count);
+  const uint32_t begin = __builtin_amdgcn_readfirstlane(nd->begin);
+  const uint32_t flags = __builtin_amdgcn_readfirstlane(nd->flags);
+  const uint32_t par = (flags & kParity) ? 1u : 0u;
+  const uint32_t* src = a.buf[par] + begin;
+  uint32_t* dst = a.buf[par ^ 1u] + begin;
+  float cmn[3], csz[3];
+  for (int j = 0; j < 3; j++) {
+    cmn[j] = nd->cbox[j];
+    csz[j] = nd->cbox[3 + j] - cmn[j];
+  }
+  const float area = area6(nd->box);
+  clear_bins<BS>(w.cnt, w.bx);
+  if (tid < 24) (&w.cb[0][0])[tid] = ((tid % 12) % 6) < 3 ? 0xffffffffu : 0u;
+  group_sync<BS>();
+  bin_centroids<BS>(a, src, n, cmn, csz, 0u, w.cnt, w.bx);
+  group_sync<BS>();
+  const uint32_t umask = fallback_axes(a, n, w.cnt);
+  for (uint32_t axis = 0; axis < 3; axis++) {
+    if (!((umask >> axis) & 1u)) continue;
+    uint32_t* X = a.tmp[axis] + begin;
+    uint32_t* Y = a.sorted[axis] + begin;
+    for (uint32_t pass = 0; pass < 4; pass++) {
+      const uint32_t* from = pass == 0 ? src : (pass & 1) ? X : Y;
+      uint32_t* to = (pass & 1) ? Y : X;
+      auto load = [&](uint32_t e) { return from[e]; };
+      auto digit = [&](uint32_t r) {
+        return (sort_key(centroid(a, r, axis)) >> (8 * pass)) & 255u;
+      };
+      wg_stable_pass<8, BS>(n, load, digit, to, w.hist, wcount);
+      group_sync<BS>();
+    }
+    for (uint32_t k = tid; k < 64; k += BS) {
+      w.cnt[axis][k] = 0;
+      for (int j = 0; j < 6; j++) w.bx[axis][k][j] = j < 3 ? 0xffffffffu : 0u;
+    }
+    group_sync<BS>();
+    bin_sorted<BS>(a, Y, n, w.cnt[axis], w.bx[axis]);
+    group_sync<BS>();
+  }
+  axis_splits<BS>(a, area, n, w.cnt, w.bx, &w.splits);
+  group_sync<BS>();
+  float best = 0.0f;
+  const int axis = choose_axis(w.splits, &best);
+  if (axis < 0 || (float)n * 120.0f < best) {
+    if (tid == 0) {
+      if (axis < 0) atomicOr(&a.ctx->error, 2u);  // assert!(!is_first), bvh.rs:303
+      nd->flags = flags | kLeaf;                  // bvh.rs:311-314
+    }
+    return;
+  }
+  const uint32_t L = __builtin_amdgcn_readfirstlane(w.splits.left[axis]);
+  const float mn = nd->cbox[axis], size = nd->cbox[3 + axis] - mn;
+  auto bin_of = [&](uint32_t r) {
+    return centroid_bin(centroid(a, r, (uint32_t)axis), mn, size, a.nbins);
+  };
+  if ((umask >> axis) & 1u) {
+    const uint32_t* srt = a.sorted[axis] + begin;
+    for (uint32_t e = tid; e < n; e += BS) dst[e] = srt[e];
+  } else {
+    auto load = [&](uint32_t e) { return src[e]; };
+    wg_stable_pass<6, BS>(n, load, bin_of, dst, w.hist, wcount);
+  }
+  group_sync<BS>();
+  side_bounds<BS>(a, dst, 0, n, true, L, 0u, bin_of, w.cb);
+  if (tid == 0) {
+    nd->left_count = L;
+    nd->flags = flags | kSplit;
+    const uint32_t c = make_children(a, nd, id, w.cb);
+    for (uint32_t s = 0; s < 2; s++) {
+      const uint32_t cn = s == 0 ? L : n - L;
+      if (cn > a.small_max)
+        next[atomicAdd(nnext, 1u)] = c + s;
+      else if (cn >= 2)
+        a.small_list[atomicAdd(&a.ctx->small_count, 1u)] = c + s;
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * kSubWaves) void k_subtree(Args a) {
+  __shared__ SubWork work[kSubWaves];
+  __shared__ uint32_t wcount[kSubWaves * 256];
+  __shared__ uint32_t list[2][kSubList];
+  __shared__ uint32_t count[2];
+  if (blockIdx.x >= a.ctx->sub_count || (a.ctx->error & 1u)) return;
+  const uint32_t wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) {
+    list[0][0] = a.sub_list[blockIdx.x];
+    count[0] = 1;
+    count[1] = 0;
+  }
+  __syncthreads();
+  uint32_t levels = 0;
+  for (uint32_t cur = 0;; cur ^= 1u, levels++) {
+    const uint32_t nodes = count[cur];
+    if (nodes == 0) break;
+    uint32_t* next = list[cur ^ 1u];
+    for (uint32_t k = 0; k < nodes; k++) {
+      const uint32_t id = __builtin_amdgcn_readfirstlane(list[cur][k]);
+      if (__builtin_amdgcn_readfirstlane(a.nodes[id].count) <= kSubWide) continue;
+      split_node<64 * kSubWaves>(a, id, work[0], wcount, next, &count[cur ^ 1u]);
+      __syncthreads();
+    }
+    for (uint32_t k = wave; k < nodes; k += kSubWaves) {
+      const uint32_t id = __builtin_amdgcn_readfirstlane(list[cur][k]);
+      if (__builtin_amdgcn_readfirstlane(a.nodes[id].count) > kSubWide) continue;
+      split_node<64>(a, id, work[wave], wcount + wave * 256, next, &count[cur ^ 1u]);
+      group_sync<64>();
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) count[cur] = 0;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) atomicMax(&a.ctx->sub_levels, levels);
 }
 
 // ---------------------------------------------------------------------------
@@ -867,6 +1071,7 @@ __device__ __forceinline__ float tree_sah_small(const float (*tp)[33], float par
 __global__ __launch_bounds__(256) void k_small(Args a) {
   const uint32_t lane = threadIdx.x & 63, half = lane >> 5;
   __shared__ float tp[2][33];
+  if (blockIdx.x * 8 >= a.ctx->small_count || a.ctx->error) return;
   if (threadIdx.x < 66) {
     const uint32_t k = threadIdx.x % 33;
     tp[threadIdx.x / 33][k] = k <= a.ntris ? (threadIdx.x < 33 ? a.tpm[k] : a.tpm1[k]) : 0.0f;
@@ -1122,7 +1327,6 @@ __global__ void k_level_reset(Ctx* ctx) {
   if (threadIdx.x == 0) {
     ctx->next_large = 0;
     ctx->next_wide = 0;
-    ctx->next_max = 0;
   }
 }
 
@@ -1219,13 +1423,13 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   // nodes + triangles of small subtrees) - 1 <= 2 N - 1.
   const size_t ninodes_cap = 2 * N + 2;
   Ctx* ctx;
-  const size_t list_cap = N / (a.small_max + 1) + 2;
-  uint32_t *listA, *listB, *small, *dcount, *dlist;
+  const size_t list_cap = N / (kSub + 1) + 2, sub_cap = N / (a.small_max + 1) + 2;
+  uint32_t *listA, *listB, *sub, *small, *dcount, *dlist;
   // chunks of the wide nodes of one level: their triangles are disjoint, so
   // at most N / kChunk + (number of wide nodes) chunks
   const size_t max_chunks = N / kChunk + N / kWide + 2;
   // depths: at most one level per triangle
-  const size_t dcount_cap = N + 64;
+  const size_t dcount_cap = 2 * N + 64;
   float *d_tpm, *d_tpm1;
   for (int pass = 0; pass < 2; pass++) {
     arena_bytes = 0;
@@ -1241,6 +1445,7 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
     take(&ctx, 1);
     take(&listA, list_cap);
     take(&listB, list_cap);
+    take(&sub, sub_cap);
     take(&small, N / 2 + 2);
     take(&a.chunk_node, max_chunks);
     take(&a.part, max_chunks * kBinWords);
@@ -1256,6 +1461,7 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   a.B = B;
   a.C = C;
   a.ctx = ctx;
+  a.sub_list = sub;
   a.small_list = small;
   // TreeSAH power tables with the C library (same values as the CPU build)
   // (two powf and a log2f per triangle count: 33 ms for 1.33 M counts on one
@@ -1307,9 +1513,12 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   }
   uint32_t zero = 0, one = 1;
   uint32_t nlist = 0;
-  if (ntris > a.small_max) {
+  if (ntris > kSub) {
     BVH_CHECK(hipMemcpyAsync(listA, &zero, 4, hipMemcpyHostToDevice, s));
     nlist = 1;
+  } else if (ntris > a.small_max) {
+    BVH_CHECK(hipMemcpyAsync(sub, &zero, 4, hipMemcpyHostToDevice, s));
+    BVH_CHECK(hipMemcpyAsync(&ctx->sub_count, &one, 4, hipMemcpyHostToDevice, s));
   } else if (ntris >= 2) {
     BVH_CHECK(hipMemcpyAsync(small, &zero, 4, hipMemcpyHostToDevice, s));
     BVH_CHECK(hipMemcpyAsync(&ctx->small_count, &one, 4, hipMemcpyHostToDevice, s));
@@ -1317,11 +1526,10 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   uint32_t* cur = listA;
   uint32_t* nxt = listB;
   bool wide = ntris > kWide;
-  uint32_t level_max = ntris;
+  uint32_t nsub = ntris > a.small_max ? 1u : 0u;  // nodes for k_subtree so far
   uint32_t levels = 0;  // iterations of the level phase
   while (nlist > 0) {
     levels++;
-    const bool narrow = level_max <= kNarrow;
     a.list = cur;
     a.nlist = nlist;
     a.next_list = nxt;
@@ -1332,18 +1540,12 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
       hipLaunchKernelGGL(k_bin_chunks, dim3((uint32_t)max_chunks), dim3(kBlock), 0, s, a);
       BVH_CHECK(hipGetLastError());
     }
-    auto decide = [&]() {
-      if (narrow)
-        hipLaunchKernelGGL(k_decide<64>, dim3(nlist), dim3(64), 0, s, a);
-      else
-        hipLaunchKernelGGL(k_decide<kBlock>, dim3(nlist), dim3(kBlock), 0, s, a);
-    };
-    decide();
+    hipLaunchKernelGGL(k_decide, dim3(nlist), dim3(kBlock), 0, s, a);
     BVH_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_sort, dim3(nlist * 3), dim3(kBlock), 0, s, a);
     BVH_CHECK(hipGetLastError());
     a.mode = 1;
-    decide();
+    hipLaunchKernelGGL(k_decide, dim3(nlist), dim3(kBlock), 0, s, a);
     BVH_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_level_reset, dim3(1), dim3(64), 0, s, ctx);
     BVH_CHECK(hipGetLastError());
@@ -1351,8 +1553,7 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
       hipLaunchKernelGGL(k_part_chunks, dim3((uint32_t)max_chunks), dim3(kBlock), 0, s, a);
       BVH_CHECK(hipGetLastError());
     }
-    // (64-thread blocks measured slower here: the stable pass's tiles)
-    hipLaunchKernelGGL(k_partition<kBlock>, dim3(nlist), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL(k_partition, dim3(nlist), dim3(kBlock), 0, s, a);
     BVH_CHECK(hipGetLastError());
     uint32_t hctl[7];
     BVH_CHECK(hipMemcpyAsync(hctl, ctx, 28, hipMemcpyDeviceToHost, s));
@@ -1360,18 +1561,20 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
     if (hctl[3]) break;
     nlist = hctl[1];
     wide = hctl[4] > 0;
-    level_max = hctl[6];
+    nsub = hctl[6];
     uint32_t* t = cur;
     cur = nxt;
     nxt = t;
   }
-  Ctx hc;
-  BVH_CHECK(hipMemcpyAsync(&hc, ctx, sizeof(Ctx), hipMemcpyDeviceToHost, s));
-  BVH_CHECK(hipStreamSynchronize(s));
-  if (hc.error == 0 && hc.small_count > 0) {
-    hipLaunchKernelGGL(k_small, dim3((hc.small_count + 7) / 8), dim3(256), 0, s, a);
+  // (both exit at once after an error, and k_small beyond the nodes listed,
+  // so neither waits for the host to read the counters)
+  if (nsub) {
+    hipLaunchKernelGGL(k_subtree, dim3(nsub), dim3(64 * kSubWaves), 0, s, a);
     BVH_CHECK(hipGetLastError());
   }
+  hipLaunchKernelGGL(k_small, dim3((ntris / 2 + 7) / 8 + 1), dim3(256), 0, s, a);
+  BVH_CHECK(hipGetLastError());
+  Ctx hc;
   BVH_CHECK(hipMemcpyAsync(&hc, ctx, sizeof(Ctx), hipMemcpyDeviceToHost, s));
   BVH_CHECK(hipStreamSynchronize(s));
   uint32_t ninodes = hc.node_count;
@@ -1394,9 +1597,9 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
     return hipSuccess;
   }
   uint32_t blocks = (ninodes + 255) / 256;
-  // depths: the level phase's nodes lie at most `levels` deep and a small
-  // subtree of at most 32 triangles adds at most 31 levels
-  const uint32_t dcap = levels + 34;
+  // depths: the level phase's nodes lie at most `levels` deep, k_subtree adds
+  // at most sub_levels and a small subtree of at most 32 triangles 31
+  const uint32_t dcap = levels + hc.sub_levels + 34;
   BVH_CHECK(hipMemsetAsync(dcount, 0, (size_t)dcap * 4, s));
   hipLaunchKernelGGL(k_depth, dim3(blocks), dim3(256), 0, s, a, ninodes, dcount, dcap);
   BVH_CHECK(hipGetLastError());
