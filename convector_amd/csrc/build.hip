@@ -11,25 +11,26 @@
 // n/8 of n > bins in one bin take the sorted bins, in chunks of
 // ceil(n/bins)); below, "32" stands for bins/2 and "64" for bins.
 //
-// Level-synchronous:
-//   k_decide (one workgroup per node of more than 32 triangles) bins the
-//     three axes in LDS and picks the split;
+// Level-synchronous down to nodes of kSub triangles:
+//   k_level_plan resets the next level's counters and lists the chunks of the
+//     wide nodes;
+//   k_decide (one workgroup per node) bins the three axes in LDS and picks
+//     the split;
 //   k_sort sorts the axes that fall back to sorted binning (stable LSD radix
 //     sort, one workgroup per node and axis);
 //   k_partition reorders the node's triangle references as the reference
 //     collects them (stable by bin) and creates the children.
-// A node of more than kWide triangles is split over chunks of kChunk
-// references: k_bin_chunks bins each chunk into a partial that k_decide
-// adds up (counts and ordered-integer min / max, so the bins are exact),
-// k_decide also turns the chunks' counts into each chunk's first output
-// position per bin, and k_part_chunks scatters the chunks and bounds their
-// children, so that the top levels, where one node holds most triangles,
-// use the whole GPU.
-// Nodes of at most 32 triangles are finished by k_small, one wave per node,
-// with the triangles in the lanes.  k_depth (which also lists the inner
-// nodes by depth) and k_bottom_up (one launch per depth over that depth's
-// list, deepest first) count leaves and the area ratio statistic; k_layout
-// places every node where crystallize puts it.
+// A node of more than kWide triangles is split over chunks of references:
+// k_bin_chunks bins each chunk into a partial, k_sum_chunks adds the partials
+// up (counts and ordered-integer min / max, so the bins are exact), and
+// k_part_chunks scatters the chunks and bounds their children, so that the
+// top levels, where one node holds most triangles, use the whole GPU.
+// k_subtree splits each node of at most kSub triangles down to nodes of at
+// most 32 within one workgroup, and k_small finishes those, two per wave, with
+// the triangles in the lanes.  k_depth and k_depth_lists list the inner nodes
+// by depth; k_bottom_up counts leaves and the area ratio statistic, deepest
+// depth first, and k_place puts every node where crystallize puts it, from the
+// root down.
 //
 // The TreeSAH cost uses powf/log2f; their values for every triangle count are
 // tabulated on the host with the C library so that near-ties resolve as in the
@@ -51,9 +52,10 @@ constexpr uint32_t kLeaf = 1, kParity = 2, kIsC1 = 4, kPending = 8, kSplit = 16;
 // an id that a small subtree reserved and did not use (no node)
 constexpr uint32_t kHole = 32;
 constexpr uint32_t kBlock = 512;
-constexpr uint32_t kChunk = 2048;   // references per chunk of a wide node
 constexpr uint32_t kWide = 4096;    // nodes above this many triangles are chunked
 constexpr uint32_t kSub = 1024;     // nodes of at most this many triangles go to k_subtree
+constexpr uint32_t kLevelBatch = 4;   // levels enqueued between the host's looks at the lists
+constexpr uint32_t kDepthFew = 2048;  // nodes of a depth that shares a launch with others
 constexpr uint32_t kBinWords = 3 * 64 * 7;  // counts, then outer bounds, of 3 x 64 bins
 
 struct INode {
@@ -65,18 +67,23 @@ struct INode {
   uint32_t flags;
   uint32_t leaves;
   float sar;
-  uint32_t depth;  // set by k_depth
+  uint32_t depth;
   uint32_t axis, split_bin, left_count, uniform_mask;
-  uint32_t chunk_base, nchunks;  // chunks of a wide node in the level's chunk list
+  // chunks of a wide node in the level's chunk list and its row of `tot`
+  uint32_t chunk_base, nchunks, slot;
+  // k_place: nodes.len() when the node is crystallised (bvh.rs:389-428) and
+  // the position of its first triangle
+  uint32_t pairs, first_tri;
 };
 
 struct Ctx {
   uint32_t node_count;
-  uint32_t next_large;
+  uint32_t large[2];      // nodes in the lists of the even and the odd levels
   uint32_t small_count;
   uint32_t error;
   uint32_t next_wide;     // wide nodes in the next level's list
-  uint32_t total_chunks;  // chunks of the current level
+  uint32_t wide_count;    // wide nodes and chunks of the current level
+  uint32_t total_chunks;
   uint32_t sub_count;     // nodes for k_subtree
   uint32_t sub_levels;    // most levels that a subtree of k_subtree took
   uint32_t max_depth;
@@ -95,7 +102,7 @@ struct Args {
   INode* nodes;
   Ctx* ctx;
   const uint32_t* list;
-  uint32_t nlist;
+  uint32_t parity;  // of the level: list holds ctx->large[parity] nodes
   uint32_t* next_list;
   uint32_t* sub_list;
   uint32_t* small_list;
@@ -105,12 +112,13 @@ struct Args {
   uint32_t ntris;
   uint32_t nbins;      // centroid bins per axis: 64 (the reference), 32 or 16
   uint32_t small_max;  // nodes of at most nbins / 2 triangles go to k_small
-  // chunked wide nodes: per chunk the node, the bins (kBinWords), the first
-  // output position per bin of the split axis (64) and the children's
-  // bounds (2 sides x 12 okeys)
+  // chunked wide nodes: the level's, per node its bins (kBinWords), and per
+  // chunk the node, the bins and the children's bounds (2 sides x 12 okeys)
+  uint32_t chunk;
+  uint32_t* wide_list;
+  uint32_t* tot;
   uint32_t* chunk_node;
   uint32_t* part;
-  uint32_t* offs;
   uint32_t* side;
 };
 
@@ -231,7 +239,7 @@ __global__ void k_root(INode* nodes, Ctx* ctx, uint32_t n) {
   r.sar = 0.0f;
   r.depth = 0;
   r.axis = r.split_bin = r.left_count = r.uniform_mask = 0;
-  r.chunk_base = r.nchunks = 0;
+  r.chunk_base = r.nchunks = r.slot = r.pairs = r.first_tri = 0;
   nodes[0] = r;
   ctx->node_count = 1;
 }
@@ -407,23 +415,25 @@ __device__ __forceinline__ void bin_sorted(const Args& a, const uint32_t* srt, u
   }
 }
 
-// Chunk list of the level's wide nodes (one thread; only levels that have
-// wide nodes run it, and those lists are short).
-// One workgroup: the list in tiles of 1024 nodes, a prefix sum of the chunk
-// counts per tile; each node's thread writes its own chunk entries.
-__global__ __launch_bounds__(1024) void k_wide_plan(Args a) {
+// Start of a level: the next level's counters back to zero and the chunk
+// list of the level's wide nodes.  One workgroup: the list in tiles of 1024
+// nodes, a prefix sum of the chunk counts per tile, and the tile's chunk
+// entries written by all threads.
+__global__ __launch_bounds__(1024) void k_level_plan(Args a) {
   __shared__ uint32_t wsum[16];
-  __shared__ uint32_t s_base;
+  __shared__ uint32_t s_base, s_wide;
+  __shared__ uint32_t t_end[1024], t_id[1024];  // the tile's wide nodes: last chunk + 1, id
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (threadIdx.x == 0) s_base = 0;
+  const uint32_t nlist = a.ctx->large[a.parity];
+  if (threadIdx.x == 0) s_base = s_wide = 0;
   __syncthreads();
-  for (uint32_t i0 = 0; i0 < a.nlist; i0 += 1024) {
+  for (uint32_t i0 = 0; i0 < nlist; i0 += 1024) {
     const uint32_t i = i0 + threadIdx.x;
     uint32_t id = 0, nc = 0;
-    if (i < a.nlist) {
+    if (i < nlist) {
       id = a.list[i];
       const uint32_t n = a.nodes[id].count;
-      nc = n > kWide ? (n + kChunk - 1) / kChunk : 0u;
+      nc = n > kWide ? (n + a.chunk - 1) / a.chunk : 0u;
     }
     uint32_t inc = nc;
     for (uint32_t off = 1; off < 64; off <<= 1) {
@@ -437,17 +447,40 @@ __global__ __launch_bounds__(1024) void k_wide_plan(Args a) {
       prior += w < wave ? wsum[w] : 0u;
       tile += wsum[w];
     }
-    const uint32_t base = s_base + prior + inc - nc;
-    if (i < a.nlist) {
-      a.nodes[id].chunk_base = base;
+    t_end[threadIdx.x] = prior + inc;
+    t_id[threadIdx.x] = id;
+    if (i < nlist) {
+      uint32_t slot = 0;
+      if (nc) {
+        slot = atomicAdd(&s_wide, 1u);
+        a.wide_list[slot] = id;
+      }
+      a.nodes[id].chunk_base = s_base + prior + inc - nc;
       a.nodes[id].nchunks = nc;
-      for (uint32_t c = 0; c < nc; c++) a.chunk_node[base + c] = id;
+      a.nodes[id].slot = slot;
+    }
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < tile; t += 1024) {
+      uint32_t lo = 0, hi = 1023;  // the first node whose chunks end above t
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (t_end[mid] > t)
+          hi = mid;
+        else
+          lo = mid + 1;
+      }
+      a.chunk_node[s_base + t] = t_id[lo];
     }
     __syncthreads();
     if (threadIdx.x == 0) s_base += tile;
     __syncthreads();
   }
-  if (threadIdx.x == 0) a.ctx->total_chunks = s_base;
+  if (threadIdx.x == 0) {
+    a.ctx->total_chunks = s_base;
+    a.ctx->wide_count = s_wide;
+    a.ctx->large[a.parity ^ 1u] = 0;
+    a.ctx->next_wide = 0;
+  }
 }
 
 // Centroid bins of one chunk of a wide node into its partial.
@@ -455,8 +488,8 @@ __global__ __launch_bounds__(kBlock) void k_bin_chunks(Args a) {
   const uint32_t c = blockIdx.x;
   if (c >= a.ctx->total_chunks) return;
   const INode* nd = &a.nodes[a.chunk_node[c]];
-  const uint32_t lo = (c - nd->chunk_base) * kChunk;
-  const uint32_t n = min(nd->count, lo + kChunk) - lo;
+  const uint32_t lo = (c - nd->chunk_base) * a.chunk;
+  const uint32_t n = min(nd->count, lo + a.chunk) - lo;
   const uint32_t* refs = a.buf[(nd->flags & kParity) ? 1 : 0] + nd->begin + lo;
   __shared__ uint32_t cnt[3][64];
   __shared__ uint32_t bx[3][64][6];
@@ -474,6 +507,39 @@ __global__ __launch_bounds__(kBlock) void k_bin_chunks(Args a) {
   for (uint32_t k = threadIdx.x; k < 3 * 64 * 6; k += kBlock) out[192 + k] = (&bx[0][0][0])[k];
 }
 
+// The bins of the wide nodes: their chunks' partials added up, 64 words of
+// one node per workgroup, every fourth chunk by each of its waves (integer
+// sums and ordered min / max: any order gives the same bins; 16 loads are
+// issued before they are combined).  One workgroup per node reading all
+// partials took 208 us on a 1.33 M-triangle node, this and the split 45.
+__global__ __launch_bounds__(256) void k_sum_chunks(Args a) {
+  if (blockIdx.x >= a.ctx->wide_count) return;
+  const INode* nd = &a.nodes[a.wide_list[blockIdx.x]];
+  __shared__ uint32_t red[4][64];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t k = blockIdx.y * 64 + lane, nch = nd->nchunks;
+  const uint32_t* q = a.part + (size_t)nd->chunk_base * kBinWords + k;
+  const int op = k < 192 ? 0 : ((k - 192) % 6) < 3 ? 1 : 2;  // sum, min, max
+  auto acc = [&](uint32_t v, uint32_t w) {
+    return op == 0 ? v + w : op == 1 ? min(v, w) : max(v, w);
+  };
+  const uint32_t none = op == 1 ? 0xffffffffu : 0u;
+  uint32_t v = none;
+  for (uint32_t c0 = wave; c0 < nch; c0 += 64) {
+    uint32_t w[16];
+#pragma unroll
+    for (uint32_t j = 0; j < 16; j++)
+      w[j] = c0 + 4 * j < nch ? q[(size_t)(c0 + 4 * j) * kBinWords] : none;
+#pragma unroll
+    for (uint32_t j = 0; j < 16; j++) v = acc(v, w[j]);
+  }
+  red[wave][lane] = v;
+  __syncthreads();
+  if (wave == 0)
+    a.tot[(size_t)nd->slot * kBinWords + k] =
+        acc(acc(red[0][lane], red[1][lane]), acc(red[2][lane], red[3][lane]));
+}
+
 // ---------------------------------------------------------------------------
 // k_decide: bins + split choice for nodes of more than 32 triangles
 // (InterimNode::split, bvh.rs:265-322).
@@ -484,6 +550,7 @@ __global__ __launch_bounds__(kBlock) void k_bin_chunks(Args a) {
 
 __global__ __launch_bounds__(kBlock) void k_decide(Args a) {
   constexpr uint32_t BS = kBlock;
+  if (blockIdx.x >= a.ctx->large[a.parity]) return;
   const uint32_t id = a.list[blockIdx.x];
   INode* nd = &a.nodes[id];
   const uint32_t flags = nd->flags;
@@ -495,9 +562,8 @@ __global__ __launch_bounds__(kBlock) void k_decide(Args a) {
   __shared__ uint32_t bx[3][64][6];
   __shared__ AxisSplits splits;
   __shared__ bool deferred;
-  __shared__ int s_axis;
   const uint32_t tid = threadIdx.x;
-  const uint32_t nch = nd->nchunks, cbase = nd->chunk_base;
+  const uint32_t nch = nd->nchunks;
   clear_bins<BS>(cnt, bx);
   __syncthreads();
   float cmn[3], csz[3];
@@ -506,40 +572,15 @@ __global__ __launch_bounds__(kBlock) void k_decide(Args a) {
     csz[k] = nd->cbox[3 + k] - cmn[k];
   }
   if (nch) {
-    // a wide node: its chunks' partials added up (integer sums and ordered
-    // min / max: any order gives the same bins; 16 loads are issued before
-    // they are combined, so that the latency of the partials' reads, written
-    // by other XCDs, is paid once per 16 chunks)
-    const uint32_t* part = a.part + (size_t)cbase * kBinWords;
+    // a wide node: k_sum_chunks has its bins
+    const uint32_t* tot = a.tot + (size_t)nd->slot * kBinWords;
     for (uint32_t k = tid; k < kBinWords; k += BS) {
       const uint32_t axis = k < 192 ? k / 64 : (k - 192) / 384;
       if ((umask >> axis) & 1u) continue;
-      const uint32_t* q = part + k;
-      const int op = k < 192 ? 0 : ((k - 192) % 6) < 3 ? 1 : 2;  // sum, min, max
-      const uint32_t id0 = op == 1 ? 0xffffffffu : 0u;
-      uint32_t v0 = id0, v1 = id0, v2 = id0, v3 = id0;
-      auto acc = [&](uint32_t v, uint32_t w) {
-        return op == 0 ? v + w : op == 1 ? min(v, w) : max(v, w);
-      };
-      uint32_t c = 0;
-      for (; c + 16 <= nch; c += 16) {
-        uint32_t w[16];
-#pragma unroll
-        for (uint32_t j = 0; j < 16; j++) w[j] = q[(size_t)(c + j) * kBinWords];
-#pragma unroll
-        for (uint32_t j = 0; j < 16; j += 4) {
-          v0 = acc(v0, w[j]);
-          v1 = acc(v1, w[j + 1]);
-          v2 = acc(v2, w[j + 2]);
-          v3 = acc(v3, w[j + 3]);
-        }
-      }
-      for (; c < nch; c++) v0 = acc(v0, q[(size_t)c * kBinWords]);
-      const uint32_t v = acc(acc(v0, v1), acc(v2, v3));
       if (k < 192)
-        (&cnt[0][0])[k] = v;
+        (&cnt[0][0])[k] = tot[k];
       else
-        (&bx[0][0][0])[k - 192] = v;
+        (&bx[0][0][0])[k - 192] = tot[k];
     }
   } else {
     bin_centroids<BS>(a, refs, n, cmn, csz, umask, cnt, bx);
@@ -566,7 +607,6 @@ __global__ __launch_bounds__(kBlock) void k_decide(Args a) {
     float best = 0.0f;
     const int best_axis = choose_axis(splits, &best);
     uint32_t f = flags & ~kPending;
-    s_axis = -1;
     if (best_axis < 0) {
       atomicOr(&a.ctx->error, 2u);  // assert!(!is_first), bvh.rs:303
       f |= kLeaf;
@@ -578,32 +618,8 @@ __global__ __launch_bounds__(kBlock) void k_decide(Args a) {
       nd->left_count = splits.left[best_axis];
       if (a.mode == 0) nd->uniform_mask = 0;
       f |= kSplit;
-      s_axis = best_axis;
     }
     nd->flags = f;
-  }
-  if (!nch) return;
-  __syncthreads();
-  // a wide node split on centroid bins: where each chunk's references of
-  // each bin start in the stably sorted segment (bins in order, chunks in
-  // order within a bin)
-  const int ax = s_axis;
-  if (ax < 0 || ((umask >> ax) & 1u) || tid >= 64) return;
-  uint32_t run = 0;
-  for (uint32_t j = 0; j < tid; j++) run += cnt[ax][j];
-  const uint32_t* part = a.part + (size_t)cbase * kBinWords + (uint32_t)ax * 64 + tid;
-  uint32_t* offs = a.offs + (size_t)cbase * 64 + tid;
-  // 16 chunks' counts are loaded before they are summed, so that the scan
-  // does not wait for one load per chunk
-  for (uint32_t c0 = 0; c0 < nch; c0 += 16) {
-    uint32_t v[16];
-#pragma unroll
-    for (uint32_t j = 0; j < 16; j++) v[j] = c0 + j < nch ? part[(size_t)(c0 + j) * kBinWords] : 0u;
-#pragma unroll
-    for (uint32_t j = 0; j < 16; j++) {
-      if (c0 + j < nch) offs[(size_t)(c0 + j) * 64] = run;
-      run += v[j];
-    }
   }
 }
 
@@ -681,6 +697,7 @@ __device__ __forceinline__ void wg_stable_pass(uint32_t n, LoadFn load, DigitFn 
 // Sorted binning input: a stable sort of the segment by barycenter
 // coordinate (bvh.rs:176-190), as 4 stable 8-bit LSD passes.
 __global__ __launch_bounds__(kBlock) void k_sort(Args a) {
+  if (blockIdx.x / 3 >= a.ctx->large[a.parity]) return;
   const uint32_t id = a.list[blockIdx.x / 3];
   const uint32_t axis = blockIdx.x % 3;
   const INode* nd = &a.nodes[id];
@@ -750,16 +767,19 @@ __device__ __forceinline__ void side_bounds(const Args& a, const uint32_t* order
   group_sync<BS>();
 }
 
-// One chunk of a wide node that splits: its references go to the positions
-// k_decide computed (a stable sort by bin, or the sorted order's copy for a
-// uniform axis), and its part of the children's bounds to its side partial.
+// One chunk of a wide node that splits: its references go behind those of
+// smaller bins and of earlier chunks' same bin (a stable sort by bin, or the
+// sorted order's copy for a uniform axis), and its part of the children's
+// bounds to its side partial.  Every chunk adds up the counts of the chunks
+// before it, 8 waves sharing them: reading on average half of a node's counts
+// per chunk costs less than a scan of its own (60 us in one workgroup).
 __global__ __launch_bounds__(kBlock) void k_part_chunks(Args a) {
   const uint32_t c = blockIdx.x;
   if (c >= a.ctx->total_chunks) return;
   const INode* nd = &a.nodes[a.chunk_node[c]];
   if (!(nd->flags & kSplit)) return;
   const uint32_t n = nd->count, begin = nd->begin;
-  const uint32_t lo = (c - nd->chunk_base) * kChunk, hi = min(n, lo + kChunk);
+  const uint32_t lo = (c - nd->chunk_base) * a.chunk, hi = min(n, lo + a.chunk);
   const uint32_t par = (nd->flags & kParity) ? 1u : 0u;
   const uint32_t* src = a.buf[par] + begin;
   uint32_t* dst = a.buf[par ^ 1u] + begin;
@@ -779,8 +799,37 @@ __global__ __launch_bounds__(kBlock) void k_part_chunks(Args a) {
     const uint32_t* srt = a.sorted[axis] + begin;
     for (uint32_t s = lo + tid; s < hi; s += kBlock) dst[s] = srt[s];
   } else {
+    __shared__ uint32_t start[64];
+    __shared__ uint32_t before[kBlock / 64][64];
+    const uint32_t lane = tid & 63u, wave = tid >> 6, prior = c - nd->chunk_base;
+    const uint32_t* q = a.part + (size_t)nd->chunk_base * kBinWords + axis * 64 + lane;
+    uint32_t sum = 0;
+    for (uint32_t c0 = wave; c0 < prior; c0 += 8 * (kBlock / 64)) {
+      uint32_t v[8];
+#pragma unroll
+      for (uint32_t j = 0; j < 8; j++) {
+        const uint32_t k = c0 + j * (kBlock / 64);
+        v[j] = k < prior ? q[(size_t)k * kBinWords] : 0u;
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < 8; j++) sum += v[j];
+    }
+    before[wave][lane] = sum;
+    __syncthreads();
+    if (wave == 0) {
+      const uint32_t own = a.tot[(size_t)nd->slot * kBinWords + axis * 64 + lane];
+      uint32_t inc = own;
+      for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(inc, d);
+        if (lane >= d) inc += y;
+      }
+      inc -= own;
+      for (uint32_t w = 0; w < kBlock / 64; w++) inc += before[w][lane];
+      start[lane] = inc;
+    }
+    __syncthreads();
     auto load = [&](uint32_t e) { return src[lo + e]; };
-    wg_stable_pass<6, kBlock>(hi - lo, load, bin_of, dst, hist, wcount, a.offs + (size_t)c * 64);
+    wg_stable_pass<6, kBlock>(hi - lo, load, bin_of, dst, hist, wcount, start);
   }
   side_bounds<kBlock>(a, uniform ? a.sorted[axis] + begin : src, lo, hi, uniform, L, split, bin_of,
                      cb);
@@ -808,9 +857,9 @@ __device__ __forceinline__ uint32_t make_children(const Args& a, INode* nd, uint
     ch[s].flags = (par ^ 1u) ? kParity : 0u;
     ch[s].leaves = 0;
     ch[s].sar = 0.0f;
-    ch[s].depth = 0;
+    ch[s].depth = nd->depth + 1;
     ch[s].axis = ch[s].split_bin = ch[s].left_count = ch[s].uniform_mask = 0;
-    ch[s].chunk_base = ch[s].nchunks = 0;
+    ch[s].chunk_base = ch[s].nchunks = ch[s].slot = ch[s].pairs = ch[s].first_tri = 0;
   }
   // smaller area first (bvh.rs:337-345)
   const bool swap = area6(ch[0].box) > area6(ch[1].box);
@@ -828,6 +877,7 @@ __device__ __forceinline__ uint32_t make_children(const Args& a, INode* nd, uint
 // references in push order) and creates the children.
 __global__ __launch_bounds__(kBlock) void k_partition(Args a) {
   constexpr uint32_t BS = kBlock;
+  if (blockIdx.x >= a.ctx->large[a.parity]) return;
   const uint32_t id = a.list[blockIdx.x];
   INode* nd = &a.nodes[id];
   const uint32_t flags = nd->flags;
@@ -887,7 +937,7 @@ __global__ __launch_bounds__(kBlock) void k_partition(Args a) {
     for (uint32_t s = 0; s < 2; s++) {
       const uint32_t count = s == 0 ? L : n - L;
       if (count > kSub) {
-        a.next_list[atomicAdd(&a.ctx->next_large, 1u)] = c + s;
+        a.next_list[atomicAdd(&a.ctx->large[a.parity ^ 1u], 1u)] = c + s;
         if (count > kWide) atomicAdd(&a.ctx->next_wide, 1u);
       } else if (count > a.small_max) {
         a.sub_list[atomicAdd(&a.ctx->sub_count, 1u)] = c + s;
@@ -1079,7 +1129,7 @@ __global__ __launch_bounds__(256) void k_small(Args a) {
   __syncthreads();
   const uint32_t si = blockIdx.x * 8 + (threadIdx.x >> 5);
   const bool here = si < a.ctx->small_count;
-  uint32_t root = 0, n = 0, sbegin = 0, rflags = 0;
+  uint32_t root = 0, n = 0, sbegin = 0, rflags = 0, depth = 0;
   int32_t parent = -1;
   float box[6] = {0, 0, 0, 0, 0, 0};
   if (here) {
@@ -1089,6 +1139,7 @@ __global__ __launch_bounds__(256) void k_small(Args a) {
     sbegin = R.begin;
     rflags = R.flags;
     parent = R.parent;
+    depth = R.depth;
     for (int k = 0; k < 6; k++) box[k] = R.box[k];
   }
   const uint32_t par = rflags & kParity;
@@ -1122,8 +1173,9 @@ __global__ __launch_bounds__(256) void k_small(Args a) {
     w.child[0] = c0;
     w.child[1] = c1;
     w.flags = f;
+    w.depth = depth;
   };
-  while (__any(open)) {
+  for (; __any(open); depth++) {
     if (open && cnt == 1) {
       write_node(flags | kLeaf, -1, -1);
       open = false;
@@ -1245,35 +1297,38 @@ __global__ __launch_bounds__(256) void k_small(Args a) {
 // Statistics and layout
 // ---------------------------------------------------------------------------
 
-// Depth of every node (a walk to the root), the tree's depth, and the
-// leaves' statistics (one leaf, summed_area_ratio 0 + 0).
-// Depth of every node; leaves start the bottom-up statistics; inner nodes
-// are counted per depth (dcount holds dcap >= max depth + 1 words), in LDS
-// per workgroup first (one global atomic per workgroup and depth: a global
-// counter per depth shared by all nodes serialises).
+// The tree's depth, the largest leaf and the leaves' statistics (one leaf,
+// summed_area_ratio 0 + 0); inner nodes are counted per depth (dcount holds
+// dcap >= max depth + 1 words), in LDS per workgroup first (one global atomic
+// per workgroup and value: a global counter shared by all nodes serialises).
 constexpr uint32_t kDepthLds = 512;
 __global__ __launch_bounds__(256) void k_depth(Args a, uint32_t ninodes, uint32_t* dcount,
                                                uint32_t dcap) {
   __shared__ uint32_t cnt[kDepthLds];
+  __shared__ uint32_t deepest, largest;
   const bool local = dcap <= kDepthLds;
   if (local)
     for (uint32_t k = threadIdx.x; k < dcap; k += 256) cnt[k] = 0;
+  if (threadIdx.x == 0) deepest = largest = 0;
   __syncthreads();
   const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
   INode* nodes = a.nodes;
   if (x < ninodes && !(nodes[x].flags & kHole)) {
-    uint32_t d = 0;
-    for (int32_t u = nodes[x].parent; u >= 0; u = nodes[u].parent) d++;
-    nodes[x].depth = d;
+    const uint32_t d = nodes[x].depth;
     if (nodes[x].flags & kLeaf) {
       nodes[x].leaves = 1;
       nodes[x].sar = 0.0f + 0.0f;
-      atomicMax(&a.ctx->max_depth, d);
+      atomicMax(&deepest, d);
+      atomicMax(&largest, nodes[x].count);
     } else if (d < dcap) {
       atomicAdd(local ? &cnt[d] : &dcount[d], 1u);
     }
   }
   __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicMax(&a.ctx->max_depth, deepest);
+    atomicMax(&a.ctx->max_leaf, largest);
+  }
   if (local)
     for (uint32_t k = threadIdx.x; k < dcap; k += 256)
       if (cnt[k]) atomicAdd(&dcount[k], cnt[k]);
@@ -1305,73 +1360,71 @@ __global__ __launch_bounds__(256) void k_depth_lists(Args a, uint32_t ninodes, u
   if (inner) list[local ? cnt[d] + rank : atomicAdd(&cursor[d], 1u)] = x;
 }
 
-// Leaf counts and summed_area_ratio (bvh.rs:380-386) of the inner nodes of
-// one depth (listed by k_depth_lists), from their children: one launch per
-// depth, deepest first, each over that depth's nodes only.
-__global__ __launch_bounds__(256) void k_bottom_up(Args a, const uint32_t* list, uint32_t n) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
+// Runs visit(x) for the inner nodes x of the depths lo .. hi (listed by
+// k_depth_lists; ends[d] is the end of depth d's part of the list), one depth
+// after the other, deepest first (UP) or last.  One depth takes any number of
+// workgroups; several, a launch each of which would mostly be its overhead,
+// one workgroup.
+template <bool UP, typename Visit>
+__device__ __forceinline__ void by_depth(const uint32_t* list, const uint32_t* ends, uint32_t lo,
+                                         uint32_t hi, Visit visit) {
+  for (uint32_t q = 0; q <= hi - lo; q++) {
+    const uint32_t d = UP ? hi - q : lo + q;
+    const uint32_t end = ends[d];
+    for (uint32_t k = (d ? ends[d - 1] : 0u) + blockIdx.x * blockDim.x + threadIdx.x; k < end;
+         k += gridDim.x * blockDim.x)
+      visit(list[k]);
+    if (lo != hi) __syncthreads();
+  }
+}
+
+// Leaf counts and summed_area_ratio (bvh.rs:380-386) of inner nodes from
+// their children.
+__global__ __launch_bounds__(1024) void k_bottom_up(Args a, const uint32_t* list,
+                                                    const uint32_t* ends, uint32_t lo,
+                                                    uint32_t hi) {
   INode* nodes = a.nodes;
-  const uint32_t x = list[k];
-  const int32_t c0 = nodes[x].child[0], c1 = nodes[x].child[1];
-  const float s0 = nodes[c0].sar, s1 = nodes[c1].sar;
-  const float A = area6(nodes[x].box);
-  const float cc = (0.0f + s0) + s1;
-  const float cs = (0.0f + area6(nodes[c0].box) / A) + area6(nodes[c1].box) / A;
-  nodes[x].leaves = nodes[c0].leaves + nodes[c1].leaves;
-  nodes[x].sar = cs + cc;
+  by_depth<true>(list, ends, lo, hi, [&](uint32_t x) {
+    const int32_t c0 = nodes[x].child[0], c1 = nodes[x].child[1];
+    const float s0 = nodes[c0].sar, s1 = nodes[c1].sar;
+    const float A = area6(nodes[x].box);
+    const float cc = (0.0f + s0) + s1;
+    const float cs = (0.0f + area6(nodes[c0].box) / A) + area6(nodes[c1].box) / A;
+    nodes[x].leaves = nodes[c0].leaves + nodes[c1].leaves;
+    nodes[x].sar = cs + cc;
+  });
 }
 
-// Counters of the next level's node lists back to zero.
-__global__ void k_level_reset(Ctx* ctx) {
-  if (threadIdx.x == 0) {
-    ctx->next_large = 0;
-    ctx->next_wide = 0;
-  }
-}
-
-// crystallize (bvh.rs:389-428): node x is written at L(parent) + [x is c1],
-// where L(u) = nodes.len() when u is crystallised; a leaf's triangles start
-// at T(x).  Both are sums over the path to the root.
-__global__ __launch_bounds__(256) void k_layout(Args a, uint32_t ninodes, DevNode* out,
+// crystallize (bvh.rs:389-428), from the root down: an inner node's two
+// children are written at nodes.len() at its turn, L(x).  The first child's
+// own children follow at L(x) + 2, the second's behind all pairs of the
+// first's subtree, and triangles follow their leaves' order.  (Every node
+// walking up to the root for these sums took 0.98 ms for 1.33 M triangles.)
+__global__ __launch_bounds__(1024) void k_place(Args a, const uint32_t* list, const uint32_t* ends,
+                                                uint32_t lo, uint32_t hi, DevNode* out,
                                                 uint32_t* order) {
-  uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= ninodes || x == 0) return;
-  const INode* nodes = a.nodes;
-  const INode& nx = nodes[x];
-  if (nx.flags & kHole) return;
-  uint32_t Lx = 0, Tx = 0, depth = 0;
-  uint32_t c = x;
-  for (;;) {
-    int32_t u = nodes[c].parent;
-    if (u < 0) break;
-    depth++;
-    if (nodes[c].flags & kIsC1) {
-      const INode& sib = nodes[nodes[u].child[0]];
-      Lx += 2 + 2 * (sib.leaves - 1);
-      Tx += sib.count;
-    } else {
-      Lx += 2;
+  INode* nodes = a.nodes;
+  by_depth<false>(list, ends, lo, hi, [&](uint32_t x) {
+    const uint32_t at = nodes[x].pairs;
+    uint32_t L = at + 2, T = nodes[x].first_tri;
+    for (uint32_t s = 0; s < 2; s++) {
+      INode& c = nodes[nodes[x].child[s]];
+      const bool leaf = c.flags & kLeaf;
+      DevNode d;
+      d.a = make_float4(c.box[0], c.box[1], c.box[2], c.box[3]);
+      d.b = make_float4(c.box[4], c.box[5], u2f(leaf ? T : L), u2f(leaf ? c.count : 0u));
+      out[at + s] = d;
+      if (leaf) {
+        const uint32_t* src = a.buf[(c.flags & kParity) ? 1 : 0] + c.begin;
+        for (uint32_t k = 0; k < c.count; k++) order[T + k] = src[k];
+      } else {
+        c.pairs = L;
+        c.first_tri = T;
+      }
+      T += c.count;
+      L += 2 * (c.leaves - 1);
     }
-    c = (uint32_t)u;
-  }
-  const bool c1 = nx.flags & kIsC1;
-  const INode& par = nodes[nx.parent];
-  uint32_t Lp = Lx - 2 - (c1 ? 2 * (nodes[par.child[0]].leaves - 1) : 0);
-  uint32_t slot = Lp + (c1 ? 1u : 0u);
-  const bool leaf = nx.flags & kLeaf;
-  uint32_t index = leaf ? Tx : Lx;
-  uint32_t len = leaf ? nx.count : 0u;
-  DevNode d;
-  d.a = make_float4(nx.box[0], nx.box[1], nx.box[2], nx.box[3]);
-  d.b = make_float4(nx.box[4], nx.box[5], u2f(index), u2f(len));
-  out[slot] = d;
-  if (leaf) {
-    const uint32_t* src = a.buf[(nx.flags & kParity) ? 1 : 0] + nx.begin;
-    for (uint32_t k = 0; k < nx.count; k++) order[Tx + k] = src[k];
-    atomicMax(&a.ctx->max_leaf, nx.count);
-    atomicMax(&a.ctx->max_depth, depth);
-  }
+  });
 }
 
 }  // namespace bvh
@@ -1425,9 +1478,12 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   Ctx* ctx;
   const size_t list_cap = N / (kSub + 1) + 2, sub_cap = N / (a.small_max + 1) + 2;
   uint32_t *listA, *listB, *sub, *small, *dcount, *dlist;
+  // references per chunk of a wide node: enough chunks for the 256 CUs, but
+  // not more partials than they are worth
+  a.chunk = N <= 131072 ? 512u : N <= 524288 ? 1024u : 2048u;
   // chunks of the wide nodes of one level: their triangles are disjoint, so
-  // at most N / kChunk + (number of wide nodes) chunks
-  const size_t max_chunks = N / kChunk + N / kWide + 2;
+  // at most N / chunk + (number of wide nodes) chunks
+  const size_t max_wide = N / (kWide + 1) + 1, max_chunks = N / a.chunk + max_wide + 1;
   // depths: at most one level per triangle
   const size_t dcount_cap = 2 * N + 64;
   float *d_tpm, *d_tpm1;
@@ -1447,9 +1503,10 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
     take(&listB, list_cap);
     take(&sub, sub_cap);
     take(&small, N / 2 + 2);
+    take(&a.wide_list, max_wide);
+    take(&a.tot, max_wide * kBinWords);
     take(&a.chunk_node, max_chunks);
     take(&a.part, max_chunks * kBinWords);
-    take(&a.offs, max_chunks * 64);
     take(&a.side, max_chunks * 24);
     take(&d_tpm, N + 1);
     take(&d_tpm1, N + 1);
@@ -1515,6 +1572,7 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   uint32_t nlist = 0;
   if (ntris > kSub) {
     BVH_CHECK(hipMemcpyAsync(listA, &zero, 4, hipMemcpyHostToDevice, s));
+    BVH_CHECK(hipMemcpyAsync(&ctx->large[0], &one, 4, hipMemcpyHostToDevice, s));
     nlist = 1;
   } else if (ntris > a.small_max) {
     BVH_CHECK(hipMemcpyAsync(sub, &zero, 4, hipMemcpyHostToDevice, s));
@@ -1523,48 +1581,51 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
     BVH_CHECK(hipMemcpyAsync(small, &zero, 4, hipMemcpyHostToDevice, s));
     BVH_CHECK(hipMemcpyAsync(&ctx->small_count, &one, 4, hipMemcpyHostToDevice, s));
   }
-  uint32_t* cur = listA;
-  uint32_t* nxt = listB;
+  uint32_t* lists[2] = {listA, listB};
   bool wide = ntris > kWide;
   uint32_t nsub = ntris > a.small_max ? 1u : 0u;  // nodes for k_subtree so far
-  uint32_t levels = 0;  // iterations of the level phase
+  uint32_t levels = 0;                            // iterations of the level phase
+  // The lists' lengths stay on the device and the grids are their bounds (a
+  // level has at most twice the nodes of the one before), so that the host
+  // waits once in kLevelBatch levels; the levels enqueued past the last one
+  // find empty lists.
   while (nlist > 0) {
-    levels++;
-    a.list = cur;
-    a.nlist = nlist;
-    a.next_list = nxt;
-    a.mode = 0;
-    if (wide) {
-      hipLaunchKernelGGL(k_wide_plan, dim3(1), dim3(1024), 0, s, a);
+    for (uint32_t q = 0; q < kLevelBatch; q++, levels++) {
+      const uint32_t most = (uint32_t)std::min<size_t>((size_t)nlist << q, list_cap);
+      const uint32_t most_wide = (uint32_t)std::min<size_t>(most, max_wide);
+      a.parity = levels & 1u;
+      a.list = lists[a.parity];
+      a.next_list = lists[a.parity ^ 1u];
+      hipLaunchKernelGGL(k_level_plan, dim3(1), dim3(1024), 0, s, a);
       BVH_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(k_bin_chunks, dim3((uint32_t)max_chunks), dim3(kBlock), 0, s, a);
+      if (wide) {
+        hipLaunchKernelGGL(k_bin_chunks, dim3((uint32_t)max_chunks), dim3(kBlock), 0, s, a);
+        BVH_CHECK(hipGetLastError());
+        hipLaunchKernelGGL(k_sum_chunks, dim3(most_wide, kBinWords / 64), dim3(256), 0, s, a);
+        BVH_CHECK(hipGetLastError());
+      }
+      a.mode = 0;
+      hipLaunchKernelGGL(k_decide, dim3(most), dim3(kBlock), 0, s, a);
+      BVH_CHECK(hipGetLastError());
+      hipLaunchKernelGGL(k_sort, dim3(most * 3), dim3(kBlock), 0, s, a);
+      BVH_CHECK(hipGetLastError());
+      a.mode = 1;
+      hipLaunchKernelGGL(k_decide, dim3(most), dim3(kBlock), 0, s, a);
+      BVH_CHECK(hipGetLastError());
+      if (wide) {
+        hipLaunchKernelGGL(k_part_chunks, dim3((uint32_t)max_chunks), dim3(kBlock), 0, s, a);
+        BVH_CHECK(hipGetLastError());
+      }
+      hipLaunchKernelGGL(k_partition, dim3(most), dim3(kBlock), 0, s, a);
       BVH_CHECK(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_decide, dim3(nlist), dim3(kBlock), 0, s, a);
-    BVH_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_sort, dim3(nlist * 3), dim3(kBlock), 0, s, a);
-    BVH_CHECK(hipGetLastError());
-    a.mode = 1;
-    hipLaunchKernelGGL(k_decide, dim3(nlist), dim3(kBlock), 0, s, a);
-    BVH_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_level_reset, dim3(1), dim3(64), 0, s, ctx);
-    BVH_CHECK(hipGetLastError());
-    if (wide) {
-      hipLaunchKernelGGL(k_part_chunks, dim3((uint32_t)max_chunks), dim3(kBlock), 0, s, a);
-      BVH_CHECK(hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_partition, dim3(nlist), dim3(kBlock), 0, s, a);
-    BVH_CHECK(hipGetLastError());
-    uint32_t hctl[7];
-    BVH_CHECK(hipMemcpyAsync(hctl, ctx, 28, hipMemcpyDeviceToHost, s));
+    Ctx hl;
+    BVH_CHECK(hipMemcpyAsync(&hl, ctx, sizeof(Ctx), hipMemcpyDeviceToHost, s));
     BVH_CHECK(hipStreamSynchronize(s));
-    if (hctl[3]) break;
-    nlist = hctl[1];
-    wide = hctl[4] > 0;
-    nsub = hctl[6];
-    uint32_t* t = cur;
-    cur = nxt;
-    nxt = t;
+    if (hl.error) break;
+    nlist = hl.large[levels & 1u];
+    wide = hl.next_wide > 0;
+    nsub = hl.sub_count;
   }
   // (both exit at once after an error, and k_small beyond the nodes listed,
   // so neither waits for the host to read the counters)
@@ -1616,18 +1677,34 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
     hoff[d] = run;
     run += hcount[d];
   }
+  // (k_depth_lists moves every depth's offset to the depth's end)
   BVH_CHECK(hipMemcpyAsync(dcount, hoff.data(), (size_t)dcap * 4, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_depth_lists, dim3(blocks), dim3(256), 0, s, a, ninodes, dcount, dcap,
                      dlist);
   BVH_CHECK(hipGetLastError());
-  for (uint32_t d = hc.max_depth; d-- > 0;) {
-    if (!hcount[d]) continue;
-    hipLaunchKernelGGL(k_bottom_up, dim3((hcount[d] + 255) / 256), dim3(256), 0, s, a,
-                       dlist + hoff[d], hcount[d]);
+  // consecutive depths of few nodes share a launch of one workgroup
+  struct Depths {
+    uint32_t lo, hi, blocks;
+  };
+  std::vector<Depths> groups;
+  for (uint32_t d = 0; d < hc.max_depth; d++) {
+    const bool few = hcount[d] <= kDepthFew;
+    if (few && !groups.empty() && groups.back().blocks == 1)
+      groups.back().hi = d;
+    else
+      groups.push_back(Depths{d, d, few ? 1u : (hcount[d] + 255) / 256});
+  }
+  for (size_t k = groups.size(); k-- > 0;) {
+    const Depths& g = groups[k];
+    hipLaunchKernelGGL(k_bottom_up, dim3(g.blocks), dim3(g.blocks == 1 ? 1024 : 256), 0, s, a,
+                       dlist, dcount, g.lo, g.hi);
     BVH_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_layout, dim3(blocks), dim3(256), 0, s, a, ninodes, nodes_out, order_out);
-  BVH_CHECK(hipGetLastError());
+  for (const Depths& g : groups) {
+    hipLaunchKernelGGL(k_place, dim3(g.blocks), dim3(g.blocks == 1 ? 1024 : 256), 0, s, a, dlist,
+                       dcount, g.lo, g.hi, nodes_out, order_out);
+    BVH_CHECK(hipGetLastError());
+  }
   BVH_CHECK(hipEventRecord(ev1, s));
   BVH_CHECK(hipMemcpyAsync(&hc, ctx, sizeof(Ctx), hipMemcpyDeviceToHost, s));
   BVH_CHECK(hipMemcpyAsync(&root_h, a.nodes, sizeof(INode), hipMemcpyDeviceToHost, s));
