@@ -722,7 +722,6 @@ static cv_status scene_finish(cv_scene* s, const cv_mesh* const* meshes, size_t 
   // traversal configuration: packed stack entries need index < 2^27 and
   // leaves of at most 31 triangles
   s->packed = s->info.max_leaf <= 31 && N < (1u << 27) && s->info.num_nodes < (1u << 27);
-  HIPTRY(s->cursor.alloc(cvk::kIsectGroups * cvk::kIsectCursorStride), "alloc");
   cv_tuning t{8, 32, 16, 1, 1};
   return scene_apply_tuning(s, t);
 }
@@ -829,7 +828,6 @@ void cv_scene_destroy(cv_scene* s) {
   s->direct.reset();
   s->lights.reset();
   s->spill.reset();
-  s->cursor.reset();
   s->q_ctrl.reset();
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
@@ -867,74 +865,69 @@ cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_
       ip = d_isects.p;
     }
   }
-  if (hits && !isects) {
-    // Hits only: the renderer's lane-refill traversal (idle lanes take new
-    // rays, lanes at leaves wait for a common leaf round) as a one-bounce
-    // step over the caller's rays, writing source indices; each lane's
-    // operations are those of the single-ray traversal, so the hits are
-    // the same bits.
-    cvk::ExtendArgs x{};
-    x.n = (uint32_t)n;
-    x.bounce = 0;
-    x.rays6 = rp;
-    x.tri_src = s->tri_src.p;
-    x.hits = reinterpret_cast<uint4*>(hp);
-    cv_status ws = cvh::ensure_wide_locked(s, s->cfg.width);
-    if (ws != CV_OK) return ws;
-    x.nodes = cvh::traversal_nodes(s, s->cfg.width);
-    x.tris = s->tris.p;
-    x.jobs = nullptr;
-    x.spill = s->spill.p;
-    // At least 4 batches of 64 rays per cursor fetch: queries end after a
-    // few dozen box tests, so one fetch per 64 rays serialises on the
-    // cursor (3.4 ms for 2^24 rays whatever the scene; 2.0 ms with 4 on
-    // 968 triangles).  Rendering keeps the tuned value (1 is fastest there).
-    x.batches = s->cfg.fetch_batches > 4 ? s->cfg.fetch_batches : 4u;
-    x.refill = s->cfg.refill <= 64 ? s->cfg.refill : 0u;
-    // Refill checks 4 times as often as the renderer's: a query ends after
-    // a few dozen box tests, so a finished lane would otherwise idle for a
-    // large share of a ray's steps (2^24 rays on suzanne: 1.79 -> 1.65 ms
-    // with 4 steps between checks instead of 16; the bunny's within 1 %).
-    x.interval = s->cfg.refill_interval > 4 ? s->cfg.refill_interval / 4 : 1u;
-    x.leaf_batch = s->cfg.leaf_batch <= 64 ? s->cfg.leaf_batch : 0u;
-    x.parts = s->cfg.parts;
-    // Up to kQueryDeal rays per lane the rays are dealt out to at most 24
-    // waves per CU, which is as fast as 32 for many rays and ends sooner with
-    // few (10^6 rays in a 200,000-triangle room: cursors 1.04 ms, dealt to 32
-    // waves per CU 1.03, to 24 0.86; 2 x 10^6: 1.51, 1.62, 1.42; 4 x 10^6:
-    // 2.29, 2.80, 2.33).  Whole-batch launches always use the cursor.
-    const uint32_t bw = s->cfg.block_waves;
-    const uint32_t few = std::min(s->cfg.blocks, 24u * cvh::num_cus());
-    const uint64_t few_lanes = (uint64_t)((few + bw - 1) / bw * bw) * 64u;
-    x.deal = n <= few_lanes * kQueryDeal && (x.refill || s->cfg.width != 2);
-    if (!x.deal) {
-      if (!s->q_ctrl.p) HIPTRY(s->q_ctrl.alloc(1), "alloc");
-      HIPTRY(cvk::launch_query_ctrl(s->q_ctrl.p, (uint32_t)n, st), "query control");
-      x.ctrl = s->q_ctrl.p;
-    }
-    HIPTRY(cvk::launch_extend(x, false, s->packed, false, s->cfg.stack,
-                              x.deal ? few : s->cfg.blocks, bw, st, s->cfg.width),
-           "intersect");
-    if (!dev) HIPTRY(hipMemcpyAsync(hits, hp, 16 * n, hipMemcpyDeviceToHost, st), "download");
-    HIPTRY(hipStreamSynchronize(st), "sync");
-    return CV_OK;
+  if (!hits && !isects) return CV_OK;
+  // The renderer's lane-refill traversal (idle lanes take new rays, lanes at
+  // leaves wait for a common leaf round) as a one-bounce step over the
+  // caller's rays; each lane's operations are those of the single-ray
+  // traversal, so the hits are the same bits.  Full records keep the
+  // reference's tree, whose counters they hold; hits take the tuned one.
+  const uint32_t width = isects ? 2u : s->cfg.width;
+  cvk::ExtendArgs x{};
+  x.n = (uint32_t)n;
+  x.bounce = 0;
+  x.rays6 = rp;
+  x.tri_src = s->tri_src.p;
+  x.hits = reinterpret_cast<uint4*>(hp);
+  x.records = ip;
+  cv_status ws = cvh::ensure_wide_locked(s, width);
+  if (ws != CV_OK) return ws;
+  x.nodes = cvh::traversal_nodes(s, width);
+  x.tris = s->tris.p;
+  x.jobs = nullptr;
+  x.spill = s->spill.p;
+  // At least 4 batches of 64 rays per cursor fetch: queries end after a
+  // few dozen box tests, so one fetch per 64 rays serialises on the
+  // cursor (3.4 ms for 2^24 rays whatever the scene; 2.0 ms with 4 on
+  // 968 triangles).  Rendering keeps the tuned value (1 is fastest there).
+  x.batches = s->cfg.fetch_batches > 4 ? s->cfg.fetch_batches : 4u;
+  x.refill = s->cfg.refill <= 64 ? s->cfg.refill : isects ? 64u : 0u;
+  // Refill checks 4 times as often as the renderer's: a query ends after
+  // a few dozen box tests, so a finished lane would otherwise idle for a
+  // large share of a ray's steps (2^24 rays on suzanne: 1.79 -> 1.65 ms
+  // with 4 steps between checks instead of 16; the bunny's within 1 %).
+  x.interval = s->cfg.refill_interval > 4 ? s->cfg.refill_interval / 4 : 1u;
+  x.leaf_batch = s->cfg.leaf_batch <= 64 ? s->cfg.leaf_batch : 0u;
+  x.parts = s->cfg.parts;
+  // Up to kQueryDeal rays per lane the rays are dealt out to at most 24
+  // waves per CU, which is as fast as 32 for many rays and ends sooner with
+  // few (10^6 rays in a 200,000-triangle room: cursors 1.04 ms, dealt to 32
+  // waves per CU 1.03, to 24 0.86; 2 x 10^6: 1.51, 1.62, 1.42; 4 x 10^6:
+  // 2.29, 2.80, 2.33).  Whole-batch launches always use the cursor.
+  const uint32_t bw = s->cfg.block_waves;
+  const uint32_t few = std::min(s->cfg.blocks, 24u * cvh::num_cus());
+  const uint64_t few_lanes = (uint64_t)((few + bw - 1) / bw * bw) * 64u;
+  x.deal = n <= few_lanes * kQueryDeal && (x.refill || width != 2);
+  if (!x.deal) {
+    if (!s->q_ctrl.p) HIPTRY(s->q_ctrl.alloc(1), "alloc");
+    HIPTRY(cvk::launch_query_ctrl(s->q_ctrl.p, (uint32_t)n, st), "query control");
+    x.ctrl = s->q_ctrl.p;
   }
-  cvk::IntersectArgs a{};
-  a.rays = rp;
-  a.n = (uint32_t)n;
-  a.cursor = s->cursor.p;
-  a.nodes = s->nodes.p;
-  a.tris = s->tris.p;
-  a.tri_src = s->tri_src.p;
-  a.tri_mat = s->tri_mat.p;
-  a.tri_uv = s->tri_uv.p;
-  a.spill = s->spill.p;
-  a.hits = hp;
-  a.isects = ip;
-  HIPTRY(cvk::launch_zero_u32(s->cursor.p, cvk::kIsectGroups * cvk::kIsectCursorStride, st),
-         "zero");
-  HIPTRY(cvk::launch_intersect(a, isects != nullptr, s->packed, s->cfg.stack, s->cfg.blocks, st),
-         "intersect");
+  const uint32_t blocks = x.deal ? few : s->cfg.blocks;
+  if (isects) {
+    cvk::IntersectArgs a{};
+    a.rays = rp;
+    a.n = (uint32_t)n;
+    a.tris = s->tris.p;
+    a.tri_src = s->tri_src.p;
+    a.tri_mat = s->tri_mat.p;
+    a.tri_uv = s->tri_uv.p;
+    a.hits = hp;
+    a.isects = ip;
+    HIPTRY(cvk::launch_records(x, a, s->packed, s->cfg.stack, blocks, bw, st), "intersect");
+  } else {
+    HIPTRY(cvk::launch_extend(x, false, s->packed, false, s->cfg.stack, blocks, bw, st, width),
+           "intersect");
+  }
   if (!dev) {
     if (hits) HIPTRY(hipMemcpyAsync(hits, hp, 16 * n, hipMemcpyDeviceToHost, st), "download");
     if (isects) HIPTRY(hipMemcpyAsync(isects, ip, 64 * n, hipMemcpyDeviceToHost, st), "download");
@@ -952,8 +945,7 @@ namespace {
 // (8 per CU), 32 LDS stack entries per lane, and the deeper entries of
 // trees up to CV_NOALLOC_MAX_DEPTH levels in the spill area.
 constexpr uint32_t kNoAllocWaves = 2048;
-constexpr int kNoAllocStack = 32;
-constexpr size_t kNoAllocSpillPerLane = CV_NOALLOC_MAX_DEPTH + 4 - kNoAllocStack;
+constexpr size_t kNoAllocSpillPerLane = CV_NOALLOC_MAX_DEPTH + 4 - cvk::kIsectStack;
 constexpr size_t kNoAllocCursorBytes =
     (size_t)cvk::kIsectGroups * cvk::kIsectCursorStride * sizeof(uint32_t);
 constexpr size_t kNoAllocBytes =
@@ -1011,9 +1003,7 @@ cv_status cv_bvh_intersect_nearest_noalloc(const cv_scene* sc, const cv_ray* ray
   // the cursors start at zero for every call (a fill kernel, no memset node)
   HIPTRY(cvk::launch_zero_u32(a.cursor, cvk::kIsectGroups * cvk::kIsectCursorStride, st),
          "zero");
-  HIPTRY(cvk::launch_intersect(a, isects != nullptr, s->packed, kNoAllocStack, kNoAllocWaves,
-                               st),
-         "intersect");
+  HIPTRY(cvk::launch_intersect(a, isects != nullptr, s->packed, kNoAllocWaves, st), "intersect");
   HIPTRY(hipStreamSynchronize(st), "sync");
   return CV_OK;
 }

@@ -103,6 +103,7 @@ struct ExtendArgs {
   const uint32_t* order;      // non-null: queue position k traverses path order[k]
   uint32_t parts;             // lane refill: 1 (one cursor) or kParts queue partitions
   uint32_t n;                 // batched queries: the number of rays
+  uint32_t* records;          // batched queries with full records: n x 16 u32
   bool deal;                  // batched queries: the rays are dealt out to the launch's waves
                               // beforehand, without cursors
 };
@@ -137,7 +138,7 @@ struct ShadeArgs {
   const JobDesc* jobs;
 };
 
-// cv_bvh_intersect_nearest's work cursors: kIsectGroups words,
+// The allocation-free query's work cursors: kIsectGroups words,
 // kIsectCursorStride words (128 bytes) apart.
 constexpr uint32_t kIsectGroups = 64;
 constexpr uint32_t kIsectCursorStride = 32;
@@ -156,8 +157,15 @@ struct IntersectArgs {
   uint32_t* isects;  // n x 16 u32 or null
 };
 
-hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, int stack,
-                            uint32_t blocks, hipStream_t s);
+// Queries with full records through the lane-refill traversal (a.records =
+// r.isects), then the pass that completes the records.
+hipError_t launch_records(const ExtendArgs& a, const IntersectArgs& r, bool packed, int stack,
+                          uint32_t blocks, uint32_t block_waves, hipStream_t s);
+// One 64-ray batch after the other per wave, kIsectStack LDS stack entries
+// per lane: the allocation-free query.
+constexpr int kIsectStack = 32;
+hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, uint32_t blocks,
+                            hipStream_t s);
 
 // CV_RNG_REF_PATCH rendering: patches (x, y, width, 0) of the job's image,
 // frames first_frame .. first_frame + nframes - 1 of each in order, into

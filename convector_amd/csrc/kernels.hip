@@ -317,8 +317,46 @@ __device__ __forceinline__ uint32_t fetch_below(uint32_t* cursor, uint32_t limit
   return __shfl(k, 0);
 }
 
+// Four words at any word address.
+typedef uint32_t words4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// A query's outputs for ray i: its hit and, when asked for, the deferred
+// MIntersection fields (triangle.rs:129-142, scene.rs:221-228).
+__device__ __forceinline__ void write_record(const IntersectArgs& a, uint32_t i, V3 o, V3 d,
+                                             const TravState& ts) {
+  const uint32_t src = ts.best == kNoHit ? kNoHit : a.tri_src[ts.best];
+  if (a.hits) {
+    reinterpret_cast<uint4*>(a.hits)[i] =
+        make_uint4(src, f2u(ts.best_t), f2u(ts.bu), f2u(ts.bv));
+  }
+  if (!a.isects) return;
+  V3 pos, nrm;
+  uint32_t mat;
+  float tu = 0.0f, tv = 0.0f;
+  if (ts.best == kNoHit) {
+    pos = muladd3(d, 1.0e5f, o);
+    nrm = d;
+    mat = kMatSky;
+  } else {
+    const float4* tp = reinterpret_cast<const float4*>(a.tris + ts.best);
+    V3 n = mk3(tp[0].w, tp[1].w, tp[2].w);
+    pos = muladd3(d, ts.best_t, o);
+    nrm = normalized3(n);
+    mat = a.tri_mat[ts.best];
+    const float* uv = a.tri_uv + 6 * (size_t)ts.best;
+    float w = (1.0f - ts.bu) - ts.bv;
+    tu = fmaf(uv[0], w, fmaf(uv[2], ts.bv, uv[4] * ts.bu));
+    tv = fmaf(uv[1], w, fmaf(uv[3], ts.bv, uv[5] * ts.bu));
+  }
+  words4* out = reinterpret_cast<words4*>(a.isects + 16 * (size_t)i);
+  out[0] = words4{f2u(pos.x), f2u(pos.y), f2u(pos.z), f2u(nrm.x)};
+  out[1] = words4{f2u(nrm.y), f2u(nrm.z), f2u(ts.best_t), mat};
+  out[2] = words4{f2u(tu), f2u(tv), src, f2u(ts.bu)};
+  out[3] = words4{f2u(ts.bv), ts.na, ts.nt, 0u};
+}
+
 // ---------------------------------------------------------------------------
-// cv_bvh_intersect_nearest
+// cv_bvh_intersect_nearest_noalloc, and the outputs of every query
 // ---------------------------------------------------------------------------
 
 // The n / 64 batches of 64 rays are split into kIsectGroups contiguous
@@ -356,49 +394,7 @@ __global__ __launch_bounds__(64) void k_intersect(IntersectArgs a) {
     TravState ts = traverse<COUNT, S, PACKED>(a.nodes, a.tris, o, d, lds + lane,
                                               a.spill + gtid, stride, valid);
     if (!valid) continue;
-    uint32_t src = ts.best == kNoHit ? kNoHit : a.tri_src[ts.best];
-    if (a.hits) {
-      reinterpret_cast<uint4*>(a.hits)[i] =
-          make_uint4(src, f2u(ts.best_t), f2u(ts.bu), f2u(ts.bv));
-    }
-    if (a.isects) {
-      // The deferred MIntersection fields (triangle.rs:129-142, scene.rs:221-228).
-      V3 pos, nrm;
-      uint32_t mat;
-      float tu = 0.0f, tv = 0.0f;
-      if (ts.best == kNoHit) {
-        pos = muladd3(d, 1.0e5f, o);
-        nrm = d;
-        mat = kMatSky;
-      } else {
-        const float4* tp = reinterpret_cast<const float4*>(a.tris + ts.best);
-        V3 n = mk3(tp[0].w, tp[1].w, tp[2].w);
-        pos = muladd3(d, ts.best_t, o);
-        nrm = normalized3(n);
-        mat = a.tri_mat[ts.best];
-        const float* uv = a.tri_uv + 6 * (size_t)ts.best;
-        float w = (1.0f - ts.bu) - ts.bv;
-        tu = fmaf(uv[0], w, fmaf(uv[2], ts.bv, uv[4] * ts.bu));
-        tv = fmaf(uv[1], w, fmaf(uv[3], ts.bv, uv[5] * ts.bu));
-      }
-      uint32_t* out = a.isects + 16 * (size_t)i;
-      out[0] = f2u(pos.x);
-      out[1] = f2u(pos.y);
-      out[2] = f2u(pos.z);
-      out[3] = f2u(nrm.x);
-      out[4] = f2u(nrm.y);
-      out[5] = f2u(nrm.z);
-      out[6] = f2u(ts.best_t);
-      out[7] = mat;
-      out[8] = f2u(tu);
-      out[9] = f2u(tv);
-      out[10] = src;
-      out[11] = f2u(ts.bu);
-      out[12] = f2u(ts.bv);
-      out[13] = ts.na;
-      out[14] = ts.nt;
-      out[15] = 0;
-    }
+    write_record(a, i, o, d, ts);
   }
 }
 
@@ -1017,9 +1013,16 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
           trav_step_wide<COUNT, S, W>(reinterpret_cast<const float4*>(nodes), tris, o, d, inv, oi,
                                       st, ts, cur, have, leaf_round, &waiting);
         if (!have && st.sp == 0) {
-          a.hits[ray] = make_uint4(QUERY ? hit_id<true>(a, ts.best) : ts.best, f2u(ts.best_t),
-                                   f2u(ts.bu), f2u(ts.bv));
-          if (COUNT) {
+          if constexpr (QUERY && COUNT) {
+            // what k_records makes the record of, at its start
+            words4* out = reinterpret_cast<words4*>(a.records + 16 * (size_t)ray);
+            out[0] = words4{ts.best, f2u(ts.best_t), f2u(ts.bu), f2u(ts.bv)};
+            out[1] = words4{ts.na, ts.nt, 0u, 0u};
+          } else {
+            a.hits[ray] = make_uint4(QUERY ? hit_id<true>(a, ts.best) : ts.best, f2u(ts.best_t),
+                                     f2u(ts.bu), f2u(ts.bv));
+          }
+          if (COUNT && !QUERY) {
             na += ts.na;
             nt += ts.nt;
           }
@@ -1028,7 +1031,7 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
       }
     }
   }
-  if (COUNT) {
+  if (COUNT && !QUERY) {
     for (int off = 32; off > 0; off >>= 1) {
       na += __shfl_down(na, off);
       nt += __shfl_down(nt, off);
@@ -1046,12 +1049,33 @@ __global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
   extend_refill<COUNT, S, PACKED, MULTI, QUERY, W, false>(a, lds_waves);
 }
 
-// Hits-only queries of few rays per lane of the launch, dealt out to its
-// waves.
-template <int S, bool PACKED, int W>
+// Queries of few rays per lane of the launch, dealt out to its waves.
+// COUNT: full records, else hits only.
+template <bool COUNT, int S, bool PACKED, int W>
 __global__ __launch_bounds__(256) void k_query_dealt(ExtendArgs a) {
   extern __shared__ uint2 lds_waves[];
-  extend_refill<false, S, PACKED, false, true, W, true>(a, lds_waves);
+  extend_refill<COUNT, S, PACKED, false, true, W, true>(a, lds_waves);
+}
+
+// The full records of a query from what its traversal left at their starts:
+// the deferred MIntersection fields (triangle.rs:129-142, scene.rs:221-228),
+// and the hits when asked for.  A pass of its own, bound by its 88 B in and
+// 64 B out per ray: in the traversal the few lanes that finish in a step
+// would run it for the whole wave.
+__global__ __launch_bounds__(256) void k_records(IntersectArgs a) {
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.n; i += gridDim.x * 256) {
+    words4* out = reinterpret_cast<words4*>(a.isects + 16 * (size_t)i);
+    const words4 h = out[0], c = out[1];
+    const float* r = a.rays + 6 * (size_t)i;
+    TravState ts;
+    ts.best = h.x;
+    ts.best_t = u2f(h.y);
+    ts.bu = u2f(h.z);
+    ts.bv = u2f(h.w);
+    ts.na = c.x;
+    ts.nt = c.y;
+    write_record(a, i, mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), ts);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1699,25 +1723,18 @@ __global__ __launch_bounds__(64) void k_ref_patch(RefPatchArgs a) {
 
 #define CVK_STACK_VARIANTS(X) X(8) X(16) X(24) X(32)
 
-template <bool COUNT, int S>
-static hipError_t launch_intersect_s(const IntersectArgs& a, bool packed, uint32_t blocks,
-                                     hipStream_t s) {
-  if (packed)
-    hipLaunchKernelGGL((k_intersect<COUNT, S, true>), dim3(blocks), dim3(64), 0, s, a);
+hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, uint32_t blocks,
+                            hipStream_t s) {
+  constexpr int S = kIsectStack;
+  if (count && packed)
+    hipLaunchKernelGGL((k_intersect<true, S, true>), dim3(blocks), dim3(64), 0, s, a);
+  else if (count)
+    hipLaunchKernelGGL((k_intersect<true, S, false>), dim3(blocks), dim3(64), 0, s, a);
+  else if (packed)
+    hipLaunchKernelGGL((k_intersect<false, S, true>), dim3(blocks), dim3(64), 0, s, a);
   else
-    hipLaunchKernelGGL((k_intersect<COUNT, S, false>), dim3(blocks), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((k_intersect<false, S, false>), dim3(blocks), dim3(64), 0, s, a);
   return hipGetLastError();
-}
-
-hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, int stack,
-                            uint32_t blocks, hipStream_t s) {
-#define CASE(S)                                                                \
-  if (stack == S)                                                              \
-    return count ? launch_intersect_s<true, S>(a, packed, blocks, s)           \
-                 : launch_intersect_s<false, S>(a, packed, blocks, s);
-  CVK_STACK_VARIANTS(CASE)
-#undef CASE
-  return hipErrorInvalidValue;
 }
 
 // Wide trees (4 or 8 children): lane refill only (whole-batch requests run
@@ -1733,7 +1750,7 @@ static hipError_t launch_extend_wide(const ExtendArgs& a, bool multi, uint32_t b
   if (multi)
     hipLaunchKernelGGL((k_extend_refill<COUNT, S, true, true, false, W>), grid, block, shmem, s, b);
   else if (b.rays6 && !COUNT && b.deal)
-    hipLaunchKernelGGL((k_query_dealt<S, true, W>), grid, block, shmem, s, b);
+    hipLaunchKernelGGL((k_query_dealt<false, S, true, W>), grid, block, shmem, s, b);
   else if (b.rays6 && !COUNT)
     hipLaunchKernelGGL((k_extend_refill<false, S, true, false, true, W>), grid, block, shmem, s,
                        b);
@@ -1760,9 +1777,9 @@ static hipError_t launch_extend_s(const ExtendArgs& a, bool packed, bool multi, 
     // batched queries: the caller's rays and source ids, compiled apart so
     // that the render instantiations carry neither
     if (a.deal && packed)
-      hipLaunchKernelGGL((k_query_dealt<S, true, 2>), grid, block, shmem, s, a);
+      hipLaunchKernelGGL((k_query_dealt<false, S, true, 2>), grid, block, shmem, s, a);
     else if (a.deal)
-      hipLaunchKernelGGL((k_query_dealt<S, false, 2>), grid, block, shmem, s, a);
+      hipLaunchKernelGGL((k_query_dealt<false, S, false, 2>), grid, block, shmem, s, a);
     else if (packed)
       hipLaunchKernelGGL((k_extend_refill<false, S, true, false, true>), grid, block, shmem, s, a);
     else
@@ -1781,6 +1798,34 @@ static hipError_t launch_extend_s(const ExtendArgs& a, bool packed, bool multi, 
   return hipGetLastError();
 }
 
+template <int S>
+static hipError_t launch_records_s(const ExtendArgs& a, const IntersectArgs& r, bool packed,
+                                   uint32_t blocks, uint32_t block_waves, hipStream_t s) {
+  const uint32_t bw = block_waves == 2 || block_waves == 4 ? block_waves : 1u;
+  const dim3 grid((blocks + bw - 1) / bw), block(64 * bw);
+  const size_t shmem = (size_t)S * 64 * sizeof(uint2) * bw;
+  if (a.deal && packed)
+    hipLaunchKernelGGL((k_query_dealt<true, S, true, 2>), grid, block, shmem, s, a);
+  else if (a.deal)
+    hipLaunchKernelGGL((k_query_dealt<true, S, false, 2>), grid, block, shmem, s, a);
+  else if (packed)
+    hipLaunchKernelGGL((k_extend_refill<true, S, true, false, true>), grid, block, shmem, s, a);
+  else
+    hipLaunchKernelGGL((k_extend_refill<true, S, false, false, true>), grid, block, shmem, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_records, dim3(r.n < (1u << 20) ? (r.n + 255) / 256 : 4096u), dim3(256), 0, s,
+                     r);
+  return hipGetLastError();
+}
+hipError_t launch_records(const ExtendArgs& a, const IntersectArgs& r, bool packed, int stack,
+                          uint32_t blocks, uint32_t block_waves, hipStream_t s) {
+#define CASE(S) \
+  if (stack == S) return launch_records_s<S>(a, r, packed, blocks, block_waves, s);
+  CVK_STACK_VARIANTS(CASE)
+#undef CASE
+  return hipErrorInvalidValue;
+}
 hipError_t launch_extend(const ExtendArgs& a, bool count, bool packed, bool multi, int stack,
                          uint32_t blocks, uint32_t block_waves, hipStream_t s, uint32_t width) {
   if (multi && !a.refill) return hipErrorInvalidValue;

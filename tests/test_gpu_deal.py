@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from convector_amd import scenes
+from test_gpu_traversal import _check_exact
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +47,24 @@ def test_dealt_frames_equal_oracle(cv, oracle, w, h):
     r.accumulate_frames_f32(hdr, 1, 1)
     ohdr, _ = o.accumulate_frames(w, h, 1, 1, oracle.RNG_PIXEL, 4)
     assert hdr.tobytes() == ohdr.tobytes()
+
+
+@pytest.mark.parametrize("waves_per_cu", [1, 32])
+@pytest.mark.parametrize("tuning", [{}, {"refill_threshold": 65, "queue_parts": 1},
+                                    {"bvh_width": 4, "block_waves": 4}])
+def test_records_equal_oracle(cv, oracle, tuning, waves_per_cu):
+    """Full records, dealt out and through the cursors, under tunings of the
+    hits-only query: every field the oracle's, the counters of the
+    reference's tree whatever width the hits are traversed with."""
+    sd = scenes.config0(subdivisions=2)
+    g = cv.Scene.from_scene_data(sd)
+    o = oracle.Scene.from_scene_data(sd)
+    g.set_tuning(extend_waves_per_cu=waves_per_cu, **tuning)
+    rays = scenes.rays_inward(4 * LANES + 65, 9, radius=0.9, target_scale=0.6)
+    ref = o.intersect(rays, isect=True)
+    for n in (1, 63, 65, LANES + 1, 4 * LANES, 4 * LANES + 65):
+        print("%d rays, %d waves per CU, %r" % (n, waves_per_cu, tuning), flush=True)
+        hits, rec = g.intersect_nearest(rays[:n], full=True)
+        assert (hits["tri_id"] == rec["tri_id"]).all()
+        _check_exact(hits, rec, {k: v[:n] for k, v in ref.items()})
+        assert (rec["reserved"] == 0).all()
