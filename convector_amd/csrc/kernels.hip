@@ -8,6 +8,8 @@
 // is persistent: its waves take rays from a device cursor, so no host round
 // trip is needed between launches.  A step renders one frame of every job
 // in a device job table; the paths of all jobs share the queues.
+#include <type_traits>
+
 #include "device_math.hpp"
 #include "internal.hpp"
 
@@ -84,12 +86,15 @@ __device__ __forceinline__ float entry_tmin(entry_t e) { return u2f((uint32_t)(e
 template <int S, bool PACKED>
 struct Stack {
   lds_u64* lds;
-  glb_u64* spill;
-  uint32_t stride;
+  glb_u64* spill;   // wave-uniform; this lane's entries from `lane` on
+  uint32_t stride, lane;
   int sp;
   entry_t top;
-  __device__ __forceinline__ Stack(uint2* l, uint2* g, uint32_t str, int p)
-      : lds((lds_u64*)l), spill((glb_u64*)g), stride(str), sp(p), top(0) {}
+  __device__ __forceinline__ Stack(uint2* l, uint2* g, uint32_t gtid, uint32_t str, int p)
+      : lds((lds_u64*)l), spill((glb_u64*)g), stride(str), lane(gtid), sp(p), top(0) {}
+  __device__ __forceinline__ glb_u64* deep(int k) const {
+    return spill + ((size_t)(k - S) * stride + lane);
+  }
   // Pushes e when p is set.  The previous top goes to slot sp - 1, which
   // lies above the memory part of the stack, so when p is not set (or the
   // stack is empty, slot 0) the LDS write is harmless and is done anyway.
@@ -102,7 +107,7 @@ struct Stack {
     } else if (k < S) {
       lds[k * 64] = top;
     } else if (p) {
-      spill[(size_t)(k - S) * stride] = top;
+      *deep(k) = top;
     }
     if (p) {
       top = e;
@@ -118,7 +123,7 @@ struct Stack {
     else if (k < S)
       top = lds[k * 64];
     else
-      top = spill[(size_t)(k - S) * stride];
+      top = *deep(k);
     return e;
   }
 };
@@ -128,38 +133,46 @@ struct Stack {
 // iteration pops the last push.  Here the last push stays in registers as
 // `cur` (have = true) and only the other child goes to the stack, which
 // visits the nodes in exactly the reference's order.
-template <int S, bool PACKED>
+// EXACT: some lane's slab distances can be NaN.
+template <bool EXACT, int S, bool PACKED>
 __device__ __forceinline__ void visit_pair(const DevNode* __restrict__ nodes, uint32_t base, V3 o,
-                                           V3 inv, bool exact, Stack<S, PACKED>& st,
-                                           entry_t& cur, bool& have) {
+                                           V3 inv, Stack<S, PACKED>& st, entry_t& cur,
+                                           bool& have) {
   const float4* p = reinterpret_cast<const float4*>(nodes + base);
   float4 a0 = p[0], b0 = p[1], a1 = p[2], b1 = p[3];
   float tmin0, tmax0, tmin1, tmax1;
-  slab_hw(a0, b0, o, inv, tmin0, tmax0);
-  slab_hw(a1, b1, o, inv, tmin1, tmax1);
-  // Zero results are where the signs of the hardware min / max may differ
-  // from minps / maxps; the sign of tmax decides the hit and the signs of two
-  // zero tmins decide the order (tmax0 == 0 | tmax1 == 0 | (tmin0 == 0 &
-  // tmin1 == 0), as one min3).  Those, and waves with a lane whose slab
-  // distances can be NaN (wave-uniform `exact`), redo the x86 chains.
-  const float z = fminf(fminf(fabsf(tmax0), fabsf(tmax1)), fmaxf(fabsf(tmin0), fabsf(tmin1)));
-  if (__builtin_expect(exact || z == 0.0f, 0)) {
-    if (exact) {
-      slab<true>(a0, b0, o, inv, tmin0, tmax0);
-      slab<true>(a1, b1, o, inv, tmin1, tmax1);
-    } else {
+  bool swap, h0, h1;
+  if (EXACT) {
+    slab<true>(a0, b0, o, inv, tmin0, tmax0);
+    slab<true>(a1, b1, o, inv, tmin1, tmax1);
+    // any_masked: mask (tmax NLT tmin) and tmax's sign bit 0 (aabb.rs:155-158)
+    h0 = !(tmax0 < tmin0) && sgn(tmax0) == 0;
+    h1 = !(tmax1 < tmin1) && sgn(tmax1) == 0;
+    // sign bit of tmin0 - tmin1 as x86 computes it: inf - inf (and NaN
+    // inputs) give the negative default NaN
+    swap = sgn_x86_sub(tmin0, tmin1) != 0;
+  } else {
+    slab_hw(a0, b0, o, inv, tmin0, tmax0);
+    slab_hw(a1, b1, o, inv, tmin1, tmax1);
+    // Zero results are where the signs of the hardware min / max may differ
+    // from minps / maxps; the sign of tmax decides the hit and the signs of
+    // two zero tmins decide the order (tmax0 == 0 | tmax1 == 0 | (tmin0 == 0 &
+    // tmin1 == 0), as one min3).  Those redo the x86 chains.
+    const float z = fminf(fminf(fabsf(tmax0), fabsf(tmax1)), fmaxf(fabsf(tmin0), fabsf(tmin1)));
+    if (__builtin_expect(z == 0.0f, 0)) {
       slab<false>(a0, b0, o, inv, tmin0, tmax0);
       slab<false>(a1, b1, o, inv, tmin1, tmax1);
+      // a negative zero tmax is a miss
+      tmax0 = f2u(tmax0) == 0x80000000u ? -1.0f : tmax0;
+      tmax1 = f2u(tmax1) == 0x80000000u ? -1.0f : tmax1;
     }
+    // the sign bit above, without NaN inputs: the class mask is NaN, -inf,
+    // -normal, -denormal, -0
+    swap = __builtin_amdgcn_classf(tmin0 - tmin1, 0x3f);
+    // the hit test above, for a tmax that is not -0
+    h0 = fmaxf(tmin0, 0.0f) <= tmax0;
+    h1 = fmaxf(tmin1, 0.0f) <= tmax1;
   }
-  // sign bit of tmin0 - tmin1 as x86 computes it: inf - inf (and NaN inputs)
-  // give the negative default NaN.  Without NaN inputs the class test (mask
-  // 0x3f: NaN, -inf, -normal, -denormal, -0) is that sign bit.
-  const bool swap = exact ? sgn_x86_sub(tmin0, tmin1) != 0
-                          : __builtin_amdgcn_classf(tmin0 - tmin1, 0x3f);
-  // any_masked: mask (tmax NLT tmin) and tmax's sign bit 0 (aabb.rs:155-158)
-  const bool h0 = !(tmax0 < tmin0) && sgn(tmax0) == 0;
-  const bool h1 = !(tmax1 < tmin1) && sgn(tmax1) == 0;
   uint32_t x0, x1;
   if (PACKED) {
     x0 = f2u(b0.z) | (f2u(b0.w) << 27);
@@ -204,35 +217,12 @@ __device__ __forceinline__ void test_tri(const DevTri* __restrict__ tris, uint32
   }
 }
 
-// One iteration of the traversal loop (bvh.rs:597-651): take the next
-// entry (the one kept in registers, else the top of the stack), skip it when
-// it is further away than the best hit (is_further_away_than,
-// aabb.rs:161-170), then visit an inner node's children or test a leaf's
-// triangles.  The ray is finished when have == false and the stack is empty.
-// The root is the entry (index 0, len 0, tmin -inf), so that its pair is
-// visited first and counted like every other pair.
-//
-// With `waiting` (lane refill), a lane that reaches a leaf outside a leaf
-// round keeps the leaf's entry and waits (*waiting); it does nothing until
-// the wave's next leaf round, when it takes the same entry again (the same
-// cull test, the same best hit) and tests the triangles.  Each lane thus
-// performs the same operations in the same order, only at later steps, while
-// the wave runs its triangle tests for many lanes at once instead of for the
-// few that reach a leaf in any one step.
-template <bool COUNT, int S, bool PACKED>
-__device__ __forceinline__ void trav_step(const DevNode* __restrict__ nodes,
-                                          const DevTri* __restrict__ tris, V3 o, V3 d, V3 inv,
-                                          bool exact, Stack<S, PACKED>& st, TravState& ts,
-                                          entry_t& cur, bool& have, bool leaf_round = true,
-                                          bool* waiting = nullptr) {
-  if (waiting && *waiting && !leaf_round) return;
-  entry_t e = cur;
-  if (!have) e = st.pop();
-  have = false;
-  if (waiting) *waiting = false;
-  if (!(entry_tmin(e) < ts.best_t)) return;
+// An entry's node: children at idx, idx + 1 (len 0) or triangles
+// [idx, idx + len).
+template <bool PACKED>
+__device__ __forceinline__ void entry_leaf(const DevNode* __restrict__ nodes, entry_t e,
+                                           uint32_t& idx, uint32_t& len) {
   const uint32_t x = entry_x(e);
-  uint32_t idx, len;
   if (PACKED) {
     idx = x & 0x07ffffffu;
     len = x >> 27;
@@ -244,21 +234,54 @@ __device__ __forceinline__ void trav_step(const DevNode* __restrict__ nodes,
     idx = f2u(nb.z);
     len = f2u(nb.w);
   }
+}
+
+template <bool COUNT>
+__device__ __forceinline__ void test_leaf(const DevTri* __restrict__ tris, uint32_t idx,
+                                          uint32_t len, V3 o, V3 d, TravState& ts) {
+  for (uint32_t k = idx; k < idx + len; k++) {
+    test_tri(tris, k, o, d, ts);
+    if (COUNT) ts.nt++;
+  }
+}
+
+// One iteration of the traversal loop (bvh.rs:597-651): take the next
+// entry (the one kept in registers, else the top of the stack), skip it when
+// it is further away than the best hit (is_further_away_than,
+// aabb.rs:161-170), then visit an inner node's children or test a leaf's
+// triangles.  The ray is finished when have == false and the stack is empty.
+// The root is the entry (index 0, len 0, tmin -inf), so that its pair is
+// visited first and counted like every other pair.
+//
+// With LEAVES == false (lane refill) a lane that reaches a leaf keeps the
+// leaf's entry and waits (returns true) for the wave's next leaf round, which
+// tests the triangles of all waiting lanes (test_leaf).  Its best hit cannot
+// change in between, so each lane performs the same operations in the same
+// order, only at later steps, while the wave runs its triangle tests for many
+// lanes at once instead of for the few that reach a leaf in any one step.
+template <bool COUNT, bool EXACT, bool LEAVES, int S, bool PACKED>
+__device__ __forceinline__ bool trav_step(const DevNode* __restrict__ nodes,
+                                          const DevTri* __restrict__ tris, V3 o, V3 d, V3 inv,
+                                          Stack<S, PACKED>& st, TravState& ts, entry_t& cur,
+                                          bool& have) {
+  entry_t e = cur;
+  if (!have) e = st.pop();
+  have = false;
+  if (!(entry_tmin(e) < ts.best_t)) return false;
+  uint32_t idx, len;
+  entry_leaf<PACKED>(nodes, e, idx, len);
   if (len == 0) {
     if (COUNT) ts.na += 2;
-    visit_pair(nodes, idx, o, inv, exact, st, cur, have);
-  } else {
-    if (waiting && !leaf_round) {
-      cur = e;
-      have = true;
-      *waiting = true;
-      return;
-    }
-    for (uint32_t k = idx; k < idx + len; k++) {
-      test_tri(tris, k, o, d, ts);
-      if (COUNT) ts.nt++;
-    }
+    visit_pair<EXACT>(nodes, idx, o, inv, st, cur, have);
+    return false;
   }
+  if (!LEAVES) {
+    cur = e;
+    have = true;
+    return true;
+  }
+  test_leaf<COUNT>(tris, idx, len, o, d, ts);
+  return false;
 }
 
 template <bool PACKED>
@@ -278,8 +301,8 @@ __device__ __forceinline__ bool needs_exact_nan(V3 o, V3 inv) {
 template <bool COUNT, int S, bool PACKED>
 __device__ __forceinline__ TravState traverse(const DevNode* __restrict__ nodes,
                                               const DevTri* __restrict__ tris, V3 o, V3 d,
-                                              uint2* lds, uint2* spill, uint32_t stride,
-                                              bool valid) {
+                                              uint2* lds, uint2* spill, uint32_t gtid,
+                                              uint32_t stride, bool valid) {
   TravState ts;
   ts.best_t = 1.0e5f;
   ts.best = kNoHit;
@@ -287,13 +310,18 @@ __device__ __forceinline__ TravState traverse(const DevNode* __restrict__ nodes,
   ts.na = 0;
   ts.nt = 0;
   V3 inv = mk3(rcp(d.x), rcp(d.y), rcp(d.z));
-  Stack<S, PACKED> st(lds, spill, stride, 0);
+  Stack<S, PACKED> st(lds, spill, gtid, stride, 0);
   const bool exact = needs_exact_nan(o, inv);
   if (!valid) return ts;
   entry_t cur = root_entry<PACKED>();
   bool have = true;
-  const bool wave_exact = __any(exact);
-  while (have || st.sp > 0) trav_step<COUNT>(nodes, tris, o, d, inv, wave_exact, st, ts, cur, have);
+  if (__any(exact)) {
+    while (have || st.sp > 0)
+      trav_step<COUNT, true, true>(nodes, tris, o, d, inv, st, ts, cur, have);
+  } else {
+    while (have || st.sp > 0)
+      trav_step<COUNT, false, true>(nodes, tris, o, d, inv, st, ts, cur, have);
+  }
   return ts;
 }
 
@@ -392,7 +420,7 @@ __global__ __launch_bounds__(64) void k_intersect(IntersectArgs a) {
       d = mk3(r[3], r[4], r[5]);
     }
     TravState ts = traverse<COUNT, S, PACKED>(a.nodes, a.tris, o, d, lds + lane,
-                                              a.spill + gtid, stride, valid);
+                                              a.spill, gtid, stride, valid);
     if (!valid) continue;
     write_record(a, i, o, d, ts);
   }
@@ -638,7 +666,7 @@ __global__ __launch_bounds__(64) void k_extend(ExtendArgs a) {
     V3 o = mk3(0, 0, 0), d = mk3(1, 0, 0);
     if (valid) load_ray(a, i, o, d);
     TravState ts = traverse<COUNT, S, PACKED>(a.nodes, a.tris, o, d, lds + lane,
-                                              a.spill + gtid, stride, valid);
+                                              a.spill, gtid, stride, valid);
     if (valid) {
       a.hits[i] = make_uint4(hit_id(a, ts.best), f2u(ts.best_t), f2u(ts.bu), f2u(ts.bv));
       if (COUNT) {
@@ -708,20 +736,16 @@ __device__ __forceinline__ void wide_cas(float& ka, uint32_t& ra, float& kb, uin
 
 // One iteration of the wide traversal: take the next entry, cull it against
 // the best hit, then test an inner node's W child boxes and keep the nearest
-// hit child in registers while the others are pushed farthest first, or
-// test a leaf's triangles (waiting for the wave's leaf round as trav_step).
+// hit child in registers while the others are pushed farthest first; at a
+// leaf, wait for the wave's leaf round (true) as trav_step.
 template <bool COUNT, int S, int W>
-__device__ __forceinline__ void trav_step_wide(const float4* __restrict__ wn,
-                                               const DevTri* __restrict__ tris, V3 o, V3 d,
-                                               V3 inv, V3 oi, Stack<S, true>& st, TravState& ts,
-                                               entry_t& cur, bool& have, bool leaf_round,
-                                               bool* waiting) {
-  if (waiting && *waiting && !leaf_round) return;
+__device__ __forceinline__ bool trav_step_wide(const float4* __restrict__ wn, V3 o, V3 inv, V3 oi,
+                                               Stack<S, true>& st, TravState& ts, entry_t& cur,
+                                               bool& have) {
   entry_t e = cur;
   if (!have) e = st.pop();
   have = false;
-  if (waiting) *waiting = false;
-  if (!(entry_tmin(e) < ts.best_t)) return;
+  if (!(entry_tmin(e) < ts.best_t)) return false;
   const uint32_t x = entry_x(e);
   if (!(x & kWideLeaf)) {
     const float4* p = wn + (size_t)x * Wide<W>::kFloat4;
@@ -772,19 +796,11 @@ __device__ __forceinline__ void trav_step_wide(const float4* __restrict__ wn,
     cur = pack_entry(ref[0], key[0]);
 #pragma unroll
     for (int j = W - 1; j >= 1; j--) st.push_if((uint32_t)j < nhit, pack_entry(ref[j], key[j]));
-  } else {
-    if (waiting && !leaf_round) {
-      cur = e;
-      have = true;
-      *waiting = true;
-      return;
-    }
-    const uint32_t first = x & 0x03ffffffu, count = (x >> 26) & 31u;
-    for (uint32_t k = first; k < first + count; k++) {
-      test_tri(tris, k, o, d, ts);
-      if (COUNT) ts.nt++;
-    }
+    return false;
   }
+  cur = e;
+  have = true;
+  return true;
 }
 
 // A short queue dealt out beforehand: the rays one wave takes, with no cursor.
@@ -850,7 +866,6 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
   const uint32_t n = QUERY ? a.n : a.ctrl->count[a.bounce];
   if (!QUERY && blockIdx.x == 0 && threadIdx.x == 0)
     atomicAdd(&a.ctrl->total_rays, (unsigned long long)n);
-  const uint64_t lt = (1ull << lane) - 1ull;
   // Queue partitions (parts == kParts): the queue is cut into chunks of
   // 2^glog rays, chunk c belonging to partition c % parts.  A wave takes
   // rays from the partition of its XCD first, so that the rays in flight on
@@ -887,7 +902,7 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
   if (parts > 1)
     part = __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & (parts - 1);  // HW_REG_XCC_ID
   uint32_t visited = 0;
-  Stack<S, PACKED> st(lds + lane, a.spill + gtid, stride, 0);
+  Stack<S, PACKED> st(lds + lane, a.spill, gtid, stride, 0);
   TravState ts;
   V3 o = mk3(0, 0, 0), d = mk3(1, 0, 0), inv = mk3(1, 0, 0), oi = mk3(0, 0, 0);
   const DevNode* nodes = a.nodes;
@@ -941,7 +956,8 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
         pool_end = end1;
       }
       if (!active) {
-        const uint32_t rank = __popcll(idle & lt);
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+            (uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
         const bool old = rank < from_pool;
         const uint32_t l = old ? base0 + rank : base1 + (rank - from_pool);
         if (old || l < end1) {
@@ -989,30 +1005,46 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
       if (drained && pool >= pool_end) break;
       continue;
     }
-    const bool wave_exact = __any(active && exact);
     // several traversal steps per refill check: the check's votes cost
     // about as much as a step's mask logic, and a lane that finishes early
-    // idles for at most interval - 1 steps
+    // idles for at most interval - 1 steps.  Bound by instruction issue in
+    // large launches (74 % VALU) and by the length of a step in the drain of
+    // all: a leaf round in the step that completes its quorum instead of the
+    // next one (which took every entry again), no exact-rule branches inside
+    // a step, and the hit test as one compare took the extend launches of a
+    // 16-sample 1080p step from 55.3 to 53.8 ms, 64 rays' chains 9 % less.
+    auto steps = [&](auto exact_rules) {
+      constexpr bool EXACT = decltype(exact_rules)::value;
 #pragma unroll 1
-    for (uint32_t rep = 0; rep < a.interval; rep++) {
-      // a leaf round when leaf_batch / 64 of the active lanes wait at
-      // leaves (a share, so that a wave with few rays left does not hold
-      // its leaves back), or every active lane does (so that the wave
-      // always progresses)
-      bool leaf_round = true;
-      if (a.leaf_batch) {
-        const uint64_t wm = __ballot(active && waiting), am = __ballot(active);
-        leaf_round = (uint32_t)__popcll(wm) * 64u >= a.leaf_batch * (uint32_t)__popcll(am) ||
-                     wm == am;
-      }
-      if (active) {
-        if constexpr (W == 2)
-          trav_step<COUNT>(nodes, tris, o, d, inv, wave_exact, st, ts, cur, have, leaf_round,
-                           &waiting);
-        else
-          trav_step_wide<COUNT, S, W>(reinterpret_cast<const float4*>(nodes), tris, o, d, inv, oi,
-                                      st, ts, cur, have, leaf_round, &waiting);
-        if (!have && st.sp == 0) {
+      for (uint32_t rep = 0; rep < a.interval; rep++) {
+        if (active && !waiting) {
+          if constexpr (W == 2)
+            waiting = trav_step<COUNT, EXACT, false>(nodes, tris, o, d, inv, st, ts, cur, have);
+          else
+            waiting = trav_step_wide<COUNT, S, W>(reinterpret_cast<const float4*>(nodes), o, inv,
+                                                  oi, st, ts, cur, have);
+        }
+        // a leaf round when leaf_batch / 64 of the active lanes wait at
+        // leaves (a share, so that a wave with few rays left does not hold
+        // its leaves back), or every active lane does (so that the wave
+        // always progresses)
+        const uint64_t wm = __ballot(waiting), am = __ballot(active);
+        if ((uint32_t)__popcll(wm) * 64u >= max(a.leaf_batch * (uint32_t)__popcll(am), 1u) ||
+            wm == am) {
+          if (waiting) {
+            uint32_t idx, len;
+            if constexpr (W == 2) {
+              entry_leaf<PACKED>(nodes, cur, idx, len);
+            } else {
+              idx = entry_x(cur) & 0x03ffffffu;
+              len = (entry_x(cur) >> 26) & 31u;
+            }
+            test_leaf<COUNT>(tris, idx, len, o, d, ts);
+            have = false;
+            waiting = false;
+          }
+        }
+        if (active && !have && st.sp == 0) {
           if constexpr (QUERY && COUNT) {
             // what k_records makes the record of, at its start
             words4* out = reinterpret_cast<words4*>(a.records + 16 * (size_t)ray);
@@ -1029,7 +1061,11 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
           active = false;
         }
       }
-    }
+    };
+    if (W == 2 && __any(active && exact))
+      steps(std::true_type{});
+    else
+      steps(std::false_type{});
   }
   if (COUNT && !QUERY) {
     for (int off = 32; off > 0; off >>= 1) {
@@ -1043,8 +1079,12 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
   }
 }
 
+// 8 waves per SIMD (64 VGPRs) where that takes no spills: at 68 the bunny's
+// 10^7 rays took 1.75 ms and at 64 1.72; with one scene per ray the 20 bytes
+// spilled cost 5 % (71 VGPRs, 7 waves).
 template <bool COUNT, int S, bool PACKED, bool MULTI, bool QUERY = false, int W = 2>
-__global__ __launch_bounds__(256) void k_extend_refill(ExtendArgs a) {
+__global__ __launch_bounds__(256, W == 2 && !COUNT && !MULTI && (PACKED || !QUERY) ? 8 : 1) void
+    k_extend_refill(ExtendArgs a) {
   extern __shared__ uint2 lds_waves[];
   extend_refill<COUNT, S, PACKED, MULTI, QUERY, W, false>(a, lds_waves);
 }
@@ -1650,7 +1690,7 @@ __global__ __launch_bounds__(64) void k_ref_patch(RefPatchArgs a) {
             for (uint32_t b = 0; b < a.max_bounces; b++) {
               const bool act = (active >> 31) == 0;
               TravState ts = traverse<false, S, PACKED>(J.nodes, J.tris, o, d, lds + lane,
-                                                        a.spill + gtid, stride, act);
+                                                        a.spill, gtid, stride, act);
               V3 pos, normal;
               uint32_t mat;
               float tu = 0.0f, tv = 0.0f;
