@@ -204,11 +204,19 @@ __global__ __launch_bounds__(256) void k_trefs(const float* v9, uint32_t n, floa
       lb[9 + k] = max(lb[9 + k], okey(c[k]));
     }
   }
+  // (a wave's bounds first: 256 LDS atomics per value follow each other)
   for (int k = 0; k < 12; k++) {
-    if ((k % 6) < 3)
-      atomicMin(&sbox[k], lb[k]);
-    else
-      atomicMax(&sbox[k], lb[k]);
+    uint32_t v = lb[k];
+    for (int off = 32; off > 0; off >>= 1) {
+      const uint32_t w = __shfl_xor(v, off);
+      v = (k % 6) < 3 ? min(v, w) : max(v, w);
+    }
+    if ((threadIdx.x & 63u) == 0) {
+      if ((k % 6) < 3)
+        atomicMin(&sbox[k], v);
+      else
+        atomicMax(&sbox[k], v);
+    }
   }
   __syncthreads();
   if (threadIdx.x < 6) {
@@ -1561,7 +1569,7 @@ hipError_t build_reference_bvh(const float* d_v9, uint32_t ntris, DevNode* nodes
   BVH_CHECK(hipMemcpyAsync(ctx, &init, sizeof(Ctx), hipMemcpyHostToDevice, s));
   {
     uint32_t blocks = (ntris + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
+    if (blocks > 1024) blocks = 1024;  // each ends with 12 atomics on the same 12 words
     hipLaunchKernelGGL(k_trefs, dim3(blocks), dim3(256), 0, s, d_v9, ntris, A, B, C, a.buf[0],
                        ctx);
     BVH_CHECK(hipGetLastError());
