@@ -252,6 +252,172 @@ __global__ __launch_bounds__(256) void k_conv_lds(ConvArgs a) {
 // ---------------------------------------------------------------------------
 constexpr uint32_t kHaloW = 32, kHaloH = 8;
 
+// The epilogue of a wave's 4 x NS fragments at row wrow of the tile (x0, y0):
+// lane: output channels row0 + t * 16 + 4 * kq + r (r = 0..3) of pixel col of
+// each fragment.  bias_s: the slice's bias in LDS (PERSIST).
+template <int NS, bool MASK, bool POOL, bool UG, bool PERSIST>
+__device__ __forceinline__ void conv_epilogue(const ConvArgs& a, f4 (&acc)[4][NS], int x0, int y0,
+                                              size_t img_base, int wrow, uint32_t col, uint32_t kq,
+                                              uint32_t row0, const float* bias_s) {
+  constexpr int MF = 4;
+  const bool vec_y = a.y && ((uintptr_t)a.y % 8 == 0) && (a.ycs % 4 == 0);
+  const bool vec_f = a.yf && ((uintptr_t)a.yf % 16 == 0) && (a.yfcs % 4 == 0);
+  if constexpr (POOL) {
+    // Fragments m (the upper row of the wave's pair) and m + 2 (the lower
+    // row) together: both are stored, and the even lane of each column
+    // pair, which holds pixel (2Y, 2X), takes its neighbour (2Y, 2X + 1)
+    // by a DPP lane swap (quad_perm [1, 0, 3, 2]) and writes the 2 x 2
+    // average of the stored bf16 values, summed in the order of k_pool.
+    // (The host checks: y aligned for 8-byte stores, whole groups of 4.)
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+      const int py = y0 + wrow;
+      if (py >= (int)a.h) continue;
+      const uint32_t px = (uint32_t)x0 + 16 * m + col;
+      const size_t p = img_base + (size_t)py * a.w_ + px;
+      const size_t q = img_base / 4 + (size_t)(py >> 1) * (a.w_ >> 1) + (px >> 1);
+#pragma unroll
+      for (int t = 0; t < NS; t++) {
+        const uint32_t j0 = row0 + t * 16 + 4 * kq;
+        if (j0 >= a.nout) continue;
+        float u[4], l[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float b = PERSIST ? bias_s[t * 16 + 4 * kq + r]
+                                  : (a.bias ? a.bias[j0 + r] : 0.0f);
+          u[r] = acc[m][t][r] + b;
+          l[r] = acc[m + 2][t][r] + b;
+          if (a.relu) {
+            u[r] = fmaxf(u[r], 0.0f);
+            l[r] = fmaxf(l[r], 0.0f);
+          }
+        }
+        const uint2 pu = make_uint2(pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]));
+        const uint2 pl = make_uint2(pack_bf16x2(l[0], l[1]), pack_bf16x2(l[2], l[3]));
+        *reinterpret_cast<uint2*>(a.y + p * a.ycs + j0) = pu;
+        *reinterpret_cast<uint2*>(a.y + (p + a.w_) * a.ycs + j0) = pl;
+        const uint32_t wu[4] = {pu.x << 16, pu.x & 0xffff0000u, pu.y << 16, pu.y & 0xffff0000u};
+        const uint32_t wl[4] = {pl.x << 16, pl.x & 0xffff0000u, pl.y << 16, pl.y & 0xffff0000u};
+        float s4[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float a0 = __uint_as_float(wu[r]), c0 = __uint_as_float(wl[r]);
+          const float b0 = __int_as_float(
+              __builtin_amdgcn_mov_dpp((int)wu[r], 0xB1, 0xF, 0xF, false));
+          const float d0 = __int_as_float(
+              __builtin_amdgcn_mov_dpp((int)wl[r], 0xB1, 0xF, 0xF, false));
+          s4[r] = 0.25f * (((a0 + b0) + c0) + d0);
+        }
+        if ((col & 1) == 0)
+          *reinterpret_cast<uint2*>(a.pool + q * a.poolcs + j0) =
+              make_uint2(pack_bf16x2(s4[0], s4[1]), pack_bf16x2(s4[2], s4[3]));
+      }
+    }
+  } else if (UG && row0 < a.ug_ch) {
+    // the upsampling's gradient: the 2 x 2 sum of the f32 values (the
+    // even lane of each column pair reads its neighbour by DPP, as in
+    // the pooling above), masked by the layer below's ReLU output
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+      const int py = y0 + wrow;
+      if (py >= (int)a.h) continue;
+      const uint32_t px = (uint32_t)x0 + 16 * m + col;
+      const size_t q = img_base / 4 + (size_t)(py >> 1) * (a.w_ >> 1) + (px >> 1);
+#pragma unroll
+      for (int t = 0; t < NS; t++) {
+        const uint32_t j0 = row0 + t * 16 + 4 * kq;
+        float sv[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float u = acc[m][t][r], l = acc[m + 2][t][r];
+          const float un = __int_as_float(
+              __builtin_amdgcn_mov_dpp(__float_as_int(u), 0xB1, 0xF, 0xF, false));
+          const float ln = __int_as_float(
+              __builtin_amdgcn_mov_dpp(__float_as_int(l), 0xB1, 0xF, 0xF, false));
+          sv[r] = ((u + un) + l) + ln;
+        }
+        if ((col & 1) == 0) {
+          const uint2 mk = *reinterpret_cast<const uint2*>(a.ug_mask + q * a.ug_mcs + j0);
+          const uint32_t mw[4] = {mk.x << 16, mk.x & 0xffff0000u, mk.y << 16,
+                                  mk.y & 0xffff0000u};
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            if (!(__uint_as_float(mw[r]) > 0.0f)) sv[r] = 0.0f;
+          *reinterpret_cast<uint2*>(a.ug_dz + q * a.ug_dzcs + j0) =
+              make_uint2(pack_bf16x2(sv[0], sv[1]), pack_bf16x2(sv[2], sv[3]));
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < MF; m++) {
+      const int py = y0 + wrow + m / 2;
+      if (py >= (int)a.h) continue;
+      const size_t p = img_base + (size_t)py * a.w_ + (uint32_t)x0 + 16 * (m % 2) + col;
+#pragma unroll
+      for (int t = 0; t < NS; t++) {
+        const uint32_t j0 = row0 + t * 16 + 4 * kq;
+        if (j0 >= a.nout) continue;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const uint32_t j = j0 + r;
+          if constexpr (PERSIST)
+            v[r] = acc[m][t][r] + bias_s[j - row0];
+          else
+            v[r] = acc[m][t][r] + ((a.bias && j < a.nout) ? a.bias[j] : 0.0f);
+          if (a.relu) v[r] = fmaxf(v[r], 0.0f);
+        }
+        const bool whole = j0 + 4 <= a.nout;
+        if constexpr (MASK) {
+          // the ReLU gradient of the layer below: 4 bf16 of its output at once
+          // (the host checks the mask's alignment and stride)
+          if (whole) {
+            const uint2 mk = *reinterpret_cast<const uint2*>(a.mask + p * a.mcs + j0);
+            const uint32_t mw[4] = {mk.x << 16, mk.x & 0xffff0000u, mk.y << 16,
+                                    mk.y & 0xffff0000u};
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              if (!(__uint_as_float(mw[r]) > 0.0f)) v[r] = 0.0f;
+          } else {
+            for (int r = 0; r < 4; r++)
+              if (j0 + r < a.nout && !(from_bf16(a.mask[p * a.mcs + j0 + r]) > 0.0f))
+                v[r] = 0.0f;
+          }
+        }
+        if (a.y) {
+          if (whole && vec_y) {
+            uint2 pk;
+            pk.x = pack_bf16x2(v[0], v[1]);
+            pk.y = pack_bf16x2(v[2], v[3]);
+            *reinterpret_cast<uint2*>(a.y + p * a.ycs + j0) = pk;
+          } else {
+            for (int r = 0; r < 4; r++)
+              if (j0 + r < a.nout) a.y[p * a.ycs + j0 + r] = to_bf16(v[r]);
+          }
+        }
+        if (a.yf) {
+          float* o = a.yf + p * a.yfcs + j0;
+          if (whole && vec_f) {
+            float4 w4 = make_float4(v[0], v[1], v[2], v[3]);
+            if (a.accumulate) {
+              const float4 old = *reinterpret_cast<const float4*>(o);
+              w4.x += old.x;
+              w4.y += old.y;
+              w4.z += old.z;
+              w4.w += old.w;
+            }
+            *reinterpret_cast<float4*>(o) = w4;
+          } else {
+            for (int r = 0; r < 4; r++)
+              if (j0 + r < a.nout) o[r] = a.accumulate ? o[r] + v[r] : v[r];
+          }
+        }
+      }
+    }
+  }
+}
+
 template <int KC, int NS, bool FLIP, bool MASK = false, bool UP = false, bool POOL = false,
           bool UG = false>
 __global__ __launch_bounds__(256, 2) void k_conv_halo(ConvArgs a) {
@@ -387,10 +553,6 @@ __global__ __launch_bounds__(256, 2) void k_conv_halo(ConvArgs a) {
       CV_HALO_LOAD_X();
     }
   }
-  // lane: output channels row0 + t * 16 + 4 * kq + r (r = 0..3) of pixel
-  // col of each fragment
-  const bool vec_y = a.y && ((uintptr_t)a.y % 8 == 0) && (a.ycs % 4 == 0);
-  const bool vec_f = a.yf && ((uintptr_t)a.yf % 16 == 0) && (a.yfcs % 4 == 0);
 #pragma unroll 1
   for (;;) {
     f4 acc[MF][NS];
@@ -459,160 +621,8 @@ __global__ __launch_bounds__(256, 2) void k_conv_halo(ConvArgs a) {
         CV_HALO_LOAD_X();
       }
     }
-    if constexpr (POOL) {
-      // Fragments m (the upper row of the wave's pair) and m + 2 (the lower
-      // row) together: both are stored, and the even lane of each column
-      // pair, which holds pixel (2Y, 2X), takes its neighbour (2Y, 2X + 1)
-      // by a DPP lane swap (quad_perm [1, 0, 3, 2]) and writes the 2 x 2
-      // average of the stored bf16 values, summed in the order of k_pool.
-      // (The host checks: y aligned for 8-byte stores, whole groups of 4.)
-#pragma unroll
-      for (int m = 0; m < 2; m++) {
-        const int py = y0 + wrow;
-        if (py >= (int)a.h) continue;
-        const uint32_t px = (uint32_t)x0 + 16 * m + col;
-        const size_t p = img_base + (size_t)py * a.w_ + px;
-        const size_t q = img_base / 4 + (size_t)(py >> 1) * (a.w_ >> 1) + (px >> 1);
-#pragma unroll
-        for (int t = 0; t < NS; t++) {
-          const uint32_t j0 = row0 + t * 16 + 4 * kq;
-          if (j0 >= a.nout) continue;
-          float u[4], l[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const float b = PERSIST ? bias_s[t * 16 + 4 * kq + r]
-                                    : (a.bias ? a.bias[j0 + r] : 0.0f);
-            u[r] = acc[m][t][r] + b;
-            l[r] = acc[m + 2][t][r] + b;
-            if (a.relu) {
-              u[r] = fmaxf(u[r], 0.0f);
-              l[r] = fmaxf(l[r], 0.0f);
-            }
-          }
-          const uint2 pu = make_uint2(pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]));
-          const uint2 pl = make_uint2(pack_bf16x2(l[0], l[1]), pack_bf16x2(l[2], l[3]));
-          *reinterpret_cast<uint2*>(a.y + p * a.ycs + j0) = pu;
-          *reinterpret_cast<uint2*>(a.y + (p + a.w_) * a.ycs + j0) = pl;
-          const uint32_t wu[4] = {pu.x << 16, pu.x & 0xffff0000u, pu.y << 16, pu.y & 0xffff0000u};
-          const uint32_t wl[4] = {pl.x << 16, pl.x & 0xffff0000u, pl.y << 16, pl.y & 0xffff0000u};
-          float s4[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const float a0 = __uint_as_float(wu[r]), c0 = __uint_as_float(wl[r]);
-            const float b0 = __int_as_float(
-                __builtin_amdgcn_mov_dpp((int)wu[r], 0xB1, 0xF, 0xF, false));
-            const float d0 = __int_as_float(
-                __builtin_amdgcn_mov_dpp((int)wl[r], 0xB1, 0xF, 0xF, false));
-            s4[r] = 0.25f * (((a0 + b0) + c0) + d0);
-          }
-          if ((col & 1) == 0)
-            *reinterpret_cast<uint2*>(a.pool + q * a.poolcs + j0) =
-                make_uint2(pack_bf16x2(s4[0], s4[1]), pack_bf16x2(s4[2], s4[3]));
-        }
-      }
-    } else if (UG && row0 < a.ug_ch) {
-      // the upsampling's gradient: the 2 x 2 sum of the f32 values (the
-      // even lane of each column pair reads its neighbour by DPP, as in
-      // the pooling above), masked by the layer below's ReLU output
-#pragma unroll
-      for (int m = 0; m < 2; m++) {
-        const int py = y0 + wrow;
-        if (py >= (int)a.h) continue;
-        const uint32_t px = (uint32_t)x0 + 16 * m + col;
-        const size_t q = img_base / 4 + (size_t)(py >> 1) * (a.w_ >> 1) + (px >> 1);
-#pragma unroll
-        for (int t = 0; t < NS; t++) {
-          const uint32_t j0 = row0 + t * 16 + 4 * kq;
-          float sv[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const float u = acc[m][t][r], l = acc[m + 2][t][r];
-            const float un = __int_as_float(
-                __builtin_amdgcn_mov_dpp(__float_as_int(u), 0xB1, 0xF, 0xF, false));
-            const float ln = __int_as_float(
-                __builtin_amdgcn_mov_dpp(__float_as_int(l), 0xB1, 0xF, 0xF, false));
-            sv[r] = ((u + un) + l) + ln;
-          }
-          if ((col & 1) == 0) {
-            const uint2 mk = *reinterpret_cast<const uint2*>(a.ug_mask + q * a.ug_mcs + j0);
-            const uint32_t mw[4] = {mk.x << 16, mk.x & 0xffff0000u, mk.y << 16,
-                                    mk.y & 0xffff0000u};
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-              if (!(__uint_as_float(mw[r]) > 0.0f)) sv[r] = 0.0f;
-            *reinterpret_cast<uint2*>(a.ug_dz + q * a.ug_dzcs + j0) =
-                make_uint2(pack_bf16x2(sv[0], sv[1]), pack_bf16x2(sv[2], sv[3]));
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int m = 0; m < MF; m++) {
-        const int py = y0 + wrow + m / 2;
-        if (py >= (int)a.h) continue;
-        const size_t p = img_base + (size_t)py * a.w_ + (uint32_t)x0 + 16 * (m % 2) + col;
-#pragma unroll
-        for (int t = 0; t < NS; t++) {
-          const uint32_t j0 = row0 + t * 16 + 4 * kq;
-          if (j0 >= a.nout) continue;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const uint32_t j = j0 + r;
-            if constexpr (PERSIST)
-              v[r] = acc[m][t][r] + bias_s[j - row0];
-            else
-              v[r] = acc[m][t][r] + ((a.bias && j < a.nout) ? a.bias[j] : 0.0f);
-            if (a.relu) v[r] = fmaxf(v[r], 0.0f);
-          }
-          const bool whole = j0 + 4 <= a.nout;
-          if constexpr (MASK) {
-            // the ReLU gradient of the layer below: 4 bf16 of its output at once
-            // (the host checks the mask's alignment and stride)
-            if (whole) {
-              const uint2 mk = *reinterpret_cast<const uint2*>(a.mask + p * a.mcs + j0);
-              const uint32_t mw[4] = {mk.x << 16, mk.x & 0xffff0000u, mk.y << 16,
-                                      mk.y & 0xffff0000u};
-#pragma unroll
-              for (int r = 0; r < 4; r++)
-                if (!(__uint_as_float(mw[r]) > 0.0f)) v[r] = 0.0f;
-            } else {
-              for (int r = 0; r < 4; r++)
-                if (j0 + r < a.nout && !(from_bf16(a.mask[p * a.mcs + j0 + r]) > 0.0f))
-                  v[r] = 0.0f;
-            }
-          }
-          if (a.y) {
-            if (whole && vec_y) {
-              uint2 pk;
-              pk.x = pack_bf16x2(v[0], v[1]);
-              pk.y = pack_bf16x2(v[2], v[3]);
-              *reinterpret_cast<uint2*>(a.y + p * a.ycs + j0) = pk;
-            } else {
-              for (int r = 0; r < 4; r++)
-                if (j0 + r < a.nout) a.y[p * a.ycs + j0 + r] = to_bf16(v[r]);
-            }
-          }
-          if (a.yf) {
-            float* o = a.yf + p * a.yfcs + j0;
-            if (whole && vec_f) {
-              float4 w4 = make_float4(v[0], v[1], v[2], v[3]);
-              if (a.accumulate) {
-                const float4 old = *reinterpret_cast<const float4*>(o);
-                w4.x += old.x;
-                w4.y += old.y;
-                w4.z += old.z;
-                w4.w += old.w;
-              }
-              *reinterpret_cast<float4*>(o) = w4;
-            } else {
-              for (int r = 0; r < 4; r++)
-                if (j0 + r < a.nout) o[r] = a.accumulate ? o[r] + v[r] : v[r];
-            }
-          }
-        }
-      }
-    }
+    conv_epilogue<NS, MASK, POOL, UG, PERSIST>(a, acc, x0, y0, img_base, wrow, col, kq, row0,
+                                               bias_s);
     if (!more) break;
     tile = next;
     x0 = nx0;
@@ -628,6 +638,152 @@ __global__ __launch_bounds__(256, 2) void k_conv_halo(ConvArgs a) {
 #undef CV_HALO_LOAD_X
 #undef CV_HALO_STORE
 #undef CV_HALO_STORE_X
+}
+
+// ---------------------------------------------------------------------------
+// The same convolution with the slice's weights of all input chunks resident
+// in LDS: one workgroup of 8 waves per CU walks the 8 x 32 tiles, waves 0-3
+// computing the lower half of the slice's 64 outputs and waves 4-7 the upper,
+// two rows each.  The chunks of a tile, and of the next tile, follow each other
+// through two input buffers: a chunk's loads are issued two chunks ahead and
+// stored one ahead, with one barrier per chunk.  Bound by the latency of a
+// chunk: k_conv_halo, whose 2 workgroups per CU read the 73 KB of a 64-channel
+// layer's weights again for every tile and drain their loads between tiles,
+// took 30.4 us for 64 -> 64 channels at 640 x 368 and 44 with the ReLU mask of
+// a training step (16 x 128 x 128), this 25.9 and 40.6; with the pooling 35.4
+// and 34.0.  (Reading every halo row once for both output rows of a wave, 22 %
+// fewer LDS reads, changed nothing: 27.2.)
+// ---------------------------------------------------------------------------
+template <int KC, bool FLIP, bool MASK = false, bool POOL = false>
+__global__ __launch_bounds__(512, 2) void k_conv_res(ConvArgs a) {
+  constexpr int NS = 2, MF = 4, WR = 64, NT = 512;
+  constexpr int HH = (int)kHaloH + 2, HW = (int)kHaloW + 2;
+  constexpr int NCH = KC / 32, RS = 40, WS = 40;
+  constexpr int XP = HH * HW * 4, XPT = (XP + NT - 1) / NT;
+  constexpr int WP = NCH * 9 * WR * 4;
+  __shared__ __attribute__((aligned(16))) uint16_t xs[2][HH * HW * RS];
+  __shared__ __attribute__((aligned(16))) uint16_t ws[NCH * 9 * WR * WS];
+  __shared__ float bias_s[WR];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t ntx = a.w_ / kHaloW, nty = (a.h + kHaloH - 1) / kHaloH;
+  const uint32_t ntiles = (a.npix / (a.h * a.w_)) * ntx * nty;
+  const uint32_t row0 = blockIdx.y * WR;
+  auto corner = [&](uint32_t t, int& tx, int& ty, size_t& base) {
+    tx = (int)((t % ntx) * kHaloW);
+    ty = (int)(((t / ntx) % nty) * kHaloH);
+    base = (size_t)(t / (ntx * nty)) * a.h * a.w_;
+  };
+  // element offset of this thread's input pieces of tile t, ~0u outside the
+  // image (loaded from the tensor's first pixel and zeroed when stored)
+  uint32_t xoff[XPT];
+  auto tile_offsets = [&](uint32_t t) {
+    int tx, ty;
+    size_t base;
+    corner(t, tx, ty, base);
+#pragma unroll
+    for (int i = 0; i < XPT; i++) {
+      const int q = (int)tid + NT * i;
+      const int pix = q >> 2, part = q & 3;
+      const int sy = ty + pix / HW - 1, sx = tx + pix % HW - 1;
+      xoff[i] = (q < XP && sy >= 0 && sy < (int)a.h && sx >= 0 && sx < (int)a.w_)
+                    ? (uint32_t)((base + (size_t)sy * a.w_ + (uint32_t)sx) * a.xcs) + part * 8
+                    : ~0u;
+    }
+  };
+  u32x4 xr[XPT];
+  auto load_x = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < XPT; i++)
+      xr[i] = *reinterpret_cast<const u32x4*>(a.x + (xoff[i] != ~0u ? xoff[i] : 0u) + c * 32);
+  };
+  auto store_x = [&](uint16_t* dst) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < XPT; i++) {
+      const int q = (int)tid + NT * i;
+      if (q < XP)
+        *reinterpret_cast<u32x4*>(&dst[(q >> 2) * RS + (q & 3) * 8]) =
+            xoff[i] != ~0u ? xr[i] : u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  // the chunk after (tile lt, chunk lc) in this workgroup's order
+  uint32_t tile = blockIdx.x, lt = tile;
+  int lc = 0;
+  auto advance = [&]() {
+    if (++lc == NCH) {
+      lc = 0;
+      lt += gridDim.x;
+      if (lt < ntiles) tile_offsets(lt);
+    }
+  };
+  tile_offsets(lt);
+  load_x(0);
+  for (int q = (int)tid; q < WP; q += NT) {
+    const int g = q & 3, r = (q >> 2) % WR, st = (q >> 2) / WR % 9, c = (q >> 2) / (WR * 9);
+    *reinterpret_cast<u32x4*>(&ws[(q >> 2) * WS + 8 * g]) = *reinterpret_cast<const u32x4*>(
+        a.w + (size_t)(row0 + (uint32_t)r) * a.kpad + st * KC + c * 32 + 8 * g);
+  }
+  if (tid < (uint32_t)WR) bias_s[tid] = (a.bias && row0 + tid < a.nout) ? a.bias[row0 + tid] : 0.0f;
+  store_x(xs[0]);
+  advance();
+  if (lt < ntiles) load_x(lc);
+  __syncthreads();
+  const uint32_t col = lane & 15, kq = lane >> 4;
+  const int wrow = 2 * (int)(wave & 3), half = (int)(wave >> 2) * NS * 16;
+  uint32_t buf = 0;
+#pragma unroll 1
+  for (; tile < ntiles; tile += gridDim.x) {
+    f4 acc[MF][NS];
+#pragma unroll
+    for (int m = 0; m < MF; m++)
+#pragma unroll
+      for (int t = 0; t < NS; t++) acc[m][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int c = 0; c < NCH; c++) {
+      const uint16_t* x = xs[buf];
+      const uint16_t* w = ws + c * 9 * WR * WS;
+#pragma unroll
+      for (int st = 0; st < 9; st++) {
+        int dy = st / 3 - 1, dx = st % 3 - 1;
+        if (FLIP) {
+          dy = -dy;
+          dx = -dx;
+        }
+        bf8 Wf[NS];
+#pragma unroll
+        for (int t = 0; t < NS; t++)
+          Wf[t] = *reinterpret_cast<const bf8*>(
+              &w[(st * WR + half + t * 16 + (int)col) * WS + 8 * kq]);
+#pragma unroll
+        for (int m = 0; m < MF; m++) {
+          const int hy = wrow + m / 2 + 1 + dy, hx = 16 * (m % 2) + (int)col + 1 + dx;
+          const bf8 X = *reinterpret_cast<const bf8*>(&x[(hy * HW + hx) * RS + 8 * (int)kq]);
+#pragma unroll
+          for (int t = 0; t < NS; t++)
+            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Wf[t], X, acc[m][t], 0, 0, 0);
+        }
+      }
+      // the next chunk into the other buffer, which the previous chunk's
+      // MFMAs have left, and the loads of the one after it
+      const bool epilogue = c + 1 == NCH;
+      int x0 = 0, y0 = 0;
+      size_t base = 0;
+      if (epilogue) corner(tile, x0, y0, base);
+      if (lt < ntiles) store_x(xs[buf ^ 1u]);
+      if (MASK && epilogue)  // (its mask loads would wait behind the next chunk's)
+        conv_epilogue<NS, MASK, POOL, false, true>(a, acc, x0, y0, base, wrow, col, kq, row0 + half,
+                                                bias_s + half);
+      if (lt < ntiles) {
+        advance();
+        if (lt < ntiles) load_x(lc);
+      }
+      if (!MASK && epilogue)
+        conv_epilogue<NS, MASK, POOL, false, true>(a, acc, x0, y0, base, wrow, col, kq, row0 + half,
+                                                bias_s + half);
+      __syncthreads();
+      buf ^= 1u;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1508,6 +1664,26 @@ bool try_halo(cv_denoiser* d, const cvd::ConvArgs& a, uint32_t nt, uint32_t ns) 
   return true;
 }
 
+// The resident-weight kernel for layers of KC input channels and whole slices
+// of 64 outputs, where a workgroup per CU gets more than one tile (below that
+// the weights it loads serve a single tile, as in k_conv_halo; the
+// upsampling's gradient with its 192 outputs, three slices that each get a
+// third of the CUs, measured 104 us against k_conv_halo's 79).
+template <int KC, bool FLIP, bool MASK = false, bool POOL = false>
+bool try_res(cv_denoiser* d, const cvd::ConvArgs& a, uint32_t nt) {
+  if (a.kc != (uint32_t)KC || nt % 4 || (a.flip != 0) != FLIP || (a.mask != nullptr) != MASK ||
+      a.xup || (a.pool != nullptr) != POOL || a.ug_dz)
+    return false;
+  const uint32_t tiles = (a.npix / (a.h * a.w_)) * (a.w_ / cvd::kHaloW) *
+                         ((a.h + cvd::kHaloH - 1) / cvd::kHaloH);
+  const uint32_t slices = nt / 4, cap = std::max(1u, cvh::num_cus() / slices);
+  if (tiles <= cap) return false;
+  const uint32_t per = (tiles + cap - 1) / cap;
+  hipLaunchKernelGGL((cvd::k_conv_res<KC, FLIP, MASK, POOL>),
+                     dim3((tiles + per - 1) / per, slices), dim3(512), 0, d->stream, a);
+  return true;
+}
+
 bool launch_conv_halo(cv_denoiser* d, const cvd::ConvArgs& a, uint32_t nt) {
   // whole 32-pixel rows, whole images, and every pixel's KC channels within
   // its stride (the tile loads read channels [0, KC) of each pixel)
@@ -1527,6 +1703,9 @@ bool launch_conv_halo(cv_denoiser* d, const cvd::ConvArgs& a, uint32_t nt) {
   if (a.xup && (a.h % 2 || a.w_ % 2 || a.xupcs % 8 || a.xupcs < 32 * a.up_chunks ||
                 32 * a.up_chunks > a.kc))
     return false;
+  if (try_res<64, false>(d, a, nt) || try_res<64, false, false, true>(d, a, nt) ||
+      try_res<64, true, true>(d, a, nt))
+    return true;
   const uint32_t ns = nt % 4 == 0 ? 4 : nt % 2 == 0 ? 2 : nt % 3 == 0 ? 3 : 1;
   return try_halo<16, 2, false>(d, a, nt, ns) || try_halo<32, 1, false>(d, a, nt, ns) ||
          try_halo<32, 2, false>(d, a, nt, ns) || try_halo<32, 4, false>(d, a, nt, ns) ||
