@@ -70,17 +70,24 @@ namespace {
 // hipMemcpy2DAsync into pageable memory, row by row; 1.0 ms this way).
 constexpr size_t kPieceBytes = 2u << 20;
 constexpr uint32_t kPieces = 8;
+constexpr int kBounceDevices = 64;
 std::mutex g_bounce_mu;
 char* g_bounce = nullptr;
-hipEvent_t g_piece_done[kPieces] = {};
+// per device (an event is recorded on streams of its own device only)
+hipEvent_t g_piece_done[kBounceDevices][kPieces] = {};
 
-cv_status bounce_init() {
+// The current device's events, with the bounce buffer allocated; g_bounce_mu
+// held.
+cv_status bounce_init(hipEvent_t** done) {
+  int dev = 0;
+  HIPTRY(hipGetDevice(&dev), "hipGetDevice");
+  if (dev < 0 || dev >= kBounceDevices) return fail(CV_ERR_INVALID_ARGUMENT, "device index");
   if (!g_bounce)
-    HIPTRY(hipHostMalloc((void**)&g_bounce, kPieceBytes * kPieces, hipHostMallocDefault),
+    HIPTRY(hipHostMalloc((void**)&g_bounce, kPieceBytes * kPieces, hipHostMallocPortable),
            "pinned alloc");
-  for (uint32_t k = 0; k < kPieces; k++)
-    if (!g_piece_done[k])
-      HIPTRY(hipEventCreateWithFlags(&g_piece_done[k], hipEventDisableTiming), "event");
+  for (hipEvent_t& e : g_piece_done[dev])
+    if (!e) HIPTRY(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
+  *done = g_piece_done[dev];
   return CV_OK;
 }
 
@@ -120,7 +127,8 @@ cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, h
   }
   if (ps.empty()) return CV_OK;
   std::lock_guard<std::mutex> lk(g_bounce_mu);
-  cv_status cs = bounce_init();
+  hipEvent_t* piece_done = nullptr;
+  cv_status cs = bounce_init(&piece_done);
   if (cs != CV_OK) return cs;
   auto host_of = [](const Piece& p) { return (char*)p.rc->host + p.row * p.rc->host_pitch + p.col; };
   auto dev_of = [](const Piece& p) { return (char*)p.rc->dev + p.row * p.rc->dev_pitch + p.col; };
@@ -158,13 +166,13 @@ cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, h
                          (uint32_t)p.rows);
       HIPTRY(hipGetLastError(), "copy");
     }
-    HIPTRY(hipEventRecord(g_piece_done[k % kPieces], st), "event");
+    HIPTRY(hipEventRecord(piece_done[k % kPieces], st), "event");
     return CV_OK;
   };
   hipError_t we = hipSuccess;
   if (to_device) {
     for (size_t k = 0; k < ps.size() && cs == CV_OK; k++) {
-      if (k >= kPieces) we = hipEventSynchronize(g_piece_done[k % kPieces]);
+      if (k >= kPieces) we = hipEventSynchronize(piece_done[k % kPieces]);
       if (we != hipSuccess) break;
       host_copy(k);
       cs = dev_copy(k);
@@ -174,7 +182,7 @@ cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, h
     for (size_t k = 0; k < ps.size() && cs == CV_OK; k++) {
       while (sent < ps.size() && sent < k + kPieces && cs == CV_OK) cs = dev_copy(sent++);
       if (cs != CV_OK) break;
-      we = hipEventSynchronize(g_piece_done[k % kPieces]);
+      we = hipEventSynchronize(piece_done[k % kPieces]);
       if (we != hipSuccess) break;
       host_copy(k);
     }
