@@ -1008,7 +1008,7 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
     // several traversal steps per refill check: the check's votes cost
     // about as much as a step's mask logic, and a lane that finishes early
     // idles for at most interval - 1 steps.  Bound by instruction issue in
-    // large launches (74 % VALU) and by the length of a step in the drain of
+    // large launches (80 % VALU) and by the length of a step in the drain of
     // all: a leaf round in the step that completes its quorum instead of the
     // next one (which took every entry again), no exact-rule branches inside
     // a step, and the hit test as one compare took the extend launches of a
