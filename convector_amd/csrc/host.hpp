@@ -11,35 +11,15 @@
 #include <vector>
 
 #include "../../include/convector.h"
+#include "copies.hpp"
 #include "internal.hpp"
 
 namespace cvh {
 
-// Records the message returned by cv_last_error() and passes the status on.
-cv_status fail(cv_status s, const std::string& msg);
-cv_status hip_fail(hipError_t e, const char* what);
 // Probes the HIP device once (CU count for the persistent launches).
 cv_status ensure_device();
 uint32_t num_cus();
 const char* last_error();
-// `rows` rows of `bytes` bytes of caller host memory and their place on the
-// device.
-struct CallerRect {
-  void* host;
-  void* dev;
-  size_t bytes, rows, host_pitch, dev_pitch;
-  static CallerRect flat(const void* host, void* dev, size_t bytes) {
-    return CallerRect{const_cast<void*>(host), dev, bytes, 1, bytes, bytes};
-  }
-};
-// Copies between caller host memory and the device through a pinned bounce
-// buffer, a piece at a time, waiting for the copies (and so for the work
-// queued before them on st): the runtime never copies from or to the caller's
-// pageable memory, and nothing touches that memory after the call returns.
-cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st);
-cv_status copy_caller_memory(void* dst, const void* src, size_t bytes, bool to_device,
-                             hipStream_t st);
-
 inline uint32_t grid_for(size_t n, uint32_t block, uint32_t cap = 1u << 20) {
   size_t b = (n + block - 1) / block;
   if (b < 1) b = 1;
@@ -108,12 +88,6 @@ struct LaunchCfg {
 };
 
 }  // namespace cvh
-
-#define HIPTRY(x, what)                                        \
-  do {                                                         \
-    hipError_t e_ = (x);                                       \
-    if (e_ != hipSuccess) return cvh::hip_fail(e_, what);      \
-  } while (0)
 
 struct cv_mesh {
   std::vector<float> v9;
