@@ -16,7 +16,10 @@ namespace {
 // the HIP runtime is torn down).  Copies go through it in pieces, each with
 // an event of its own, so that the host's copy of one piece overlaps the
 // device's of the next (a 1280 x 736 bitmap and gbuffer, 7.5 MB: 10.2 ms by
-// hipMemcpy2DAsync into pageable memory, row by row; 1.0 ms this way).
+// hipMemcpy2DAsync into pageable memory, row by row; 1.0 ms this way).  Coherent
+// memory: kernels write the pieces and the host reads them after waiting for
+// their events, which need not release to the system (without the flag,
+// portable memory is not coherent).
 constexpr size_t kPieceBytes = 2u << 20;
 constexpr uint32_t kPieces = 8;
 constexpr int kBounceDevices = 64;
@@ -32,7 +35,8 @@ cv_status bounce_init(hipEvent_t** done) {
   HIPTRY(hipGetDevice(&dev), "hipGetDevice");
   if (dev < 0 || dev >= kBounceDevices) return fail(CV_ERR_INVALID_ARGUMENT, "device index");
   if (!g_bounce)
-    HIPTRY(hipHostMalloc((void**)&g_bounce, kPieceBytes * kPieces, hipHostMallocPortable),
+    HIPTRY(hipHostMalloc((void**)&g_bounce, kPieceBytes * kPieces,
+                         hipHostMallocPortable | hipHostMallocCoherent),
            "pinned alloc");
   for (hipEvent_t& e : g_piece_done[dev])
     if (!e) HIPTRY(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");

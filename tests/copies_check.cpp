@@ -103,10 +103,19 @@ void check_shapes() {
   }
 }
 
+// Kernels write the pinned pieces and the host reads them after waiting for an
+// event: the memory is coherent, or the events release to the system.
+void check_coherent() {
+  copy_shapes({{1024, 4, 1024, 2048, 0}}, new_stream());
+  CHECK((fake::host_flags & hipHostMallocCoherent) || (fake::event_flags & hipEventReleaseToSystem));
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "shapes")
     check_shapes();
+  else if (name == "coherent")
+    check_coherent();
   else
     return 2;
   printf("ok\n");

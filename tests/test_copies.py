@@ -13,7 +13,7 @@ TESTS = os.path.dirname(os.path.abspath(__file__))
 @pytest.fixture(scope="module")
 def check(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("copies") / "copies_check")
-    r = subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-Wall", "-Wno-unused-function", "-pthread",
+    r = subprocess.run(["g++", "-O2", "-g", "-std=c++17", "-Wall", "-Wno-unused-function", "-pthread",
                         "-I", os.path.join(TESTS, "host_hip"),
                         os.path.join(TESTS, "copies_check.cpp"), "-o", exe],
                        capture_output=True, text=True)
@@ -28,3 +28,7 @@ def check(tmp_path_factory):
 
 def test_pieces_and_boundaries(check):
     check("shapes")
+
+
+def test_pieces_are_coherent(check):
+    check("coherent")
