@@ -28,12 +28,31 @@ char* g_bounce = nullptr;
 // per device (an event is recorded on streams of its own device only)
 hipEvent_t g_piece_done[kBounceDevices][kPieces] = {};
 
-// The current device's events, with the bounce buffer allocated; g_bounce_mu
-// held.
-cv_status bounce_init(hipEvent_t** done) {
-  int dev = 0;
-  HIPTRY(hipGetDevice(&dev), "hipGetDevice");
-  if (dev < 0 || dev >= kBounceDevices) return fail(CV_ERR_INVALID_ARGUMENT, "device index");
+// Makes the stream's device current while it lives: a copy works whatever
+// device the calling thread has current (its events and launches belong to
+// the stream's device).
+struct OnDeviceOf {
+  int device = 0, before = -1;
+  cv_status enter(hipStream_t st) {
+    int current = 0;
+    HIPTRY(hipGetDevice(&current), "hipGetDevice");
+    HIPTRY(hipStreamGetDevice(st, &device), "hipStreamGetDevice");
+    if (device < 0 || device >= kBounceDevices)
+      return fail(CV_ERR_INVALID_ARGUMENT, "device index");
+    if (device != current) {
+      HIPTRY(hipSetDevice(device), "hipSetDevice");
+      before = current;
+    }
+    return CV_OK;
+  }
+  ~OnDeviceOf() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
+// The events of device dev (current), with the bounce buffer allocated;
+// g_bounce_mu held.
+cv_status bounce_init(int dev, hipEvent_t** done) {
   if (!g_bounce)
     HIPTRY(hipHostMalloc((void**)&g_bounce, kPieceBytes * kPieces,
                          hipHostMallocPortable | hipHostMallocCoherent),
@@ -82,9 +101,12 @@ cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, h
     }
   }
   if (ps.empty()) return CV_OK;
+  OnDeviceOf on;
+  cv_status cs = on.enter(st);
+  if (cs != CV_OK) return cs;
   std::lock_guard<std::mutex> lk(g_bounce_mu);
   hipEvent_t* piece_done = nullptr;
-  cv_status cs = bounce_init(&piece_done);
+  cs = bounce_init(on.device, &piece_done);
   if (cs != CV_OK) return cs;
   auto host_of = [](const Piece& p) { return (char*)p.rc->host + p.row * p.rc->host_pitch + p.col; };
   auto dev_of = [](const Piece& p) { return (char*)p.rc->dev + p.row * p.rc->dev_pitch + p.col; };

@@ -110,12 +110,29 @@ void check_coherent() {
   CHECK((fake::host_flags & hipHostMallocCoherent) || (fake::event_flags & hipEventReleaseToSystem));
 }
 
+// A copy works whatever device the calling thread has current, with events of
+// the stream's device, and leaves the current device as it was.
+void check_devices() {
+  fake::devices = 3;
+  for (int on : {2, 0, 1}) {
+    fake::current = on;
+    hipStream_t st = new_stream();
+    for (int current : {0, 1, 2}) {
+      fake::current = current;
+      copy_shapes({{1024, 4, 1024, 2048, 0}, {3 * P, 1, 0, 0, 0}}, st);
+      CHECK(fake::current == current);
+    }
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "shapes")
     check_shapes();
   else if (name == "coherent")
     check_coherent();
+  else if (name == "devices")
+    check_devices();
   else
     return 2;
   printf("ok\n");

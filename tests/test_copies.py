@@ -32,3 +32,7 @@ def test_pieces_and_boundaries(check):
 
 def test_pieces_are_coherent(check):
     check("coherent")
+
+
+def test_any_current_device(check):
+    check("devices")
