@@ -678,7 +678,8 @@ cv_status cv_scene_copy_bvh(const cv_scene* s, cv_bvh_node* nodes, uint32_t* ord
   const cvh::CallerRect down[2] = {
       cvh::CallerRect::flat(nodes, s->nodes.p, nodes ? (size_t)s->info.num_nodes * 32 : 0),
       cvh::CallerRect::flat(order, s->tri_src.p, order ? (size_t)s->ntris * 4 : 0)};
-  return cvh::copy_caller_rects(down, 2, false, s->stream);
+  // the tree never changes: a copy does not wait for the scene's queries
+  return cvh::copy_settled_rects(down, 2, s->stream);
 }
 
 void cv_scene_destroy(cv_scene* s) {

@@ -3,6 +3,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <condition_variable>
 #include <mutex>
 #include <vector>
 
@@ -11,22 +12,85 @@
 namespace cvh {
 
 namespace {
-// One pinned bounce buffer for the whole process, allocated on first use and
-// kept until the process ends (freeing pinned memory at exit can run after
-// the HIP runtime is torn down).  Copies go through it in pieces, each with
-// an event of its own, so that the host's copy of one piece overlaps the
-// device's of the next (a 1280 x 736 bitmap and gbuffer, 7.5 MB: 10.2 ms by
-// hipMemcpy2DAsync into pageable memory, row by row; 1.0 ms this way).  Coherent
-// memory: kernels write the pieces and the host reads them after waiting for
-// their events, which need not release to the system (without the flag,
-// portable memory is not coherent).
+// Copies go through pinned memory in pieces, each with an event of its own, so
+// that the host's copy of one piece overlaps the device's of the next (a
+// 1280 x 736 bitmap and gbuffer, 7.5 MB: 10.2 ms by hipMemcpy2DAsync into
+// pageable memory, row by row; 1.0 ms this way).  Coherent memory: kernels write
+// the pieces and the host reads them after waiting for their events, which need
+// not release to the system (without the flag, portable memory is not coherent).
 constexpr size_t kPieceBytes = 2u << 20;
 constexpr uint32_t kPieces = 8;
-constexpr int kBounceDevices = 64;
-std::mutex g_bounce_mu;
-char* g_bounce = nullptr;
-// per device (an event is recorded on streams of its own device only)
-hipEvent_t g_piece_done[kBounceDevices][kPieces] = {};
+constexpr int kDevices = 64;
+
+// The pieces of one copy at a time.  The process has kRings of them, so that
+// threads copy at the same time; a ring's 16 MB are allocated when so many
+// copies run at once for the first time (one copy after the other uses the
+// first ring only), and kept until the process ends (freeing pinned memory at
+// exit can run after the HIP runtime is torn down).
+constexpr uint32_t kRings = 4;
+struct Ring {
+  bool leased = false;
+  char* pieces = nullptr;
+  // per device: an event is recorded on streams of its own device only
+  hipEvent_t done[kDevices][kPieces] = {};
+  hipStream_t stream[kDevices] = {};  // for copies that no queued work precedes
+};
+Ring g_rings[kRings];
+std::mutex g_rings_mu;
+// (never destroyed: a thread may still wait when the process exits)
+std::condition_variable& g_ring_free = *new std::condition_variable;
+
+// Leases a ring for a copy on st.  The last free one goes only to a copy whose
+// stream has no earlier work left, so that copies behind a long launch never
+// hold up one that can start.
+class Lease {
+ public:
+  ~Lease() {
+    if (!ring_) return;
+    std::lock_guard<std::mutex> lk(g_rings_mu);
+    ring_->leased = false;
+    g_ring_free.notify_one();
+  }
+  cv_status take(hipStream_t st, bool ready) {
+    std::unique_lock<std::mutex> lk(g_rings_mu);
+    for (;;) {
+      uint32_t free = 0;
+      Ring* first = nullptr;
+      for (Ring& r : g_rings) {
+        if (r.leased) continue;
+        if (!first) first = &r;
+        free++;
+      }
+      if (free > (ready ? 0u : 1u)) {
+        first->leased = true;
+        ring_ = first;
+        return CV_OK;
+      }
+      if (ready) {
+        g_ring_free.wait(lk);
+      } else {
+        lk.unlock();
+        HIPTRY(hipStreamSynchronize(st), "copy");
+        ready = true;
+        lk.lock();
+      }
+    }
+  }
+  // The ring with its memory, and its events on device dev (current).
+  cv_status init(int dev) {
+    if (!ring_->pieces)
+      HIPTRY(hipHostMalloc((void**)&ring_->pieces, kPieceBytes * kPieces,
+                           hipHostMallocPortable | hipHostMallocCoherent),
+             "pinned alloc");
+    for (hipEvent_t& e : ring_->done[dev])
+      if (!e) HIPTRY(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
+    return CV_OK;
+  }
+  Ring* operator->() const { return ring_; }
+
+ private:
+  Ring* ring_ = nullptr;
+};
 
 // Makes the stream's device current while it lives: a copy works whatever
 // device the calling thread has current (its events and launches belong to
@@ -37,7 +101,7 @@ struct OnDeviceOf {
     int current = 0;
     HIPTRY(hipGetDevice(&current), "hipGetDevice");
     HIPTRY(hipStreamGetDevice(st, &device), "hipStreamGetDevice");
-    if (device < 0 || device >= kBounceDevices)
+    if (device < 0 || device >= kDevices)
       return fail(CV_ERR_INVALID_ARGUMENT, "device index");
     if (device != current) {
       HIPTRY(hipSetDevice(device), "hipSetDevice");
@@ -50,19 +114,6 @@ struct OnDeviceOf {
   }
 };
 
-// The events of device dev (current), with the bounce buffer allocated;
-// g_bounce_mu held.
-cv_status bounce_init(int dev, hipEvent_t** done) {
-  if (!g_bounce)
-    HIPTRY(hipHostMalloc((void**)&g_bounce, kPieceBytes * kPieces,
-                         hipHostMallocPortable | hipHostMallocCoherent),
-           "pinned alloc");
-  for (hipEvent_t& e : g_piece_done[dev])
-    if (!e) HIPTRY(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
-  *done = g_piece_done[dev];
-  return CV_OK;
-}
-
 // Rows of `words` 16-byte words between a pitched and a packed buffer.
 __global__ void k_copy_rows(const uint4* src, size_t spitch, uint4* dst, size_t dpitch,
                             uint32_t words, uint32_t rows) {
@@ -71,15 +122,17 @@ __global__ void k_copy_rows(const uint4* src, size_t spitch, uint4* dst, size_t 
     dst[(size_t)(k / words) * dpitch + k % words] = src[(size_t)(k / words) * spitch + k % words];
 }
 
-// The part of a rect that one piece of the bounce buffer takes: rows
+// The part of a rect that one piece of pinned memory takes: rows
 // [row, row + rows) of `bytes` bytes from byte `col` on.
 struct Piece {
   const CallerRect* rc;
   size_t col, bytes, row, rows;
 };
-}  // namespace
 
-cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st) {
+// settled: no queued work reads or writes the device memory, so that the copy
+// runs on the ring's own stream, on the device of st.
+cv_status copy_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st,
+                     bool settled) {
   std::vector<Piece> ps;
   for (size_t i = 0; i < n; i++) {
     const CallerRect& r = rects[i];
@@ -104,15 +157,20 @@ cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, h
   OnDeviceOf on;
   cv_status cs = on.enter(st);
   if (cs != CV_OK) return cs;
-  std::lock_guard<std::mutex> lk(g_bounce_mu);
-  hipEvent_t* piece_done = nullptr;
-  cs = bounce_init(on.device, &piece_done);
-  if (cs != CV_OK) return cs;
+  Lease ring;
+  if ((cs = ring.take(st, settled)) != CV_OK || (cs = ring.init(on.device)) != CV_OK) return cs;
+  if (settled) {
+    hipStream_t& own = ring->stream[on.device];
+    if (!own) HIPTRY(hipStreamCreateWithFlags(&own, hipStreamNonBlocking), "hipStreamCreate");
+    st = own;
+  }
+  char* const pieces = ring->pieces;
+  hipEvent_t* const piece_done = ring->done[on.device];
   auto host_of = [](const Piece& p) { return (char*)p.rc->host + p.row * p.rc->host_pitch + p.col; };
   auto dev_of = [](const Piece& p) { return (char*)p.rc->dev + p.row * p.rc->dev_pitch + p.col; };
   auto host_copy = [&](size_t k) {
     const Piece& p = ps[k];
-    char* b = g_bounce + (k % kPieces) * kPieceBytes;
+    char* b = pieces + (k % kPieces) * kPieceBytes;
     for (size_t y = 0; y < p.rows; y++) {
       char* h = host_of(p) + y * p.rc->host_pitch;
       if (to_device)
@@ -123,7 +181,7 @@ cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, h
   };
   auto dev_copy = [&](size_t k) -> cv_status {
     const Piece& p = ps[k];
-    char* b = g_bounce + (k % kPieces) * kPieceBytes;
+    char* b = pieces + (k % kPieces) * kPieceBytes;
     const bool words = !((p.bytes | p.rc->dev_pitch | (size_t)dev_of(p)) & 15);
     if (p.rows == 1 && (to_device || !words)) {
       HIPTRY(hipMemcpyAsync(to_device ? dev_of(p) : b, to_device ? b : dev_of(p), p.bytes,
@@ -160,12 +218,21 @@ cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, h
       host_copy(k);
     }
   }
-  // the bounce buffer is the next caller's from here on
+  // the ring is the next caller's from here on
   const hipError_t se = hipStreamSynchronize(st);
   if (cs != CV_OK) return cs;
   HIPTRY(we, "copy");
   HIPTRY(se, "copy");
   return CV_OK;
+}
+}  // namespace
+
+cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st) {
+  return copy_rects(rects, n, to_device, st, false);
+}
+
+cv_status copy_settled_rects(const CallerRect* rects, size_t n, hipStream_t st) {
+  return copy_rects(rects, n, false, st, true);
 }
 
 cv_status copy_caller_memory(void* dst, const void* src, size_t bytes, bool to_device,

@@ -25,13 +25,16 @@ struct CallerRect {
     return CallerRect{const_cast<void*>(host), dev, bytes, 1, bytes, bytes};
   }
 };
-// Copies between caller host memory and the device through a pinned bounce
-// buffer, a piece at a time, waiting for the copies (and so for the work
-// queued before them on st): the runtime never copies from or to the caller's
-// pageable memory, and nothing touches that memory after the call returns.
+// Copies between caller host memory and the device through pinned memory, a
+// piece at a time, waiting for the copies (and so for the work queued before
+// them on st): the runtime never copies from or to the caller's pageable
+// memory, and nothing touches that memory after the call returns.
 cv_status copy_caller_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st);
 cv_status copy_caller_memory(void* dst, const void* src, size_t bytes, bool to_device,
                              hipStream_t st);
+// Downloads device memory that no queued work writes (a scene's tree) without
+// waiting for the work of st, whose device it lies on.
+cv_status copy_settled_rects(const CallerRect* rects, size_t n, hipStream_t st);
 
 }  // namespace cvh
 

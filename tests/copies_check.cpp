@@ -3,6 +3,10 @@
 #include "../convector_amd/csrc/copies.hip"
 
 #include <stdio.h>
+#include <unistd.h>
+
+#include <chrono>
+#include <future>
 
 namespace cvh {
 cv_status fail(cv_status s, const std::string&) { return s; }
@@ -125,6 +129,68 @@ void check_devices() {
   }
 }
 
+// Copies that wait for earlier work of their streams do not hold up those that
+// can start at once, however many they are; the pinned memory stays bounded.
+void check_threads() {
+  std::vector<char> dev(3 * P + 5, 'd');
+  std::vector<std::vector<char>> host(8, std::vector<char>(dev.size()));
+  fake::Gate gate;
+  std::vector<std::future<cv_status>> waiting;
+  auto download = [&](size_t k, hipStream_t st) {
+    return cvh::copy_caller_memory(host[k].data(), dev.data(), dev.size(), false, st);
+  };
+  for (size_t k = 0; k < 6; k++) {
+    hipStream_t st = new_stream();
+    fake::close_gate(st, &gate);
+    waiting.push_back(std::async(std::launch::async, download, k, st));
+  }
+  for (auto& w : waiting)
+    CHECK(w.wait_for(std::chrono::milliseconds(200)) == std::future_status::timeout);
+  for (size_t k = 6; k < 8; k++) {
+    auto free_one = std::async(std::launch::async, download, k, new_stream());
+    const bool done = free_one.wait_for(std::chrono::seconds(10)) == std::future_status::ready;
+    if (!done) {
+      printf("a copy waits for the work of other streams\n");
+      fflush(stdout);
+      _exit(1);
+    }
+    CHECK(free_one.get() == CV_OK && host[k] == dev);
+  }
+  gate.unlock();
+  for (size_t k = 0; k < 6; k++) CHECK(waiting[k].get() == CV_OK && host[k] == dev);
+  CHECK(fake::host_allocs <= 4);
+}
+
+// Many threads at once, each with a stream of its own: every copy arrives.
+void check_crowd() {
+  std::vector<std::future<void>> all;
+  for (int t = 0; t < 12; t++)
+    all.push_back(std::async(std::launch::async, [] {
+      hipStream_t st = new_stream();
+      for (int k = 0; k < 3; k++)
+        copy_shapes({{1024, 700, 1040, 1536, 0}, {P + 9, 1, 0, 0, 4}}, st);
+    }));
+  for (auto& a : all) a.get();
+  CHECK(fake::host_allocs <= 4);
+}
+
+// Device memory that no queued work writes is copied without waiting for the
+// object's stream.
+void check_settled() {
+  fake::devices = 2;
+  fake::current = 1;
+  hipStream_t st = new_stream();
+  fake::current = 0;
+  fake::Gate gate;
+  fake::close_gate(st, &gate);
+  std::vector<char> dev(3 * P + 5, 'd'), host(dev.size());
+  const CallerRect r = CallerRect::flat(host.data(), dev.data(), dev.size());
+  auto copy = std::async(std::launch::async, [&] { return cvh::copy_settled_rects(&r, 1, st); });
+  if (copy.wait_for(std::chrono::seconds(10)) != std::future_status::ready) _exit(1);
+  CHECK(copy.get() == CV_OK && host == dev);
+  gate.unlock();
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "shapes")
@@ -133,6 +199,12 @@ int main(int argc, char** argv) {
     check_coherent();
   else if (name == "devices")
     check_devices();
+  else if (name == "threads")
+    check_threads();
+  else if (name == "crowd")
+    check_crowd();
+  else if (name == "settled")
+    check_settled();
   else
     return 2;
   printf("ok\n");

@@ -36,3 +36,8 @@ def test_pieces_are_coherent(check):
 
 def test_any_current_device(check):
     check("devices")
+
+
+@pytest.mark.parametrize("name", ["threads", "crowd", "settled"])
+def test_concurrent_copies(check, name):
+    check(name)
