@@ -485,16 +485,19 @@ static cv_status scene_finish(cv_scene* s, const cv_mesh* const* meshes, size_t 
   HIPTRY(d_uv.alloc(6ull * N), "alloc");
   HIPTRY(d_mat.alloc(N), "alloc");
   {
+    // (array by array: each array's parts follow each other on the device and
+    // share transfers; one per mesh and array took 20,000 meshes 0.48 s)
     std::vector<cvh::CallerRect> up;
-    size_t at = 0;
-    for (size_t i = 0; i < nmeshes; i++) {
-      const cv_mesh& m = *meshes[i];
-      const size_t k = m.ntris();
-      up.push_back(cvh::CallerRect::flat(m.v9.data(), d_v9.p + 9 * at, k * 36));
-      up.push_back(cvh::CallerRect::flat(m.uv6.data(), d_uv.p + 6 * at, k * 24));
-      up.push_back(cvh::CallerRect::flat(m.mat.data(), d_mat.p + at, k * 4));
-      at += k;
-    }
+    auto array = [&](auto* dev, auto part) {
+      for (size_t i = 0; i < nmeshes; i++) {
+        const auto& v = part(*meshes[i]);
+        up.push_back(cvh::CallerRect::flat(v.data(), dev, v.size() * 4, i > 0));
+        dev += v.size();
+      }
+    };
+    array(d_v9.p, [](const cv_mesh& m) -> auto& { return m.v9; });
+    array(d_uv.p, [](const cv_mesh& m) -> auto& { return m.uv6; });
+    array(d_mat.p, [](const cv_mesh& m) -> auto& { return m.mat; });
     cv_status us = cvh::copy_caller_rects(up.data(), up.size(), true, st);
     if (us != CV_OK) return us;
   }

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <condition_variable>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "copies.hpp"
@@ -122,37 +123,78 @@ __global__ void k_copy_rows(const uint4* src, size_t spitch, uint4* dst, size_t 
     dst[(size_t)(k / words) * dpitch + k % words] = src[(size_t)(k / words) * spitch + k % words];
 }
 
-// The part of a rect that one piece of pinned memory takes: rows
-// [row, row + rows) of `bytes` bytes from byte `col` on.
+// What one piece of pinned memory takes: `rows` rows of `bytes` bytes on the
+// device, packed in the piece, and the spans of host memory (from spans[first]
+// on) whose bytes follow each other there.
+struct Span {
+  char* host;
+  size_t bytes, rows, pitch;
+};
 struct Piece {
-  const CallerRect* rc;
-  size_t col, bytes, row, rows;
+  char* dev;
+  size_t bytes, rows, pitch, first, spans;
+};
+struct Plan {
+  std::vector<Span> spans;
+  std::vector<Piece> pieces;
+  bool open = false;  // the last piece may take what follows it on the device
+
+  void flat(char* host, char* dev, size_t n) {
+    while (n) {
+      Piece* last = open ? &pieces.back() : nullptr;
+      if (last && (last->dev + last->bytes != dev || last->bytes == kPieceBytes)) last = nullptr;
+      const size_t c = std::min(n, kPieceBytes - (last ? last->bytes : 0));
+      if (last) {
+        last->bytes += c;
+        last->spans++;
+      } else {
+        pieces.push_back(Piece{dev, c, 1, 0, spans.size(), 1});
+      }
+      spans.push_back(Span{host, c, 1, 0});
+      open = true;
+      host += c;
+      dev += c;
+      n -= c;
+    }
+  }
+  void add(const CallerRect& r) {
+    if (!r.follows) open = false;
+    if (!r.bytes || !r.rows) return;
+    char *host = (char*)r.host, *dev = (char*)r.dev;
+    const bool words = !((r.bytes | r.dev_pitch | (size_t)r.dev) & 15);
+    if (r.rows == 1 || (r.host_pitch == r.bytes && r.dev_pitch == r.bytes)) {
+      flat(host, dev, r.bytes * r.rows);
+    } else if (r.bytes > kPieceBytes || !words) {
+      // rows longer than a piece (an HDR rectangle from 43,691 pixels of width
+      // on) or not of 16-byte words
+      for (size_t y = 0; y < r.rows; y++) {
+        open = false;
+        flat(host + y * r.host_pitch, dev + y * r.dev_pitch, r.bytes);
+      }
+      open = false;
+    } else {
+      const size_t per = kPieceBytes / r.bytes;
+      for (size_t y = 0; y < r.rows; y += per) {
+        const size_t rows = std::min(per, r.rows - y);
+        pieces.push_back(Piece{dev + y * r.dev_pitch, r.bytes, rows, r.dev_pitch, spans.size(), 1});
+        spans.push_back(Span{host + y * r.host_pitch, r.bytes, rows, r.host_pitch});
+      }
+      open = false;
+    }
+  }
 };
 
 // settled: no queued work reads or writes the device memory, so that the copy
 // runs on the ring's own stream, on the device of st.
 cv_status copy_rects(const CallerRect* rects, size_t n, bool to_device, hipStream_t st,
                      bool settled) {
-  std::vector<Piece> ps;
-  for (size_t i = 0; i < n; i++) {
-    const CallerRect& r = rects[i];
-    if (!r.bytes || !r.rows) continue;
-    const bool packed = r.rows == 1 || (r.host_pitch == r.bytes && r.dev_pitch == r.bytes);
-    const bool words = !((r.bytes | r.dev_pitch | (size_t)r.dev) & 15);
-    if (packed || r.bytes > kPieceBytes || !words) {
-      // contiguous, or rows longer than a piece (an HDR rectangle from 43,691
-      // pixels of width on) or not of 16-byte words: bytes of one row (or of
-      // all)
-      const size_t row_bytes = packed ? r.bytes * r.rows : r.bytes;
-      for (size_t y = 0; y < (packed ? 1 : r.rows); y++)
-        for (size_t c = 0; c < row_bytes; c += kPieceBytes)
-          ps.push_back(Piece{&r, c, std::min(kPieceBytes, row_bytes - c), y, 1});
-    } else {
-      const size_t per = kPieceBytes / r.bytes;
-      for (size_t y = 0; y < r.rows; y += per)
-        ps.push_back(Piece{&r, 0, r.bytes, y, std::min(per, r.rows - y)});
-    }
+  Plan plan;
+  try {
+    for (size_t i = 0; i < n; i++) plan.add(rects[i]);
+  } catch (const std::bad_alloc&) {
+    return fail(CV_ERR_OUT_OF_MEMORY, "copy plan");
   }
+  const std::vector<Piece>& ps = plan.pieces;
   if (ps.empty()) return CV_OK;
   OnDeviceOf on;
   cv_status cs = on.enter(st);
@@ -166,31 +208,31 @@ cv_status copy_rects(const CallerRect* rects, size_t n, bool to_device, hipStrea
   }
   char* const pieces = ring->pieces;
   hipEvent_t* const piece_done = ring->done[on.device];
-  auto host_of = [](const Piece& p) { return (char*)p.rc->host + p.row * p.rc->host_pitch + p.col; };
-  auto dev_of = [](const Piece& p) { return (char*)p.rc->dev + p.row * p.rc->dev_pitch + p.col; };
   auto host_copy = [&](size_t k) {
-    const Piece& p = ps[k];
     char* b = pieces + (k % kPieces) * kPieceBytes;
-    for (size_t y = 0; y < p.rows; y++) {
-      char* h = host_of(p) + y * p.rc->host_pitch;
-      if (to_device)
-        memcpy(b + y * p.bytes, h, p.bytes);
-      else
-        memcpy(h, b + y * p.bytes, p.bytes);
+    for (size_t j = 0; j < ps[k].spans; j++) {
+      const Span& sp = plan.spans[ps[k].first + j];
+      for (size_t y = 0; y < sp.rows; y++, b += sp.bytes) {
+        char* h = sp.host + y * sp.pitch;
+        if (to_device)
+          memcpy(b, h, sp.bytes);
+        else
+          memcpy(h, b, sp.bytes);
+      }
     }
   };
   auto dev_copy = [&](size_t k) -> cv_status {
     const Piece& p = ps[k];
     char* b = pieces + (k % kPieces) * kPieceBytes;
-    const bool words = !((p.bytes | p.rc->dev_pitch | (size_t)dev_of(p)) & 15);
+    const bool words = !((p.bytes | p.pitch | (size_t)p.dev) & 15);
     if (p.rows == 1 && (to_device || !words)) {
-      HIPTRY(hipMemcpyAsync(to_device ? dev_of(p) : b, to_device ? b : dev_of(p), p.bytes,
+      HIPTRY(hipMemcpyAsync(to_device ? p.dev : b, to_device ? b : p.dev, p.bytes,
                             to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, st),
              "copy");
     } else {
-      const uint4* src = (const uint4*)(to_device ? b : dev_of(p));
-      uint4* dst = (uint4*)(to_device ? dev_of(p) : b);
-      const size_t pk = p.bytes / 16, pitch = p.rc->dev_pitch / 16;
+      const uint4* src = (const uint4*)(to_device ? b : p.dev);
+      uint4* dst = (uint4*)(to_device ? p.dev : b);
+      const size_t pk = p.bytes / 16, pitch = p.pitch / 16;
       const uint32_t blocks = (uint32_t)std::min<size_t>((pk * p.rows + 255) / 256, 256);
       hipLaunchKernelGGL(k_copy_rows, dim3(blocks), dim3(256), 0, st, src,
                          to_device ? pk : pitch, dst, to_device ? pitch : pk, (uint32_t)pk,
@@ -237,11 +279,8 @@ cv_status copy_settled_rects(const CallerRect* rects, size_t n, hipStream_t st) 
 
 cv_status copy_caller_memory(void* dst, const void* src, size_t bytes, bool to_device,
                              hipStream_t st) {
-  CallerRect r;
-  r.host = to_device ? const_cast<void*>(src) : dst;
-  r.dev = to_device ? dst : const_cast<void*>(src);
-  r.bytes = r.host_pitch = r.dev_pitch = bytes;
-  r.rows = 1;
+  const CallerRect r = to_device ? CallerRect::flat(src, dst, bytes)
+                                 : CallerRect::flat(dst, const_cast<void*>(src), bytes);
   return copy_caller_rects(&r, 1, to_device, st);
 }
 

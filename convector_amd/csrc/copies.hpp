@@ -21,8 +21,11 @@ struct CallerRect {
   void* host;
   void* dev;
   size_t bytes, rows, host_pitch, dev_pitch;
-  static CallerRect flat(const void* host, void* dev, size_t bytes) {
-    return CallerRect{const_cast<void*>(host), dev, bytes, 1, bytes, bytes};
+  // the rect before it ends where this one begins, in the same allocation: the
+  // two share transfers
+  bool follows;
+  static CallerRect flat(const void* host, void* dev, size_t bytes, bool follows = false) {
+    return CallerRect{const_cast<void*>(host), dev, bytes, 1, bytes, bytes, follows};
   }
 };
 // Copies between caller host memory and the device through pinned memory, a

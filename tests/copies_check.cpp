@@ -64,7 +64,7 @@ void copy_shapes(const std::vector<Shape>& shapes, hipStream_t st) {
       else
         m.before = m.host;
       rects.push_back(CallerRect{m.host.data() + kEdge, m.dev + kEdge + s.dev_off, s.bytes, s.rows,
-                                 s.host_pitch, s.dev_pitch});
+                                 s.host_pitch, s.dev_pitch, false});
     }
     CHECK(cvh::copy_caller_rects(rects.data(), rects.size(), up, st) == CV_OK);
     for (size_t i = 0; i < shapes.size(); i++) {
@@ -191,6 +191,40 @@ void check_settled() {
   gate.unlock();
 }
 
+// Small pieces of caller memory that follow each other in an array on the device
+// (those of many meshes) share transfers, in both directions, whatever their
+// sizes; what only happens to lie behind the piece before does not.
+void check_many() {
+  for (bool up : {true, false}) {
+    std::vector<std::vector<char>> host;
+    std::vector<CallerRect> rects;
+    size_t total = 0;
+    for (size_t k = 0; k < 20000; k++) {
+      // (20000 parts of two arrays of half as many, the first of each empty)
+      host.emplace_back(k % 10000 == 0 ? 0 : k == 777 ? 2 * P + 100 : 36 * (1 + k % 50));
+      for (size_t j = 0; j < host[k].size(); j++) host[k][j] = (char)(3 * k + j);
+      total += host[k].size();
+    }
+    std::vector<char> dev(total, 'd'), want;
+    for (size_t j = 0; !up && j < total; j++) dev[j] = (char)(j * 11 + (j >> 9));
+    size_t at = 0, transfers = 0, array = 0;
+    for (auto& h : host) {
+      rects.push_back(CallerRect::flat(h.data(), dev.data() + at, h.size(), rects.size() % 10000));
+      at += h.size();
+      array += h.size();
+      if (rects.size() % 10000 == 0) {
+        transfers += (array + P - 1) / P;
+        array = 0;
+      }
+    }
+    fake::transfers = 0;
+    CHECK(cvh::copy_caller_rects(rects.data(), rects.size(), up, new_stream()) == CV_OK);
+    for (auto& h : host) want.insert(want.end(), h.begin(), h.end());
+    CHECK(want == dev);
+    CHECK(fake::transfers == transfers);
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "shapes")
@@ -205,6 +239,8 @@ int main(int argc, char** argv) {
     check_crowd();
   else if (name == "settled")
     check_settled();
+  else if (name == "many")
+    check_many();
   else
     return 2;
   printf("ok\n");

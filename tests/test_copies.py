@@ -41,3 +41,7 @@ def test_any_current_device(check):
 @pytest.mark.parametrize("name", ["threads", "crowd", "settled"])
 def test_concurrent_copies(check, name):
     check(name)
+
+
+def test_neighbours_share_transfers(check):
+    check("many")
