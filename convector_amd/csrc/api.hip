@@ -711,6 +711,7 @@ cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_
   if (!sc || (n && !rays)) return fail(CV_ERR_INVALID_ARGUMENT, "null argument");
   if (n == 0) return CV_OK;
   if (n >= (1ull << 31)) return fail(CV_ERR_INVALID_ARGUMENT, "too many rays");
+  if (!hits && !isects) return CV_OK;
   cv_scene* s = const_cast<cv_scene*>(sc);
   std::lock_guard<std::mutex> g(s->mu);
   hipStream_t st = s->stream;
@@ -733,7 +734,6 @@ cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_
       ip = d_isects.p;
     }
   }
-  if (!hits && !isects) return CV_OK;
   // The renderer's lane-refill traversal (idle lanes take new rays, lanes at
   // leaves wait for a common leaf round) as a one-bounce step over the
   // caller's rays; each lane's operations are those of the single-ray
