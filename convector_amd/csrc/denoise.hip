@@ -450,7 +450,8 @@ __global__ __launch_bounds__(256, 2) void k_conv_halo(ConvArgs a) {
   size_t img_base = 0;
   const uint32_t row0 = blockIdx.y * WR;  // first output of the slice
   // this thread's input pieces: element offset of chunk 0, or ~0u outside
-  // the image; its weight pieces: element offset of chunk 0
+  // the image (a launch's input is below 2^32 elements: images_per_launch);
+  // its weight pieces: element offset of chunk 0
   uint32_t xoff[XPT], woff[WPT];
   // tile t's corner and its input pieces' offsets
   auto tile_offsets = [&](uint32_t t, int& tx0, int& ty0, size_t& tbase) {
@@ -673,8 +674,9 @@ __global__ __launch_bounds__(512, 2) void k_conv_res(ConvArgs a) {
     ty = (int)(((t / ntx) % nty) * kHaloH);
     base = (size_t)(t / (ntx * nty)) * a.h * a.w_;
   };
-  // element offset of this thread's input pieces of tile t, ~0u outside the
-  // image (loaded from the tensor's first pixel and zeroed when stored)
+  // element offset of this thread's input pieces of tile t (below 2^32:
+  // images_per_launch), ~0u outside the image (loaded from the tensor's first
+  // pixel and zeroed when stored)
   uint32_t xoff[XPT];
   auto tile_offsets = [&](uint32_t t) {
     int tx, ty;
@@ -1684,6 +1686,28 @@ bool try_res(cv_denoiser* d, const cvd::ConvArgs& a, uint32_t nt) {
   return true;
 }
 
+// The halo-tile kernels address an input with 32-bit element offsets from its
+// first pixel, so one launch takes as many whole images of `channels` elements
+// a pixel as lie below 2^32 elements; 0: not even one.
+uint32_t images_per_launch(uint32_t h, uint32_t w, uint32_t channels) {
+  return (uint32_t)(((1ull << 32) - 1) / ((uint64_t)h * w * channels));
+}
+
+// Images [first, first + n) of a convolution.
+cvd::ConvArgs image_range(cvd::ConvArgs a, uint32_t first, uint32_t n) {
+  const size_t p = (size_t)first * a.h * a.w_, q = p / 4;
+  a.npix = n * a.h * a.w_;
+  a.x += p * a.xcs;
+  if (a.y) a.y += p * a.ycs;
+  if (a.yf) a.yf += p * a.yfcs;
+  if (a.mask) a.mask += p * a.mcs;
+  if (a.xup) a.xup += q * a.xupcs;
+  if (a.pool) a.pool += q * a.poolcs;
+  if (a.ug_dz) a.ug_dz += q * a.ug_dzcs;
+  if (a.ug_mask) a.ug_mask += q * a.ug_mcs;
+  return a;
+}
+
 bool launch_conv_halo(cv_denoiser* d, const cvd::ConvArgs& a, uint32_t nt) {
   // whole 32-pixel rows, whole images, and every pixel's KC channels within
   // its stride (the tile loads read channels [0, KC) of each pixel)
@@ -1703,6 +1727,14 @@ bool launch_conv_halo(cv_denoiser* d, const cvd::ConvArgs& a, uint32_t nt) {
   if (a.xup && (a.h % 2 || a.w_ % 2 || a.xupcs % 8 || a.xupcs < 32 * a.up_chunks ||
                 32 * a.up_chunks > a.kc))
     return false;
+  const uint32_t imgs = a.npix / (a.h * a.w_);
+  const uint32_t fit =
+      images_per_launch(a.h, a.w_, a.xup ? std::max(a.xcs, (a.xupcs + 3) / 4) : a.xcs);
+  if (fit < imgs) {
+    for (uint32_t k = 0; k < imgs; k += fit)
+      if (!fit || !launch_conv_halo(d, image_range(a, k, std::min(fit, imgs - k)), nt)) return false;
+    return true;
+  }
   if (try_res<64, false>(d, a, nt) || try_res<64, false, false, true>(d, a, nt) ||
       try_res<64, true, true>(d, a, nt))
     return true;
@@ -2019,7 +2051,11 @@ cv_status forward(cv_denoiser* d, bool materialize, bool materialize_pool, float
   if ((cs = (x)) != CV_OK) return cs
   // the pooled encoder outputs come from the convolutions' epilogues (the
   // same bits as k_pool, which the materialized path runs)
-  const bool fuse_pool = !materialize_pool && d->halo_convs && W % (2 * cvd::kHaloW) == 0;
+  // (fused where the halo-tile kernels take the layer: an image of theirs must
+  // fit one launch with the pooled layer's 32 or the upsampled one's 96
+  // channels)
+  const bool fuse_pool = !materialize_pool && d->halo_convs && W % (2 * cvd::kHaloW) == 0 &&
+                         images_per_launch(H, W, 32) > 0;
   CVD_TRY(conv_fwd(d, L[0], d->x0.p, 16, d->e0a.p, 32, nullptr, 0, H, W));
   if (fuse_pool) {
     CVD_TRY(conv_fwd(d, L[1], d->e0a.p, 32, d->cat0.p + 64, 96, nullptr, 0, H, W, nullptr, 0, 0,
@@ -2040,7 +2076,8 @@ cv_status forward(cv_denoiser* d, bool materialize, bool materialize_pool, float
   }
   CVD_TRY(conv_fwd(d, L[4], d->p1.p, 64, d->b2a.p, 128, nullptr, 0, H2, W2));
   CVD_TRY(conv_fwd(d, L[5], d->b2a.p, 128, d->b2b.p, 128, nullptr, 0, H2, W2));
-  const bool fuse_up = !materialize && d->halo_convs && W1 % cvd::kHaloW == 0;
+  const bool fuse_up = !materialize && d->halo_convs && W1 % cvd::kHaloW == 0 &&
+                       images_per_launch(H, W, 96) > 0;
   if (fuse_up) {
     CVD_TRY(conv_fwd(d, L[6], d->cat1.p, 192, d->d1a.p, 64, nullptr, 0, H1, W1, d->b2b.p, 128, 4));
   } else {
