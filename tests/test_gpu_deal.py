@@ -2,8 +2,8 @@
 every ray is traversed once and gives the oracle's hit at the sizes where the
 dealing changes shape -- fewer rays than the smallest share, one more than a
 share or a stripe of 64 rays per wave, the last dealt size and the first that
-goes through the cursors -- for grids that are and are not a multiple of the
-8 XCDs."""
+goes through the cursors.  (The grids are all multiples of the 8 XCDs on a
+device of 256 CUs; test_deal_map.py has the others.)"""
 import numpy as np
 import pytest
 
