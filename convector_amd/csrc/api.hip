@@ -589,6 +589,7 @@ static cv_status scene_finish(cv_scene* s, const cv_mesh* const* meshes, size_t 
   // traversal configuration: packed stack entries need index < 2^27 and
   // leaves of at most 31 triangles
   s->packed = s->info.max_leaf <= 31 && N < (1u << 27) && s->info.num_nodes < (1u << 27);
+  HIPTRY(s->cursor.alloc(cvk::kIsectGroups * cvk::kIsectCursorStride), "alloc");
   cv_tuning t{8, 32, 16, 1, 1};
   return scene_apply_tuning(s, t);
 }
@@ -696,6 +697,7 @@ void cv_scene_destroy(cv_scene* s) {
   s->direct.reset();
   s->lights.reset();
   s->spill.reset();
+  s->cursor.reset();
   s->q_ctrl.reset();
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
@@ -703,7 +705,12 @@ void cv_scene_destroy(cv_scene* s) {
 
 // --------------------------------------------------------------- traversal
 
-// Hits-only queries of at most this many rays per lane are dealt out.
+// Hits-only queries of at most this many rays per lane of 24 waves per CU are
+// dealt out: 1.57 M rays, below where the cursors draw level (250 k / 1 M / 2 M /
+// 4 M / 6 M decoherent rays in us, dealt against cursors: suzanne 109 / 182 /
+// 285 / 478 / 664 and 242 / 284 / 324 / 470 / 640, bunny 162 / 299 / 487 / 834 /
+// 1174 and 346 / 415 / 498 / 829 / 1117, a room of 200,000 triangles 450 / 816 /
+// 1212 / 2192 / 3115 and 808 / 975 / 1339 / 2203 / 3016; coherent rays alike).
 static constexpr uint32_t kQueryDeal = 4;
 
 cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_t n, cv_hit* hits,
@@ -734,66 +741,77 @@ cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_
       ip = d_isects.p;
     }
   }
-  // The renderer's lane-refill traversal (idle lanes take new rays, lanes at
-  // leaves wait for a common leaf round) as a one-bounce step over the
-  // caller's rays; each lane's operations are those of the single-ray
-  // traversal, so the hits are the same bits.  Full records keep the
-  // reference's tree, whose counters they hold; hits take the tuned one.
-  const uint32_t width = isects ? 2u : s->cfg.width;
-  cvk::ExtendArgs x{};
-  x.n = (uint32_t)n;
-  x.bounce = 0;
-  x.rays6 = rp;
-  x.tri_src = s->tri_src.p;
-  x.hits = reinterpret_cast<uint4*>(hp);
-  x.records = ip;
-  cv_status ws = cvh::ensure_wide_locked(s, width);
-  if (ws != CV_OK) return ws;
-  x.nodes = cvh::traversal_nodes(s, width);
-  x.tris = s->tris.p;
-  x.jobs = nullptr;
-  x.spill = s->spill.p;
-  // At least 4 batches of 64 rays per cursor fetch: queries end after a
-  // few dozen box tests, so one fetch per 64 rays serialises on the
-  // cursor (3.4 ms for 2^24 rays whatever the scene; 2.0 ms with 4 on
-  // 968 triangles).  Rendering keeps the tuned value (1 is fastest there).
-  x.batches = s->cfg.fetch_batches > 4 ? s->cfg.fetch_batches : 4u;
-  x.refill = s->cfg.refill <= 64 ? s->cfg.refill : isects ? 64u : 0u;
-  // Refill checks 4 times as often as the renderer's: a query ends after
-  // a few dozen box tests, so a finished lane would otherwise idle for a
-  // large share of a ray's steps (2^24 rays on suzanne: 1.79 -> 1.65 ms
-  // with 4 steps between checks instead of 16; the bunny's within 1 %).
-  x.interval = s->cfg.refill_interval > 4 ? s->cfg.refill_interval / 4 : 1u;
-  x.leaf_batch = s->cfg.leaf_batch <= 64 ? s->cfg.leaf_batch : 0u;
-  x.parts = s->cfg.parts;
-  // Up to kQueryDeal rays per lane the rays are dealt out to at most 24
-  // waves per CU, which is as fast as 32 for many rays and ends sooner with
-  // few (10^6 rays in a 200,000-triangle room: cursors 1.04 ms, dealt to 32
-  // waves per CU 1.03, to 24 0.86; 2 x 10^6: 1.51, 1.62, 1.42; 4 x 10^6:
-  // 2.29, 2.80, 2.33).  Whole-batch launches always use the cursor.
+  // Few rays are dealt out to at most 24 waves per CU beforehand, which is as
+  // fast as 32 for many rays and ends sooner with few.
   const uint32_t bw = s->cfg.block_waves;
   const uint32_t few = std::min(s->cfg.blocks, 24u * cvh::num_cus());
-  const uint64_t few_lanes = (uint64_t)((few + bw - 1) / bw * bw) * 64u;
-  x.deal = n <= few_lanes * kQueryDeal && (x.refill || width != 2);
-  if (!x.deal) {
-    if (!s->q_ctrl.p) HIPTRY(s->q_ctrl.alloc(1), "alloc");
-    HIPTRY(cvk::launch_query_ctrl(s->q_ctrl.p, (uint32_t)n, st), "query control");
-    x.ctrl = s->q_ctrl.p;
-  }
-  const uint32_t blocks = x.deal ? few : s->cfg.blocks;
   if (isects) {
+    // Full records on the reference's tree, whose counters they hold: 64 rays
+    // a wave until the slowest ends, dealt out up to one ray per lane and from
+    // the cursors above.  (The lane-refill traversal with a pass of its own for
+    // the records was 5-14 % faster for 10^6 and more decoherent rays in rooms
+    // of 50,000 triangles and more, but 5-27 % slower for coherent ones in
+    // smaller rooms and on the bunny.)
     cvk::IntersectArgs a{};
     a.rays = rp;
     a.n = (uint32_t)n;
+    a.cursor = s->cursor.p;
+    a.nodes = s->nodes.p;
     a.tris = s->tris.p;
     a.tri_src = s->tri_src.p;
     a.tri_mat = s->tri_mat.p;
     a.tri_uv = s->tri_uv.p;
+    a.spill = s->spill.p;
     a.hits = hp;
     a.isects = ip;
-    HIPTRY(cvk::launch_records(x, a, s->packed, s->cfg.stack, blocks, bw, st), "intersect");
+    const bool deal = n <= (uint64_t)few * 64u;
+    if (!deal)
+      HIPTRY(cvk::launch_zero_u32(s->cursor.p, cvk::kIsectGroups * cvk::kIsectCursorStride, st),
+             "zero");
+    HIPTRY(cvk::launch_intersect(a, true, s->packed, deal, s->cfg.stack,
+                                 deal ? few : s->cfg.blocks, st),
+           "intersect");
   } else {
-    HIPTRY(cvk::launch_extend(x, false, s->packed, false, s->cfg.stack, blocks, bw, st, width),
+    // Hits only: the renderer's lane-refill traversal (idle lanes take new
+    // rays, lanes at leaves wait for a common leaf round) as a one-bounce step
+    // over the caller's rays; each lane's operations are those of the
+    // single-ray traversal, so the hits are the same bits.
+    cvk::ExtendArgs x{};
+    x.n = (uint32_t)n;
+    x.bounce = 0;
+    x.rays6 = rp;
+    x.tri_src = s->tri_src.p;
+    x.hits = reinterpret_cast<uint4*>(hp);
+    cv_status ws = cvh::ensure_wide_locked(s, s->cfg.width);
+    if (ws != CV_OK) return ws;
+    x.nodes = cvh::traversal_nodes(s, s->cfg.width);
+    x.tris = s->tris.p;
+    x.jobs = nullptr;
+    x.spill = s->spill.p;
+    // At least 4 batches of 64 rays per cursor fetch: queries end after a
+    // few dozen box tests, so one fetch per 64 rays serialises on the
+    // cursor (3.4 ms for 2^24 rays whatever the scene; 2.0 ms with 4 on
+    // 968 triangles).  Rendering keeps the tuned value (1 is fastest there).
+    x.batches = s->cfg.fetch_batches > 4 ? s->cfg.fetch_batches : 4u;
+    x.refill = s->cfg.refill <= 64 ? s->cfg.refill : 0u;
+    // Refill checks 4 times as often as the renderer's: a query ends after
+    // a few dozen box tests, so a finished lane would otherwise idle for a
+    // large share of a ray's steps (2^24 rays on suzanne: 1.79 -> 1.65 ms
+    // with 4 steps between checks instead of 16; the bunny's within 1 %).
+    x.interval = s->cfg.refill_interval > 4 ? s->cfg.refill_interval / 4 : 1u;
+    x.leaf_batch = s->cfg.leaf_batch <= 64 ? s->cfg.leaf_batch : 0u;
+    x.parts = s->cfg.parts;
+    // Dealt out up to kQueryDeal rays per lane; whole-batch launches always
+    // use the cursor.
+    const uint64_t few_lanes = (uint64_t)((few + bw - 1) / bw * bw) * 64u;
+    x.deal = n <= few_lanes * kQueryDeal && (x.refill || s->cfg.width != 2);
+    if (!x.deal) {
+      if (!s->q_ctrl.p) HIPTRY(s->q_ctrl.alloc(1), "alloc");
+      HIPTRY(cvk::launch_query_ctrl(s->q_ctrl.p, (uint32_t)n, st), "query control");
+      x.ctrl = s->q_ctrl.p;
+    }
+    HIPTRY(cvk::launch_extend(x, false, s->packed, false, s->cfg.stack,
+                              x.deal ? few : s->cfg.blocks, bw, st, s->cfg.width),
            "intersect");
   }
   if (!dev) {
@@ -871,7 +889,8 @@ cv_status cv_bvh_intersect_nearest_noalloc(const cv_scene* sc, const cv_ray* ray
   // the cursors start at zero for every call (a fill kernel, no memset node)
   HIPTRY(cvk::launch_zero_u32(a.cursor, cvk::kIsectGroups * cvk::kIsectCursorStride, st),
          "zero");
-  HIPTRY(cvk::launch_intersect(a, isects != nullptr, s->packed, kNoAllocWaves, st), "intersect");
+  HIPTRY(cvk::launch_intersect(a, isects != nullptr, s->packed, false, cvk::kIsectStack,
+                               kNoAllocWaves, st), "intersect");
   HIPTRY(hipStreamSynchronize(st), "sync");
   return CV_OK;
 }

@@ -103,7 +103,6 @@ struct ExtendArgs {
   const uint32_t* order;      // non-null: queue position k traverses path order[k]
   uint32_t parts;             // lane refill: 1 (one cursor) or kParts queue partitions
   uint32_t n;                 // batched queries: the number of rays
-  uint32_t* records;          // batched queries with full records: n x 16 u32
   bool deal;                  // batched queries: the rays are dealt out to the launch's waves
                               // beforehand, without cursors
 };
@@ -138,7 +137,7 @@ struct ShadeArgs {
   const JobDesc* jobs;
 };
 
-// The allocation-free query's work cursors: kIsectGroups words,
+// k_intersect's work cursors: kIsectGroups words,
 // kIsectCursorStride words (128 bytes) apart.
 constexpr uint32_t kIsectGroups = 64;
 constexpr uint32_t kIsectCursorStride = 32;
@@ -157,15 +156,13 @@ struct IntersectArgs {
   uint32_t* isects;  // n x 16 u32 or null
 };
 
-// Queries with full records through the lane-refill traversal (a.records =
-// r.isects), then the pass that completes the records.
-hipError_t launch_records(const ExtendArgs& a, const IntersectArgs& r, bool packed, int stack,
-                          uint32_t blocks, uint32_t block_waves, hipStream_t s);
-// One 64-ray batch after the other per wave, kIsectStack LDS stack entries
-// per lane: the allocation-free query.
+// One 64-ray batch after the other per wave from the cursors, or (deal: full
+// records, n at most 64 * blocks) one batch of at most 64 rays for each wave.
+// stack: LDS stack entries per lane; kIsectStack for the allocation-free query,
+// the only one that may ask for hits without counters.
 constexpr int kIsectStack = 32;
-hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, uint32_t blocks,
-                            hipStream_t s);
+hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, bool deal, int stack,
+                            uint32_t blocks, hipStream_t s);
 
 // CV_RNG_REF_PATCH rendering: patches (x, y, width, 0) of the job's image,
 // frames first_frame .. first_frame + nframes - 1 of each in order, into

@@ -348,10 +348,21 @@ __device__ __forceinline__ uint32_t fetch_below(uint32_t* cursor, uint32_t limit
 // Four words at any word address.
 typedef uint32_t words4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// A query's outputs for ray i: its hit and, when asked for, the deferred
-// MIntersection fields (triangle.rs:129-142, scene.rs:221-228).
-__device__ __forceinline__ void write_record(const IntersectArgs& a, uint32_t i, V3 o, V3 d,
-                                             const TravState& ts) {
+// Rays traversed until the wave's slowest lane ends: lane's ray i (when valid),
+// its hit and, when asked for, the deferred MIntersection fields
+// (triangle.rs:129-142, scene.rs:221-228).
+template <bool COUNT, int S, bool PACKED>
+__device__ __forceinline__ void intersect_ray(const IntersectArgs& a, uint32_t i, bool valid,
+                                              uint2* lds, uint32_t gtid, uint32_t stride) {
+  V3 o = mk3(0, 0, 0), d = mk3(1, 0, 0);
+  if (valid) {
+    const float* r = a.rays + 6 * (size_t)i;
+    o = mk3(r[0], r[1], r[2]);
+    d = mk3(r[3], r[4], r[5]);
+  }
+  const TravState ts =
+      traverse<COUNT, S, PACKED>(a.nodes, a.tris, o, d, lds, a.spill, gtid, stride, valid);
+  if (!valid) return;
   const uint32_t src = ts.best == kNoHit ? kNoHit : a.tri_src[ts.best];
   if (a.hits) {
     reinterpret_cast<uint4*>(a.hits)[i] =
@@ -384,7 +395,7 @@ __device__ __forceinline__ void write_record(const IntersectArgs& a, uint32_t i,
 }
 
 // ---------------------------------------------------------------------------
-// cv_bvh_intersect_nearest_noalloc, and the outputs of every query
+// cv_bvh_intersect_nearest with full records, cv_bvh_intersect_nearest_noalloc
 // ---------------------------------------------------------------------------
 
 // The n / 64 batches of 64 rays are split into kIsectGroups contiguous
@@ -411,18 +422,8 @@ __global__ __launch_bounds__(64) void k_intersect(IntersectArgs a) {
       --left;
       continue;
     }
-    uint32_t i = (lo + k) * 64u + lane;
-    bool valid = i < a.n;
-    V3 o = mk3(0, 0, 0), d = mk3(1, 0, 0);
-    if (valid) {
-      const float* r = a.rays + 6 * (size_t)i;
-      o = mk3(r[0], r[1], r[2]);
-      d = mk3(r[3], r[4], r[5]);
-    }
-    TravState ts = traverse<COUNT, S, PACKED>(a.nodes, a.tris, o, d, lds + lane,
-                                              a.spill, gtid, stride, valid);
-    if (!valid) continue;
-    write_record(a, i, o, d, ts);
+    const uint32_t i = (lo + k) * 64u + lane;
+    intersect_ray<COUNT, S, PACKED>(a, i, i < a.n, lds + lane, gtid, stride);
   }
 }
 
@@ -1045,16 +1046,9 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
           }
         }
         if (active && !have && st.sp == 0) {
-          if constexpr (QUERY && COUNT) {
-            // what k_records makes the record of, at its start
-            words4* out = reinterpret_cast<words4*>(a.records + 16 * (size_t)ray);
-            out[0] = words4{ts.best, f2u(ts.best_t), f2u(ts.bu), f2u(ts.bv)};
-            out[1] = words4{ts.na, ts.nt, 0u, 0u};
-          } else {
-            a.hits[ray] = make_uint4(QUERY ? hit_id<true>(a, ts.best) : ts.best, f2u(ts.best_t),
-                                     f2u(ts.bu), f2u(ts.bv));
-          }
-          if (COUNT && !QUERY) {
+          a.hits[ray] = make_uint4(QUERY ? hit_id<true>(a, ts.best) : ts.best, f2u(ts.best_t),
+                                   f2u(ts.bu), f2u(ts.bv));
+          if (COUNT) {
             na += ts.na;
             nt += ts.nt;
           }
@@ -1067,7 +1061,7 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
     else
       steps(std::false_type{});
   }
-  if (COUNT && !QUERY) {
+  if (COUNT) {
     for (int off = 32; off > 0; off >>= 1) {
       na += __shfl_down(na, off);
       nt += __shfl_down(nt, off);
@@ -1089,33 +1083,25 @@ __global__ __launch_bounds__(256, W == 2 && !COUNT && !MULTI && (PACKED || !QUER
   extend_refill<COUNT, S, PACKED, MULTI, QUERY, W, false>(a, lds_waves);
 }
 
-// Queries of few rays per lane of the launch, dealt out to its waves.
-// COUNT: full records, else hits only.
-template <bool COUNT, int S, bool PACKED, int W>
+// Hits-only queries of few rays per lane of the launch, dealt out to its waves.
+template <int S, bool PACKED, int W>
 __global__ __launch_bounds__(256) void k_query_dealt(ExtendArgs a) {
   extern __shared__ uint2 lds_waves[];
-  extend_refill<COUNT, S, PACKED, false, true, W, true>(a, lds_waves);
+  extend_refill<false, S, PACKED, false, true, W, true>(a, lds_waves);
 }
 
-// The full records of a query from what its traversal left at their starts:
-// the deferred MIntersection fields (triangle.rs:129-142, scene.rs:221-228),
-// and the hits when asked for.  A pass of its own, bound by its 88 B in and
-// 64 B out per ray: in the traversal the few lanes that finish in a step
-// would run it for the whole wave.
-__global__ __launch_bounds__(256) void k_records(IntersectArgs a) {
-  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.n; i += gridDim.x * 256) {
-    words4* out = reinterpret_cast<words4*>(a.isects + 16 * (size_t)i);
-    const words4 h = out[0], c = out[1];
-    const float* r = a.rays + 6 * (size_t)i;
-    TravState ts;
-    ts.best = h.x;
-    ts.best_t = u2f(h.y);
-    ts.bu = u2f(h.z);
-    ts.bv = u2f(h.w);
-    ts.na = c.x;
-    ts.nt = c.y;
-    write_record(a, i, mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), ts);
-  }
+// Full records of at most one ray per lane, dealt out to the launch's waves.
+// Bound by the longest chain of a wave.  300,000 decoherent rays: in a room of
+// 200,000 triangles 0.38-0.44 ms, on 968 triangles 0.090; from the cursors, which
+// most waves of such a launch only find used up, 0.48 and 0.13; in the
+// lane-refill loop with its votes and a pass for the records 0.45 and 0.12.
+template <int S, bool PACKED>
+__global__ __launch_bounds__(64) void k_intersect_dealt(IntersectArgs a) {
+  __shared__ uint2 lds[S * 64];
+  const uint32_t lane = lane_id();
+  const Deal deal = deal_rays<false>(a.n, gridDim.x);
+  intersect_ray<true, S, PACKED>(a, deal.mine * deal.rest + lane, lane < deal.end, lds + lane,
+                                 blockIdx.x * 64 + lane, gridDim.x * 64);
 }
 
 // ---------------------------------------------------------------------------
@@ -1763,18 +1749,35 @@ __global__ __launch_bounds__(64) void k_ref_patch(RefPatchArgs a) {
 
 #define CVK_STACK_VARIANTS(X) X(8) X(16) X(24) X(32)
 
-hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, uint32_t blocks,
-                            hipStream_t s) {
-  constexpr int S = kIsectStack;
-  if (count && packed)
-    hipLaunchKernelGGL((k_intersect<true, S, true>), dim3(blocks), dim3(64), 0, s, a);
+template <int S>
+static hipError_t launch_intersect_s(const IntersectArgs& a, bool count, bool packed, bool deal,
+                                     uint32_t blocks, hipStream_t s) {
+  const dim3 grid(blocks), block(64);
+  if (deal && (!count || a.n > (uint64_t)blocks * 64u)) return hipErrorInvalidValue;
+  if (deal && packed)
+    hipLaunchKernelGGL((k_intersect_dealt<S, true>), grid, block, 0, s, a);
+  else if (deal)
+    hipLaunchKernelGGL((k_intersect_dealt<S, false>), grid, block, 0, s, a);
+  else if (count && packed)
+    hipLaunchKernelGGL((k_intersect<true, S, true>), grid, block, 0, s, a);
   else if (count)
-    hipLaunchKernelGGL((k_intersect<true, S, false>), dim3(blocks), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((k_intersect<true, S, false>), grid, block, 0, s, a);
+  else if (S != kIsectStack)  // hits only: the allocation-free query's
+    return hipErrorInvalidValue;
   else if (packed)
-    hipLaunchKernelGGL((k_intersect<false, S, true>), dim3(blocks), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((k_intersect<false, kIsectStack, true>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((k_intersect<false, S, false>), dim3(blocks), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((k_intersect<false, kIsectStack, false>), grid, block, 0, s, a);
   return hipGetLastError();
+}
+
+hipError_t launch_intersect(const IntersectArgs& a, bool count, bool packed, bool deal, int stack,
+                            uint32_t blocks, hipStream_t s) {
+#define CASE(S) \
+  if (stack == S) return launch_intersect_s<S>(a, count, packed, deal, blocks, s);
+  CVK_STACK_VARIANTS(CASE)
+#undef CASE
+  return hipErrorInvalidValue;
 }
 
 // Wide trees (4 or 8 children): lane refill only (whole-batch requests run
@@ -1790,7 +1793,7 @@ static hipError_t launch_extend_wide(const ExtendArgs& a, bool multi, uint32_t b
   if (multi)
     hipLaunchKernelGGL((k_extend_refill<COUNT, S, true, true, false, W>), grid, block, shmem, s, b);
   else if (b.rays6 && !COUNT && b.deal)
-    hipLaunchKernelGGL((k_query_dealt<false, S, true, W>), grid, block, shmem, s, b);
+    hipLaunchKernelGGL((k_query_dealt<S, true, W>), grid, block, shmem, s, b);
   else if (b.rays6 && !COUNT)
     hipLaunchKernelGGL((k_extend_refill<false, S, true, false, true, W>), grid, block, shmem, s,
                        b);
@@ -1817,9 +1820,9 @@ static hipError_t launch_extend_s(const ExtendArgs& a, bool packed, bool multi, 
     // batched queries: the caller's rays and source ids, compiled apart so
     // that the render instantiations carry neither
     if (a.deal && packed)
-      hipLaunchKernelGGL((k_query_dealt<false, S, true, 2>), grid, block, shmem, s, a);
+      hipLaunchKernelGGL((k_query_dealt<S, true, 2>), grid, block, shmem, s, a);
     else if (a.deal)
-      hipLaunchKernelGGL((k_query_dealt<false, S, false, 2>), grid, block, shmem, s, a);
+      hipLaunchKernelGGL((k_query_dealt<S, false, 2>), grid, block, shmem, s, a);
     else if (packed)
       hipLaunchKernelGGL((k_extend_refill<false, S, true, false, true>), grid, block, shmem, s, a);
     else
@@ -1838,34 +1841,6 @@ static hipError_t launch_extend_s(const ExtendArgs& a, bool packed, bool multi, 
   return hipGetLastError();
 }
 
-template <int S>
-static hipError_t launch_records_s(const ExtendArgs& a, const IntersectArgs& r, bool packed,
-                                   uint32_t blocks, uint32_t block_waves, hipStream_t s) {
-  const uint32_t bw = block_waves == 2 || block_waves == 4 ? block_waves : 1u;
-  const dim3 grid((blocks + bw - 1) / bw), block(64 * bw);
-  const size_t shmem = (size_t)S * 64 * sizeof(uint2) * bw;
-  if (a.deal && packed)
-    hipLaunchKernelGGL((k_query_dealt<true, S, true, 2>), grid, block, shmem, s, a);
-  else if (a.deal)
-    hipLaunchKernelGGL((k_query_dealt<true, S, false, 2>), grid, block, shmem, s, a);
-  else if (packed)
-    hipLaunchKernelGGL((k_extend_refill<true, S, true, false, true>), grid, block, shmem, s, a);
-  else
-    hipLaunchKernelGGL((k_extend_refill<true, S, false, false, true>), grid, block, shmem, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_records, dim3(r.n < (1u << 20) ? (r.n + 255) / 256 : 4096u), dim3(256), 0, s,
-                     r);
-  return hipGetLastError();
-}
-hipError_t launch_records(const ExtendArgs& a, const IntersectArgs& r, bool packed, int stack,
-                          uint32_t blocks, uint32_t block_waves, hipStream_t s) {
-#define CASE(S) \
-  if (stack == S) return launch_records_s<S>(a, r, packed, blocks, block_waves, s);
-  CVK_STACK_VARIANTS(CASE)
-#undef CASE
-  return hipErrorInvalidValue;
-}
 hipError_t launch_extend(const ExtendArgs& a, bool count, bool packed, bool multi, int stack,
                          uint32_t blocks, uint32_t block_waves, hipStream_t s, uint32_t width) {
   if (multi && !a.refill) return hipErrorInvalidValue;

@@ -220,12 +220,13 @@ typedef struct cv_isect {
 /* Scene::intersect_nearest / Bvh::intersect_nearest / intersect_debug
  * (scene.rs:220-244, bvh.rs:589-669), batched, one ray per GPU lane.  Each
  * ray is traversed as the reference traverses a packet holding that ray in
- * every lane.  hits and isects may each be NULL.  The traversal takes the
- * scene's tuning (with isects, bvh_width 2: its counters are the reference
- * tree's), at least 4 batches of 64 rays per fetch, and checks for refills
- * every refill_interval / 4 steps (at least 1); up to 4 rays per lane of 24
- * waves per CU are dealt out to the waves instead of fetched.  hits must be
- * 16-byte aligned.  Returns after the results are written. */
+ * every lane.  hits and isects may each be NULL.  A call with hits and no
+ * isects traverses with the scene's tuning, taking at least 4 batches of 64
+ * rays per fetch and checking for refills every refill_interval / 4 steps (at
+ * least 1); one with isects traverses the reference's tree, whose counters
+ * they hold, 64 rays a wave.  Few rays (hits: up to 4 per lane of 24 waves per
+ * CU, isects: up to one) are dealt out to the waves instead of fetched.  hits
+ * must be 16-byte aligned.  Returns after the results are written. */
 cv_status cv_bvh_intersect_nearest(const cv_scene* scene, const cv_ray* rays, size_t n,
                                    cv_hit* hits, cv_isect* isects, uint32_t flags);
 

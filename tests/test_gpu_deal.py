@@ -68,3 +68,37 @@ def test_records_equal_oracle(cv, oracle, tuning, waves_per_cu):
         assert (hits["tri_id"] == rec["tri_id"]).all()
         _check_exact(hits, rec, {k: v[:n] for k, v in ref.items()})
         assert (rec["reserved"] == 0).all()
+
+
+@pytest.mark.parametrize("stack", [8, 16, 24, 32])
+@pytest.mark.parametrize("leaves", [None, 40])
+def test_records_around_one_ray_per_lane(cv, oracle, stack, leaves):
+    """Full records at the last dealt size and the first that goes through the
+    cursors, for every stack size, on the built tree and on an imported one of
+    two leaves of more triangles than a packed stack entry counts."""
+    if leaves:
+        t, m = scenes.free_triangles(scenes.Stream(5), 100)
+        sd = scenes.SceneData(tris=np.asarray(t, np.float32), materials=m)
+        nodes = np.zeros(2, cv.NODE_DTYPE)
+        for k, (a, b) in enumerate([(0, leaves), (leaves, 100)]):
+            v = sd.tris[a:b].reshape(-1, 3)
+            nodes[k] = (v.min(0), v.max(0), a, b - a)
+        g = cv.Scene.from_scene_data(sd, with_bvh=(nodes, np.arange(100, dtype=np.uint32)))
+        assert g.bvh_info()["max_leaf"] == 60
+    else:
+        sd = scenes.config0(subdivisions=2)
+        g = cv.Scene.from_scene_data(sd)
+    g.set_tuning(extend_waves_per_cu=1, stack_entries=stack)
+    rays = scenes.rays_inward(LANES + 65, 19, radius=0.9, target_scale=0.6)
+    ref = oracle.Scene.from_scene_data(sd).intersect(rays, isect=True)
+    for n in (LANES - 1, LANES, LANES + 1, LANES + 65):
+        print("%d rays, stack %d, leaves %r" % (n, stack, leaves), flush=True)
+        hits, rec = g.intersect_nearest(rays[:n], full=True)
+        part = {k: v[:n] for k, v in ref.items()}
+        if leaves:  # the counters are the imported tree's
+            assert (hits["tri_id"] == part["tri"]).all()
+            assert (hits["t"].view(np.uint32) == part["tuv"][:, 0].copy().view(np.uint32)).all()
+            assert set(np.unique(rec["numi_aabb"])) == {2} and rec["numi_tri"].max() == 100
+        else:
+            _check_exact(hits, rec, part)
+        assert (hits["tri_id"] == rec["tri_id"]).all()
