@@ -801,17 +801,25 @@ cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_
     x.interval = s->cfg.refill_interval > 4 ? s->cfg.refill_interval / 4 : 1u;
     x.leaf_batch = s->cfg.leaf_batch <= 64 ? s->cfg.leaf_batch : 0u;
     x.parts = s->cfg.parts;
-    // Dealt out up to kQueryDeal rays per lane; whole-batch launches always
-    // use the cursor.
-    const uint64_t few_lanes = (uint64_t)((few + bw - 1) / bw * bw) * 64u;
-    x.deal = n <= few_lanes * kQueryDeal && (x.refill || s->cfg.width != 2);
+    // Dealt out to the waves that are resident at once (shares of further waves
+    // only start when others end), up to kQueryDeal rays per lane of 24 waves
+    // per CU and half as many where the launch shape holds fewer: there a lane's
+    // share ends further from the next one's (a room of 50,000 triangles with 16
+    // stack entries, 20 waves: 10^6 rays, 3 per lane, 0.80 ms from the cursors
+    // and 0.93 dealt; 600,000, 1.8 per lane, 0.84 and 0.66).  Whole-batch
+    // launches always use the cursor.
+    const uint32_t waves = std::min(
+        few, cvk::query_dealt_waves(s->packed, s->cfg.stack, bw, s->cfg.width) * cvh::num_cus());
+    const uint64_t lanes = (uint64_t)((waves + bw - 1) / bw * bw) * 64u;
+    const uint32_t per_lane = waves == 24u * cvh::num_cus() ? kQueryDeal : kQueryDeal / 2;
+    x.deal = n <= lanes * per_lane && (x.refill || s->cfg.width != 2);
     if (!x.deal) {
       if (!s->q_ctrl.p) HIPTRY(s->q_ctrl.alloc(1), "alloc");
       HIPTRY(cvk::launch_query_ctrl(s->q_ctrl.p, (uint32_t)n, st), "query control");
       x.ctrl = s->q_ctrl.p;
     }
     HIPTRY(cvk::launch_extend(x, false, s->packed, false, s->cfg.stack,
-                              x.deal ? few : s->cfg.blocks, bw, st, s->cfg.width),
+                              x.deal ? waves : s->cfg.blocks, bw, st, s->cfg.width),
            "intersect");
   }
   if (!dev) {

@@ -192,6 +192,8 @@ hipError_t launch_query_ctrl(Ctrl* ctrl, uint32_t n, hipStream_t s);
 hipError_t launch_extend(const ExtendArgs& a, bool count, bool packed, bool multi, int stack,
                          uint32_t blocks, uint32_t block_waves, hipStream_t s,
                          uint32_t width = 2);
+// Waves per CU that a dealt query of that launch shape keeps resident.
+uint32_t query_dealt_waves(bool packed, int stack, uint32_t block_waves, uint32_t width);
 hipError_t launch_generate(const GenerateArgs& a, uint32_t blocks, hipStream_t s);
 // The ray sort of one bounce (four kernels: clear, keys, scan, scatter);
 // `paths` bounds the step's path count (the grid of the per-path kernels).

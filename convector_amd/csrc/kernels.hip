@@ -1841,6 +1841,40 @@ static hipError_t launch_extend_s(const ExtendArgs& a, bool packed, bool multi, 
   return hipGetLastError();
 }
 
+// Waves of k_query_dealt resident on a CU, asked once per instantiation and
+// workgroup size.
+template <int S, bool PACKED, int W, uint32_t BW>
+static uint32_t dealt_waves() {
+  static const uint32_t n = [] {
+    int groups = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&groups, k_query_dealt<S, PACKED, W>, 64 * BW,
+                                                     (size_t)S * 64 * sizeof(uint2) * BW) !=
+            hipSuccess ||
+        groups <= 0)
+      return 8u;
+    return (uint32_t)groups * BW;
+  }();
+  return n;
+}
+template <int S, bool PACKED, int W>
+static uint32_t dealt_waves_of(uint32_t block_waves) {
+  return block_waves == 4   ? dealt_waves<S, PACKED, W, 4>()
+         : block_waves == 2 ? dealt_waves<S, PACKED, W, 2>()
+                            : dealt_waves<S, PACKED, W, 1>();
+}
+
+uint32_t query_dealt_waves(bool packed, int stack, uint32_t block_waves, uint32_t width) {
+#define CASE(S)                                                        \
+  if (stack == S)                                                      \
+    return width == 8   ? dealt_waves_of<S, true, 8>(block_waves)      \
+           : width == 4 ? dealt_waves_of<S, true, 4>(block_waves)      \
+           : packed     ? dealt_waves_of<S, true, 2>(block_waves)      \
+                        : dealt_waves_of<S, false, 2>(block_waves);
+  CVK_STACK_VARIANTS(CASE)
+#undef CASE
+  return 8;
+}
+
 hipError_t launch_extend(const ExtendArgs& a, bool count, bool packed, bool multi, int stack,
                          uint32_t blocks, uint32_t block_waves, hipStream_t s, uint32_t width) {
   if (multi && !a.refill) return hipErrorInvalidValue;

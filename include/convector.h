@@ -225,8 +225,9 @@ typedef struct cv_isect {
  * rays per fetch and checking for refills every refill_interval / 4 steps (at
  * least 1); one with isects traverses the reference's tree, whose counters
  * they hold, 64 rays a wave.  Few rays (hits: up to 4 per lane of 24 waves per
- * CU, isects: up to one) are dealt out to the waves instead of fetched.  hits
- * must be 16-byte aligned.  Returns after the results are written. */
+ * CU, or 2 per lane where the tuning keeps fewer waves resident; isects: up to
+ * one) are dealt out to the waves instead of fetched.  hits must be 16-byte
+ * aligned.  Returns after the results are written. */
 cv_status cv_bvh_intersect_nearest(const cv_scene* scene, const cv_ray* rays, size_t n,
                                    cv_hit* hits, cv_isect* isects, uint32_t flags);
 

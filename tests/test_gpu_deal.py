@@ -2,12 +2,14 @@
 every ray is traversed once and gives the oracle's hit at the sizes where the
 dealing changes shape -- fewer rays than the smallest share, one more than a
 share or a stripe of 64 rays per wave, the last dealt size and the first that
-goes through the cursors.  (The grids are all multiples of the 8 XCDs on a
+goes through the cursors (2 rays per lane of the resident waves, 4 where 24
+waves per CU are).  (The grids are all multiples of the 8 XCDs on a
 device of 256 CUs; test_deal_map.py has the others.)"""
 import numpy as np
 import pytest
 
 from convector_amd import scenes
+from helpers import check_tolerance
 from test_gpu_traversal import _check_exact
 
 pytestmark = pytest.mark.gpu
@@ -26,11 +28,33 @@ def test_dealt_queries_equal_oracle(cv, oracle, block_waves, waves_per_cu):
     rays = scenes.rays_inward(4 * lanes + 1, 7, radius=0.9, target_scale=0.6)
     ref = o.intersect(rays)
     for n in (1, 3, 4, 5, 63, 65, 4096, 4097, lanes - 1, lanes, lanes + 1, lanes + 4097,
-              4 * lanes - 63, 4 * lanes, 4 * lanes + 1):
+              2 * lanes, 2 * lanes + 1, 4 * lanes - 63, 4 * lanes, 4 * lanes + 1):
         print("%d rays, %d waves per CU, %d per block" % (n, waves_per_cu, block_waves), flush=True)
         hits = g.intersect_nearest(rays[:n])
         assert (hits["tri_id"] == ref["tri"][:n]).all(), n
         assert (hits["t"].view(np.uint32) == ref["tuv"][:n, 0].copy().view(np.uint32)).all(), n
+
+
+@pytest.mark.parametrize("tuning,waves,rays", [
+    ({}, 24, 4), ({"stack_entries": 16}, 20, 2), ({"stack_entries": 32, "block_waves": 4}, 8, 2),
+    ({"bvh_width": 8}, None, 2)])
+def test_dealt_queries_by_residency(cv, oracle, tuning, waves, rays):
+    """The last dealt size and the first from the cursors for launch shapes that
+    keep all 24 waves per CU resident and ones that do not."""
+    sd = scenes.config0(subdivisions=2)
+    g = cv.Scene.from_scene_data(sd)
+    g.set_tuning(**tuning)
+    last = (waves or 16) * LANES * rays
+    r = scenes.rays_inward(last + 1, 8, radius=0.9, target_scale=0.6)
+    ref = oracle.Scene.from_scene_data(sd).intersect(r)
+    for n in (last - 1, last, last + 1):
+        print("%d rays, %r" % (n, tuning), flush=True)
+        hits = g.intersect_nearest(r[:n])
+        if "bvh_width" in tuning:
+            check_tolerance(sd, hits, {k: v[:n] for k, v in ref.items()}, r[:n])
+        else:
+            assert (hits["tri_id"] == ref["tri"][:n]).all()
+            assert (hits["t"].view(np.uint32) == ref["tuv"][:n, 0].copy().view(np.uint32)).all()
 
 
 @pytest.mark.parametrize("w,h", [(16, 4), (128, 124), (128, 128), (128, 132)])
