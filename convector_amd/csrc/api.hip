@@ -705,13 +705,15 @@ void cv_scene_destroy(cv_scene* s) {
 
 // --------------------------------------------------------------- traversal
 
-// Hits-only queries of at most this many rays per lane of 24 waves per CU are
-// dealt out: 1.57 M rays, below where the cursors draw level (250 k / 1 M / 2 M /
-// 4 M / 6 M decoherent rays in us, dealt against cursors: suzanne 109 / 182 /
-// 285 / 478 / 664 and 242 / 284 / 324 / 470 / 640, bunny 162 / 299 / 487 / 834 /
-// 1174 and 346 / 415 / 498 / 829 / 1117, a room of 200,000 triangles 450 / 816 /
-// 1212 / 2192 / 3115 and 808 / 975 / 1339 / 2203 / 3016; coherent rays alike).
-static constexpr uint32_t kQueryDeal = 4;
+// Hits-only queries of at most this many rays per lane are dealt out: 8 of 24
+// waves per CU, 3.1 M rays, where the cursors draw level in every scene (250 k /
+// 1 M / 2 M / 3 M / 4 M / 6 M decoherent rays in us, dealt against cursors:
+// suzanne 109 / 182 / 285 / 374 / 478 / 664 and 242 / 284 / 324 / 404 / 470 / 640,
+// bunny 162 / 299 / 487 / 661 / 834 / 1174 and 346 / 415 / 498 / 665 / 829 / 1117,
+// a room of 200,000 triangles 450 / 816 / 1212 / 1717 / 2192 / 3115 and 808 / 975 /
+// 1339 / 1760 / 2203 / 3016; coherent rays alike), and 2 where fewer waves are
+// resident.
+static constexpr uint32_t kQueryDeal = 8, kQueryDealFew = 2;
 
 cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_t n, cv_hit* hits,
                                    cv_isect* isects, uint32_t flags) {
@@ -802,16 +804,15 @@ cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_
     x.leaf_batch = s->cfg.leaf_batch <= 64 ? s->cfg.leaf_batch : 0u;
     x.parts = s->cfg.parts;
     // Dealt out to the waves that are resident at once (shares of further waves
-    // only start when others end), up to kQueryDeal rays per lane of 24 waves
-    // per CU and half as many where the launch shape holds fewer: there a lane's
-    // share ends further from the next one's (a room of 50,000 triangles with 16
+    // only start when others end).  Where the launch shape holds fewer than 24
+    // per CU the shares of 3 rays per lane already end too far apart (a room of 50,000 triangles with 16
     // stack entries, 20 waves: 10^6 rays, 3 per lane, 0.80 ms from the cursors
     // and 0.93 dealt; 600,000, 1.8 per lane, 0.84 and 0.66).  Whole-batch
     // launches always use the cursor.
     const uint32_t waves = std::min(
         few, cvk::query_dealt_waves(s->packed, s->cfg.stack, bw, s->cfg.width) * cvh::num_cus());
     const uint64_t lanes = (uint64_t)((waves + bw - 1) / bw * bw) * 64u;
-    const uint32_t per_lane = waves == 24u * cvh::num_cus() ? kQueryDeal : kQueryDeal / 2;
+    const uint32_t per_lane = waves == 24u * cvh::num_cus() ? kQueryDeal : kQueryDealFew;
     x.deal = n <= lanes * per_lane && (x.refill || s->cfg.width != 2);
     if (!x.deal) {
       if (!s->q_ctrl.p) HIPTRY(s->q_ctrl.alloc(1), "alloc");

@@ -224,7 +224,7 @@ typedef struct cv_isect {
  * isects traverses with the scene's tuning, taking at least 4 batches of 64
  * rays per fetch and checking for refills every refill_interval / 4 steps (at
  * least 1); one with isects traverses the reference's tree, whose counters
- * they hold, 64 rays a wave.  Few rays (hits: up to 4 per lane of 24 waves per
+ * they hold, 64 rays a wave.  Few rays (hits: up to 8 per lane of 24 waves per
  * CU, or 2 per lane where the tuning keeps fewer waves resident; isects: up to
  * one) are dealt out to the waves instead of fetched.  hits must be 16-byte
  * aligned.  Returns after the results are written. */

@@ -43,10 +43,11 @@ def _shares(n, grid, bw, whole_stripes):
 def test_every_ray_is_dealt_once(grid, bw, whole_stripes):
     lanes = grid * bw * 64
     sizes = [1, 3, 4, 5, 63, 64, 65, 4096, 4097, lanes - 1, lanes]
-    if whole_stripes:  # queries of up to 4 rays per lane; bounces of up to one
-        sizes += [lanes + 1, lanes + 4097, 4 * lanes - 63, 4 * lanes]
+    # hits-only queries of up to 8 rays per lane; records and bounces of up to one
+    if whole_stripes:
+        sizes += [lanes + 1, lanes + 4097, 4 * lanes - 63, 4 * lanes, 8 * lanes - 1, 8 * lanes]
     for n in sizes:
-        if n > (4 if whole_stripes else 1) * lanes:
+        if n > (8 if whole_stripes else 1) * lanes:
             continue
         seen = np.zeros(n, np.int64)
         for q in _shares(n, grid, bw, whole_stripes):

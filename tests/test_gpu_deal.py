@@ -2,7 +2,7 @@
 every ray is traversed once and gives the oracle's hit at the sizes where the
 dealing changes shape -- fewer rays than the smallest share, one more than a
 share or a stripe of 64 rays per wave, the last dealt size and the first that
-goes through the cursors (2 rays per lane of the resident waves, 4 where 24
+goes through the cursors (2 rays per lane of the resident waves, 8 where 24
 waves per CU are).  (The grids are all multiples of the 8 XCDs on a
 device of 256 CUs; test_deal_map.py has the others.)"""
 import numpy as np
@@ -36,7 +36,7 @@ def test_dealt_queries_equal_oracle(cv, oracle, block_waves, waves_per_cu):
 
 
 @pytest.mark.parametrize("tuning,waves,rays", [
-    ({}, 24, 4), ({"stack_entries": 16}, 20, 2), ({"stack_entries": 32, "block_waves": 4}, 8, 2),
+    ({}, 24, 8), ({"stack_entries": 16}, 20, 2), ({"stack_entries": 32, "block_waves": 4}, 8, 2),
     ({"bvh_width": 8}, None, 2)])
 def test_dealt_queries_by_residency(cv, oracle, tuning, waves, rays):
     """The last dealt size and the first from the cursors for launch shapes that
