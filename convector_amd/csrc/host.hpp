@@ -119,7 +119,7 @@ struct cv_scene {
   cvh::LaunchCfg cfg;              // traversal launch shape (cv_scene_set_tuning)
   cvh::DevBuf<uint2> spill;        // stack spill area of cv_bvh_intersect_nearest
   cvh::DevBuf<uint32_t> cursor;    // full-record queries: k_intersect's work cursors
-  cvh::DevBuf<cvk::Ctrl> q_ctrl;   // hits-only queries: one-bounce step control block
+  cvh::DevBuf<cvk::Ctrl> q_ctrl;   // hits-only queries from the cursors: control block of a step
   // the tree collapsed to 4 and 8 children per node (built on first use)
   cvh::DevBuf<float4> wide[2];
   uint32_t wide_nodes[2] = {0, 0};

@@ -180,8 +180,8 @@ struct RefPatchArgs {
 // spill area's waves).
 hipError_t launch_ref_patch(const RefPatchArgs& a, bool packed, int stack, uint32_t blocks,
                             hipStream_t s);
-// Hits-only queries through launch_extend: a zeroed control block with
-// count[0] = n.
+// Hits-only queries through launch_extend that are not dealt out: a zeroed
+// control block with count[0] = n.
 hipError_t launch_query_ctrl(Ctrl* ctrl, uint32_t n, hipStream_t s);
 // multi: rays of the step belong to more than one scene (per-ray node and
 // triangle pointers from the job table).

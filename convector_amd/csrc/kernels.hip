@@ -878,8 +878,8 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
   // A render's queue of at most one ray per lane and DEALT queries are dealt
   // out beforehand instead: every wave of the launch taking its atomics from the
   // cursors, most to find them used up, keeps a launch of few rays busy for
-  // 100-200 us (256 rays on 968 triangles: 207 us, dealt 60; 600,000 in a
-  // 200,000-triangle room: 1.00 ms, dealt 0.69).  A render's bounce of more
+  // 100-200 us (256 rays on 968 triangles: 205 us, dealt 56; 600,000 in a
+  // 200,000-triangle room: 0.96 ms, dealt 0.62).  A render's bounce of more
   // rays stays with the cursors: neighbouring paths cost alike, so fixed
   // shares end further apart (1280 x 736 frames: no faster).
   const uint32_t waves = gridDim.x * (blockDim.x >> 6);
@@ -1009,11 +1009,12 @@ __device__ __forceinline__ void extend_refill(const ExtendArgs& a, uint2* lds_wa
     // several traversal steps per refill check: the check's votes cost
     // about as much as a step's mask logic, and a lane that finishes early
     // idles for at most interval - 1 steps.  Bound by instruction issue in
-    // large launches (80 % VALU) and by the length of a step in the drain of
-    // all: a leaf round in the step that completes its quorum instead of the
+    // large launches (80 % of one VALU instruction per CU per cycle, of whose
+    // lanes 38 of 64 are active in renders and 33 in 10^7 decoherent rays on the
+    // bunny) and by the length of a step in the drain of all: a leaf round in the step that completes its quorum instead of the
     // next one (which took every entry again), no exact-rule branches inside
     // a step, and the hit test as one compare took the extend launches of a
-    // 16-sample 1080p step from 55.3 to 53.8 ms, 64 rays' chains 9 % less.
+    // 16-sample 1080p step from 55.4 to 53.6 ms, 64 rays' chains 9 % less.
     auto steps = [&](auto exact_rules) {
       constexpr bool EXACT = decltype(exact_rules)::value;
 #pragma unroll 1
@@ -1970,7 +1971,7 @@ hipError_t launch_fold_features(float* feat, float* slots, size_t slot_stride, u
 
 // cv_bvh_intersect_nearest without cv_isect output runs the lane-refill
 // traversal of the extend step over the caller's rays: the control block of
-// a one-bounce step.
+// a one-bounce step for the queries that are not dealt out.
 // One word per lane: zeros, and n in count[0].
 __global__ __launch_bounds__(64) void k_query_ctrl(Ctrl* ctrl, uint32_t n) {
   static_assert(sizeof(Ctrl) % 4 == 0, "Ctrl is whole words");
