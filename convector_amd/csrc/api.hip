@@ -805,10 +805,10 @@ cv_status cv_bvh_intersect_nearest(const cv_scene* sc, const cv_ray* rays, size_
     x.parts = s->cfg.parts;
     // Dealt out to the waves that are resident at once (shares of further waves
     // only start when others end).  Where the launch shape holds fewer than 24
-    // per CU the shares of 3 rays per lane already end too far apart (a room of 50,000 triangles with 16
-    // stack entries, 20 waves: 10^6 rays, 3 per lane, 0.80 ms from the cursors
-    // and 0.93 dealt; 600,000, 1.8 per lane, 0.84 and 0.66).  Whole-batch
-    // launches always use the cursor.
+    // per CU the shares of 3 rays per lane already end too far apart (a room of
+    // 50,000 triangles with 16 stack entries, 20 waves: 10^6 rays, 3 per lane,
+    // 0.80 ms from the cursors and 0.93 dealt; 600,000, 1.8 per lane, 0.84 and
+    // 0.66).  Whole-batch launches always use the cursor.
     const uint32_t waves = std::min(
         few, cvk::query_dealt_waves(s->packed, s->cfg.stack, bw, s->cfg.width) * cvh::num_cus());
     const uint64_t lanes = (uint64_t)((waves + bw - 1) / bw * bw) * 64u;
