@@ -1,6 +1,6 @@
 /*
  * cv_oracle.h -- CPU restatement of Convector's per-ray path, used ONLY as
- * test infrastructure (the checker for the HIP path and the timed CPU
+ * test infrastructure (what the HIP path is compared with and the timed CPU
  * baseline).  Nothing in the product links or loads this library.
  *
  * Every function restates a function of the reference (ruuda/convector, Rust)

@@ -1,8 +1,8 @@
 """ctypes binding of the CPU oracle (oracle/liboracle.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, the smoke check of
-__graft_entry__ and the cpu_baseline leg of bench.py, and only as the checker
-or the timed CPU baseline.  The product (convector_amd) never imports it.
+__graft_entry__ and the cpu_baseline leg of bench.py, and only to compare with
+or as the timed CPU baseline.  The product (convector_amd) never imports it.
 """
 from __future__ import annotations
 

@@ -1,5 +1,5 @@
-"""FP32 PyTorch restatement of the denoiser network (the checker of the HIP
-kernels): the same layers, parameter layout and loss as
+"""FP32 PyTorch restatement of the denoiser network (what the HIP
+kernels are compared with): the same layers, parameter layout and loss as
 convector_amd/csrc/denoise.hip, with BF16 rounding applied where the GPU
 stores BF16 (weights, the input and every hidden activation) when bf16=True.
 Runs on the CPU."""
